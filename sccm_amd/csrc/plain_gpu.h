@@ -1,8 +1,10 @@
 // plain_gpu.h -- host interface of the plain-form mesh-point kernels
 // (plain_gpu.hip), used by pnamp_gpu.hip.
 //
-// The plain form works on units = (pair, Euler point), numbered
-// u = pair * n_euler + euler.  For a range of units it runs
+// The plain form works on units = (pair, Euler point evaluated), numbered
+// u = pair * nec + index in ecan: of two mirrored Euler points one is
+// evaluated, and of the nphi^2 gauge pairs those that no symmetry gives (see
+// gauge_class in pnamp_gpu.hip).  For a range of units it runs
 //   k_plain_setup  per unit: the gauge-independent products of the rotation
 //                  with the states (7 n x n complex matrices) -> work buffer;
 //   k_plain_gauge  per (unit, gauge point): Pfaffian, T^-1, densities, energy,
@@ -16,6 +18,10 @@
 
 struct PlainArgs {
   int n, h, nalp, nbet, ngam, NE, nphi, npack;
+  int nec, ngc;                    // Euler points and gauge pairs evaluated
+  const int2 *ecan;                // [nec]: Euler index, its mirror's or -1
+  const int2 *gcls;                // [ngc]: gauge indices (phi_p, phi_n) of the pairs evaluated
+  const int *gmap;                 // [nphi^2]: the pair evaluated, | 1 << 16 as its conjugate
   int zval, nval;
   double cscale, vac_scale, snpfaf, e0;
   const int *q0, *q1;              // [npairs] state indices (device)
@@ -33,10 +39,10 @@ struct PlainArgs {
   const double *q2;                // [5][n*n]
   const int4 *orbp;                // [nob2] orbit pairs
   int nob2;
-  // outputs, indexed by global unit
-  double2 *zres;                   // [units][PNAMP_NOBS]
-  int *status;                     // [units]
-  double2 *ze2, *zrho;             // [units][10], [units][nob2] (E2 only)
+  // outputs per (pair, Euler point of the mesh)
+  double2 *zres;                   // [npairs][NE][PNAMP_NOBS]
+  int *status;                     // [npairs][NE]
+  double2 *ze2, *zrho;             // [npairs][NE][10], [npairs][NE][nob2] (E2 only)
 };
 
 // n supported by the plain kernels: even, 8 <= n <= 64 (size classes

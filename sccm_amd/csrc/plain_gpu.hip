@@ -76,7 +76,8 @@ struct PlainCfg {
 
 // ------------------------------------------------------------------ setup
 struct PSetup {
-  int n, h, nalp, ngam, npack, NE, u0;
+  int n, h, nalp, ngam, npack, NE, u0;  // NE here and below: Euler points evaluated
+  const int2 *ecan;
   const double *alp, *gam, *rtab;
   const int *pk_a, *pk_b, *blk_off, *blk_sz, *blk_base, *twom;
   const int *q0, *q1;
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256) void k_plain_setup(PSetup p) {
   __shared__ double2 sR[RPK];
   __shared__ short m_off[32], m_sz[32], m_base[32];
   const int tid = threadIdx.x, n = p.n, h = p.h, nn = n * n;
-  const int ul = blockIdx.x, u = p.u0 + ul, ip = u / p.NE, iang = u - ip * p.NE;
+  const int ul = blockIdx.x, u = p.u0 + ul, ip = u / p.NE, iang = p.ecan[u - ip * p.NE].x;
   const int ig = iang % p.ngam, ia = (iang / p.ngam) % p.nalp, ib = iang / (p.ngam * p.nalp);
   const double alp = p.alp[ia], gam = p.gam[ig];
   const int q0 = p.q0[ip], q1 = p.q1[ip];
@@ -165,19 +166,20 @@ __global__ __launch_bounds__(256) void k_plain_setup(PSetup p) {
 
 // ------------------------------------------------------------------ gauge point
 struct PGauge {
-  int n, h, nphi, NE, zval, nval, nl, lbytes, nob2, nog, u0, nwg;
-  double cscale, vac_scale, snpfaf, e0;
-  const int *q0, *q1, *pz, *pn;
-  const double *U, *V, *Z, *det;
+  int n, h, nphi, NE, ngc, nl, lbytes, nob2, nog, u0, nwg;
+  const int2 *gcls;  // [ngc]: gauge indices of the pairs evaluated
+  double cscale, e0;
+  const int *q0, *q1;
+  const double *U, *V, *Z;
   const double2 *hoist;
   const double *mtab, *t1b;
   const uint4 *lofs;
   const double *lme;
   const double *q2;
   const int4 *orbp;
-  double2 *gout;  // [unit - u0][nphi^2][nog]: observables per gauge point, not yet norm-weighted
-  int *gst;       // [unit - u0][nphi^2]
-  double2 *gpf;   // [unit - u0][nphi^2]: Pfaffian of the gauge point's skew matrix
+  double2 *gout;  // [unit - u0][ngc][nog]: observables per gauge point, not yet norm-weighted
+  int *gst;       // [unit - u0][ngc]
+  double2 *gpf;   // [unit - u0][ngc]: Pfaffian of the gauge point's skew matrix
 };
 
 __device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int m) {
@@ -206,13 +208,13 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const unsigned L = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (L >= (unsigned)p.nwg) return;
-  const int ng = p.nphi * p.nphi;
+  const int ng = p.ngc;
   const int g = (int)(L % (unsigned)ng), ul = (int)(L / (unsigned)ng), u = p.u0 + ul;
   const int ip = u / p.NE;
   const int q0 = p.q0[ip];
-  const int lp = g / p.nphi, ln = g - lp * p.nphi;
-  const double phip = (p.nphi == 1) ? 0.0 : (2.0 * M_PI / p.nphi) * lp;
-  const double phin = (p.nphi == 1) ? 0.0 : (2.0 * M_PI / p.nphi) * ln;
+  const int2 gl = p.gcls[g];
+  const double phip = (2.0 * M_PI / p.nphi) * gl.x;
+  const double phin = (2.0 * M_PI / p.nphi) * gl.y;
   const double2 ep = cexpi(phip), en = cexpi(phin);
   const double2 *const H = p.hoist + (size_t)ul * 7 * nn;
   const double *const Z0 = p.Z + (size_t)q0 * nn;
@@ -359,17 +361,17 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
   double2 *const rowb = AB;                        // Gauss-Jordan row buffers [2][N] (the A-block is free then)
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // XCD-aware order: the nphi^2 workgroups of one unit stay on one XCD (and
+  // XCD-aware order: the ngc workgroups of one unit stay on one XCD (and
   // its L2, where the unit's setup matrices are); gridDim.x is a multiple of 8
   const unsigned L = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (L >= (unsigned)p.nwg) return;
-  const int ng = p.nphi * p.nphi;
+  const int ng = p.ngc;
   const int g = (int)(L % (unsigned)ng), ul = (int)(L / (unsigned)ng), u = p.u0 + ul;
   const int ip = u / p.NE;
   const int q0 = p.q0[ip], q1 = p.q1[ip];
-  const int lp = g / p.nphi, ln = g - lp * p.nphi;
-  const double phip = (p.nphi == 1) ? 0.0 : (2.0 * M_PI / p.nphi) * lp;
-  const double phin = (p.nphi == 1) ? 0.0 : (2.0 * M_PI / p.nphi) * ln;
+  const int2 gl = p.gcls[g];
+  const double phip = (2.0 * M_PI / p.nphi) * gl.x;
+  const double phin = (2.0 * M_PI / p.nphi) * gl.y;
   const double2 ep = cexpi(phip), en = cexpi(phin);
   const double2 *const H = p.hoist + (size_t)ul * 7 * nn;
   const double *const Z0 = p.Z + (size_t)q0 * nn;
@@ -639,7 +641,9 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
 
 // ------------------------------------------------------------------ gauge sum
 struct PSum {
-  int ng, nog, nob2, u0, nunits, NE, nphi, zval, nval;
+  int ng, ngc, nog, nob2, u0, NE, nefull, nphi, zval, nval;
+  const int2 *ecan;
+  const int *gmap;  // [nphi^2]: the gauge pair evaluated, | 1 << 16 as its conjugate
   double vac_scale, snpfaf;
   const int *q0, *q1, *pz, *pn;
   const double *det;
@@ -651,36 +655,50 @@ struct PSum {
 
 // Fomenko sum over the gauge points of one unit: the norm weight
 // znorm = <0|Phi0><0|Phi1> Pf e^{-i (phi_p Z + phi_n N)} times each observable
-// (PNAMP_Kernel3D.f90:262-387), divided by nphi^2.
+// (PNAMP_Kernel3D.f90:262-387), divided by nphi^2; a mirrored Euler point
+// takes the conjugate sums.
 __global__ __launch_bounds__(64) void k_plain_sum(PSum p) {
   __shared__ double2 zn[256];
+  __shared__ int gm[256];
   const int ul = blockIdx.x, u = p.u0 + ul, ip = u / p.NE;
+  const int2 en = p.ecan[u - ip * p.NE];
+  const size_t ue = (size_t)ip * p.nefull + en.x, um = (size_t)ip * p.nefull + (en.y >= 0 ? en.y : en.x);
   const double inv = 1.0 / (double)p.ng;
   const double vac = p.snpfaf * (p.det[p.q0[ip]] * p.vac_scale) * (p.det[p.q1[ip]] * p.vac_scale);
   const double zv = p.pz ? p.pz[ip] : p.zval, nv = p.pn ? p.pn[ip] : p.nval;
   for (int g = threadIdx.x; g < p.ng; g += 64) {
     const int lp = g / p.nphi, ln = g - lp * p.nphi;
-    const double phip = (p.nphi == 1) ? 0.0 : (2.0 * M_PI / p.nphi) * lp;
-    const double phin = (p.nphi == 1) ? 0.0 : (2.0 * M_PI / p.nphi) * ln;
-    zn[g] = cmul(cscale(vac, p.gpf[(size_t)ul * p.ng + g]), cexpi(-phip * zv - phin * nv));
+    const double phip = (2.0 * M_PI / p.nphi) * lp;
+    const double phin = (2.0 * M_PI / p.nphi) * ln;
+    const int m = p.gmap[g];
+    gm[g] = m;
+    double2 pf = p.gpf[(size_t)ul * p.ngc + (m & 0xffff)];
+    if (m >> 16) pf = cconj(pf);
+    zn[g] = cmul(cscale(vac, pf), cexpi(-phip * zv - phin * nv));
   }
   __syncthreads();
-  const double2 *gi = p.gout + (size_t)ul * p.ng * p.nog;
+  const double2 *gi = p.gout + (size_t)ul * p.ngc * p.nog;
   for (int o = threadIdx.x; o < p.nog; o += 64) {
     double2 s = cz();
     for (int g = 0; g < p.ng; ++g) {
       if (o == 0) s = cadd(s, zn[g]);
-      else cfma(s, zn[g], gi[(size_t)g * p.nog + o]);
+      else {
+        double2 v = gi[(size_t)(gm[g] & 0xffff) * p.nog + o];
+        if (gm[g] >> 16) v = cconj(v);
+        cfma(s, zn[g], v);
+      }
     }
     s = cscale(inv, s);
-    if (o < NOBS) p.zres[(size_t)u * NOBS + o] = s;
-    else if (o < NOG_E2) p.ze2[(size_t)u * 10 + (o - NOBS)] = s;
-    else p.zrho[(size_t)u * p.nob2 + (o - NOG_E2)] = s;
+    const double2 sc = (en.y >= 0) ? cconj(s) : s;
+    if (o < NOBS) p.zres[um * NOBS + o] = sc, p.zres[ue * NOBS + o] = s;
+    else if (o < NOG_E2) p.ze2[um * 10 + (o - NOBS)] = sc, p.ze2[ue * 10 + (o - NOBS)] = s;
+    else p.zrho[um * p.nob2 + (o - NOG_E2)] = sc, p.zrho[ue * p.nob2 + (o - NOG_E2)] = s;
   }
   if (threadIdx.x == 0) {
     int st = 0;
-    for (int g = 0; g < p.ng && !st; ++g) st = p.gst[(size_t)ul * p.ng + g];
-    p.status[u] = st;
+    for (int g = 0; g < p.ngc && !st; ++g) st = p.gst[(size_t)ul * p.ngc + g];
+    p.status[um] = st;
+    p.status[ue] = st;
   }
 }
 
@@ -730,7 +748,7 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 bool plain_supported(int n) { return n >= 8 && !(n & 1) && class_of(n) != 0; }
 
 size_t plain_unit_bytes(const PlainArgs &a) {
-  const size_t nn = (size_t)a.n * a.n, ng = (size_t)a.nphi * a.nphi;
+  const size_t nn = (size_t)a.n * a.n, ng = (size_t)a.ngc;
   const size_t nog = a.q2 ? (size_t)NOG_E2 + a.nob2 : (size_t)NOBS;
   return align256(sizeof(double2) * 7 * nn) + align256(sizeof(double2) * ng * nog) + align256(sizeof(int) * ng) +
          align256(sizeof(double2) * ng);
@@ -754,7 +772,7 @@ hipError_t plain_prepare(int n, bool e2) {
 hipError_t plain_run(const PlainArgs &a, int u0, int nu, void *work, hipStream_t s) {
   const int N = class_of(a.n);
   if (!N || nu <= 0) return hipErrorInvalidValue;
-  const size_t nn = (size_t)a.n * a.n, ng = (size_t)a.nphi * a.nphi;
+  const size_t nn = (size_t)a.n * a.n, ng = (size_t)a.ngc;
   const bool e2 = a.q2 != nullptr;
   const int nog = e2 ? NOG_E2 + a.nob2 : NOBS;
   // work buffer: all units' setup matrices, then all gauge outputs, then all gauge status
@@ -763,10 +781,10 @@ hipError_t plain_run(const PlainArgs &a, int u0, int nu, void *work, hipStream_t
   double2 *gout = (double2 *)(w + align256(sizeof(double2) * 7 * nn * nu));
   int *gst = (int *)((char *)gout + align256(sizeof(double2) * ng * nog * nu));
   double2 *gpf = (double2 *)((char *)gst + align256(sizeof(int) * ng * nu));
-  if (ng > 256) return hipErrorInvalidValue;  // nphi <= 16
+  if (a.nphi > 16) return hipErrorInvalidValue;  // nphi <= 16
 
   PSetup sp;
-  sp.n = a.n; sp.h = a.h; sp.nalp = a.nalp; sp.ngam = a.ngam; sp.npack = a.npack; sp.NE = a.NE; sp.u0 = u0;
+  sp.n = a.n; sp.h = a.h; sp.nalp = a.nalp; sp.ngam = a.ngam; sp.npack = a.npack; sp.NE = a.nec; sp.ecan = a.ecan; sp.u0 = u0;
   sp.alp = a.alp; sp.gam = a.gam; sp.rtab = a.rtab; sp.pk_a = a.pk_a; sp.pk_b = a.pk_b;
   sp.blk_off = a.blk_off; sp.blk_sz = a.blk_sz; sp.blk_base = a.blk_base; sp.twom = a.twom;
   sp.q0 = a.q0; sp.q1 = a.q1; sp.U = a.U; sp.V = a.V; sp.Z = a.Z; sp.hoist = hoist;
@@ -775,12 +793,12 @@ hipError_t plain_run(const PlainArgs &a, int u0, int nu, void *work, hipStream_t
   if (err != hipSuccess) return err;
 
   PGauge gp;
-  gp.n = a.n; gp.h = a.h; gp.nphi = a.nphi; gp.NE = a.NE; gp.zval = a.zval; gp.nval = a.nval;
+  gp.n = a.n; gp.h = a.h; gp.nphi = a.nphi; gp.NE = a.nec; gp.ngc = a.ngc; gp.gcls = a.gcls;
   gp.nl = a.nl; gp.lbytes = a.lbytes; gp.nob2 = a.nob2; gp.nog = nog; gp.u0 = u0;
   gp.nwg = (int)(ng * nu);
-  gp.cscale = a.cscale; gp.vac_scale = a.vac_scale; gp.snpfaf = a.snpfaf; gp.e0 = a.e0;
-  gp.q0 = a.q0; gp.q1 = a.q1; gp.pz = a.pz; gp.pn = a.pn;
-  gp.U = a.U; gp.V = a.V; gp.Z = a.Z; gp.det = a.det; gp.hoist = hoist;
+  gp.cscale = a.cscale; gp.e0 = a.e0;
+  gp.q0 = a.q0; gp.q1 = a.q1;
+  gp.U = a.U; gp.V = a.V; gp.Z = a.Z; gp.hoist = hoist;
   gp.mtab = a.mtab; gp.t1b = a.t1b; gp.lofs = a.lofs; gp.lme = a.lme; gp.q2 = a.q2; gp.orbp = a.orbp;
   gp.gout = gout; gp.gst = gst; gp.gpf = gpf;
   const unsigned grid = (unsigned)((ng * nu + 7) / 8 * 8);
@@ -795,7 +813,8 @@ hipError_t plain_run(const PlainArgs &a, int u0, int nu, void *work, hipStream_t
   if (err != hipSuccess) return err;
 
   PSum sm;
-  sm.ng = (int)ng; sm.nog = nog; sm.nob2 = a.nob2; sm.u0 = u0; sm.nunits = nu; sm.NE = a.NE; sm.nphi = a.nphi;
+  sm.ng = a.nphi * a.nphi; sm.ngc = a.ngc; sm.nog = nog; sm.nob2 = a.nob2; sm.u0 = u0;
+  sm.NE = a.nec; sm.nefull = a.NE; sm.ecan = a.ecan; sm.gmap = a.gmap; sm.nphi = a.nphi;
   sm.zval = a.zval; sm.nval = a.nval; sm.vac_scale = a.vac_scale; sm.snpfaf = a.snpfaf;
   sm.q0 = a.q0; sm.q1 = a.q1; sm.pz = a.pz; sm.pn = a.pn; sm.det = a.det;
   sm.gout = gout; sm.gpf = gpf; sm.gst = gst; sm.zres = a.zres; sm.ze2 = a.ze2; sm.zrho = a.zrho; sm.status = a.status;

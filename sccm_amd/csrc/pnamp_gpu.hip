@@ -237,8 +237,40 @@ constexpr int NPHI_MAX = 16;
 constexpr int FAC_OUT = 9;   // per (pair, Euler, species, phi): Pf, E2, Ekin, Tr rho, A, t_+, t_-, t_z, E2 (kappa part, mixed forms)
 constexpr int MIX_FP64 = 0, MIX_FP32 = 1, MIX_BF16 = 2;  // precision of the V contraction
 
+// Euler points and gauge angles that have to be evaluated.  The states are
+// real, so R(2 pi - alpha, beta, 2 pi - gamma) = R(alpha, beta, gamma)* (the
+// two phases of 2 pi m cancel) and every mesh-point quantity at the mirrored
+// Euler point and the gauge angles -phi is the complex conjugate of the one
+// at (alpha, beta, gamma), phi; its gauge sum ZRES is the conjugate.  And
+// T(phi + pi) = -T(phi), S(phi + pi) = S(phi): densities and Pfaffian have
+// period pi in a species' gauge angle.  So of an Euler point and its mirror
+// one is evaluated (ecan: its index and the mirror's, -1 where the mesh has
+// none or the point is its own), at an even number of gauge angles half of
+// them, and where every Euler point is its own mirror (axial meshes, alpha =
+// gamma = 0) only 0 <= phi <= pi (or pi / 2).  The needed angles are the first
+// nd of the nphi Fomenko points; gauge_class names the one that angle f takes
+// and whether as its conjugate.
+// Measured, every point evaluated -> this: pf GCM of 210 pairs (alpha = gamma
+// 10, beta 20, nphi 9) 216.7 -> 114.0 ms, f5pg9 batch (nphi 8) 27.7 -> 8.0 ms,
+// axial pf pairs in the plain form 15.5 -> 8.4 ms.
+struct GaugeClass {
+  int c;
+  bool conj;
+};
+__host__ __device__ __forceinline__ GaugeClass gauge_class(int f, int nphi, int self) {
+  const int half = (nphi & 1) ? nphi : nphi / 2;
+  const int f2 = f % half;
+  return (self && 2 * f2 > half) ? GaugeClass{half - f2, true} : GaugeClass{f2, false};
+}
+__host__ __device__ __forceinline__ int gauge_classes(int nphi, int self) {
+  const int half = (nphi & 1) ? nphi : nphi / 2;
+  return self ? half / 2 + 1 : half;
+}
+__device__ __forceinline__ double2 cconj_if(bool c, double2 a) { return make_double2(a.x, c ? -a.y : a.y); }
+
 struct SetupParams {
-  int n, h, nalp, ngam, npack, NE;
+  int n, h, nalp, ngam, npack, NE;  // NE here and in the other k_fac_* kernels: Euler points evaluated
+  const int2 *ecan;                 // [NE]: Euler index, its mirror's or -1
   const double *alp, *gam;
   const double *Uf, *Vf;            // [nstates][2][h*h], species blocks, column-major
   const double *Z;                  // [nstates][n*n]
@@ -253,7 +285,8 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
   __shared__ double2 sR[RPACK_MAX];
   __shared__ short m_off[HMAX], m_sz[HMAX], m_base[HMAX];
   const int tid = threadIdx.x;
-  const int iang = blockIdx.x, ip = blockIdx.y, sp = blockIdx.z;
+  const int ie = blockIdx.x, ip = blockIdx.y, sp = blockIdx.z;
+  const int iang = p.ecan[ie].x;
   const int n = p.n, h = p.h, hh = h * h;
   const int ig = iang % p.ngam, ia = (iang / p.ngam) % p.nalp, ib = iang / (p.ngam * p.nalp);
   const double alp = p.alp[ia], gam = p.gam[ig];
@@ -279,7 +312,7 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
   }
   __syncthreads();
   double2 *RV1 = sm, *RcU1 = sm + hh, *RZ1 = sm + 2 * hh;
-  double2 *out = p.sbuf + (((size_t)ip * p.NE + iang) * 2 + sp) * 5 * hh;
+  double2 *out = p.sbuf + (((size_t)ip * p.NE + ie) * 2 + sp) * 5 * hh;
   for (int e = tid; e < hh; e += NTS) {
     const int i = e % h, j = e / h;
     const int off = m_off[i], sz = m_sz[i], base = m_base[i];
@@ -317,7 +350,7 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
 }
 
 struct PhiParams {
-  int n, nphi, NE, nwg;
+  int n, nphi, nd, NE, nwg;         // nphi gauge angles, nd of them evaluated
   double cscale;
   const double2 *sbuf;              // k_fac_setup output
   const double *UfT, *VfT;          // [nstates][2][h*h], species blocks, row-major (U_s(j, k) at j h + k)
@@ -537,7 +570,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k
   // block) stay on one XCD and its L2; gridDim.x is a multiple of 8.
   const unsigned L = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (L >= (unsigned)p.nwg) return;
-  const int nphi = p.nphi, n = p.n;
+  const int nphi = p.nd, n = p.n;
   const int f = (int)(L % (unsigned)nphi);
   unsigned t = L / (unsigned)nphi;
   const int sp = (int)(t & 1u);
@@ -549,7 +582,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k
   const int q0 = p.q0[ip];
   const auto V0T = ro_const(p.VfT + ((size_t)q0 * 2 + sp) * HH), U0T = ro_const(p.UfT + ((size_t)q0 * 2 + sp) * HH);
   const double *Z0 = p.Z + (size_t)q0 * n * n + (size_t)sp * H * (n + 1);  // species block, ld n
-  const double phi = (nphi == 1) ? 0.0 : (2.0 * M_PI / nphi) * f;
+  const double phi = (2.0 * M_PI / p.nphi) * f;
   const double2 e1 = cexpi(phi), e2 = cexpi(2.0 * phi);
 
   if constexpr (PART == PART_PF || PART == PART_PFS) {
@@ -942,7 +975,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k
 }
 
 struct CombParams {
-  int h, NE, zval, nval;
+  int h, NE, nphi, self, zval, nval;
+  int nefull;                       // Euler points of the mesh
+  const int2 *ecan;                 // [NE]: Euler index, its mirror's or -1
   double vac_scale, snpfaf, sgn_h, e0;
   const double *det;
   const int *q0, *q1;
@@ -957,9 +992,9 @@ struct CombParams {
   const double2 *out, *rho;
   const int *fstatus;               // [npairs][NE][2][nphi]
   const float2 *gpn;                // mixed forms: G = W_pn rho_n from k_vgemm, [npairs][NE][nphi][h*h]
-  double2 *samples;                 // optional: [npairs][NE][nphi][nphi][2] = norm, energy per gauge pair
-  double2 *zres;                    // [npairs][NE][NOBS]
-  int *status;                      // [npairs][NE]
+  double2 *samples;                 // optional: [npairs][nefull][nphi][nphi][2] = norm, energy per gauge pair
+  double2 *zres;                    // [npairs][nefull][NOBS]
+  int *status;                      // [npairs][nefull]
 };
 
 // One workgroup per (pair, Euler point).  The proton-neutron energy is the
@@ -969,14 +1004,16 @@ struct CombParams {
 // HFB_Energy_COMPLEX reduces to V [rho_p(c,a) rho_n(d,b) + rho_p(a,c) rho_n(b,d)]).
 // G = W rho_n(phi_n) is formed once per phi_n from the dense Delta-m blocks of W, then
 // the nphi^2 dot products with rho_p(phi_p); the gauge points are summed into
-// ZRES.  NP = nphi is a template argument so the per-gauge register arrays
-// stay in registers.  With GMIX (mixed forms) G comes from k_vgemm instead.
+// ZRES.  NP = nd (the gauge angles evaluated) is a template argument so the
+// per-gauge register arrays stay in registers; the dot products also take
+// rho_p* G (four real sums, the same multiply-adds), for the gauge pairs of
+// which one angle is a conjugate.  With GMIX (mixed forms) G comes from k_vgemm instead.
 template <int NP, bool GMIX>
 // (up to nine gauge angles four waves per SIMD: two eight-wave workgroups per
 // CU, as many as their LDS allows; more angles need more than 128 VGPRs)
 __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4 : 2))) void k_fac_combine(CombParams p) {
   extern __shared__ double2 dsm[];  // rho_n -> G [NP][h^2], then the block column lists; rho_p from global memory
-  __shared__ double2 epn[NP * NP];
+  __shared__ double2 epn[NP * NP], epc[NP * NP];  // rho_p^T G, rho_p^+ G
   __shared__ double red[(NTC + 63) / 64 * 2 * NOBS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int iang = blockIdx.x, ip = blockIdx.y;
@@ -1067,9 +1104,9 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
   }
   const int grp = tid >> 5, gl = tid & 31;
   for (int fp = grp; fp < NP; fp += NTC / 32) {
-    double2 acc[NP];
+    double2 acc[NP], acq[NP];  // (re re, im im), (re im, im re)
 #pragma unroll
-    for (int f = 0; f < NP; ++f) acc[f] = cz();
+    for (int f = 0; f < NP; ++f) acc[f] = acq[f] = cz();
     const double2 *rpf = p.rho + (base * NP + fp) * hh;
     // this lane's rho_p elements x = gl + 32 i, eight loads issued together
     // (clamped; weight 0 past h^2)
@@ -1082,41 +1119,71 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
         const int x = x0 + gl + 32 * i, xc = min(x, hh - 1);
         const double2 av = (x < hh) ? ra[i] : cz();
 #pragma unroll
-        for (int f = 0; f < NP; ++f) cfma(acc[f], av, rn[(size_t)f * hh + xc]);
+        for (int f = 0; f < NP; ++f) {
+          const double2 gv = rn[(size_t)f * hh + xc];
+          acc[f].x = fma(av.x, gv.x, acc[f].x);
+          acc[f].y = fma(av.y, gv.y, acc[f].y);
+          acq[f].x = fma(av.x, gv.y, acq[f].x);
+          acq[f].y = fma(av.y, gv.x, acq[f].y);
+        }
       }
     }
 #pragma unroll
     for (int f = 0; f < NP; ++f) {
-      double re = acc[f].x, im = acc[f].y;
+      double re = acc[f].x - acc[f].y, im = acq[f].x + acq[f].y;
+      double rc = acc[f].x + acc[f].y, ic = acq[f].x - acq[f].y;
       for (int off = 16; off > 0; off >>= 1) {
         re += __shfl_xor(re, off);
         im += __shfl_xor(im, off);
       }
       if (gl == 0) epn[fp * NP + f] = make_double2(re, im);
+      if (p.self) {
+        for (int off = 16; off > 0; off >>= 1) {
+          rc += __shfl_xor(rc, off);
+          ic += __shfl_xor(ic, off);
+        }
+        if (gl == 0) epc[fp * NP + f] = make_double2(rc, ic);
+      }
     }
   }
   __syncthreads();
   const double2 *op = p.out + base * NP * FAC_OUT, *on = p.out + (base + 1) * NP * FAC_OUT;
   const double vac = p.snpfaf * p.sgn_h * (p.det[p.q0[ip]] * p.vac_scale) * (p.det[p.q1[ip]] * p.vac_scale);
   double v[2 * NOBS] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int t = tid; t < NP * NP; t += NTC) {
-    const int fp = t / NP, fn = t % NP;
-    const double phip = (NP == 1) ? 0.0 : (2.0 * M_PI / NP) * fp;
-    const double phin = (NP == 1) ? 0.0 : (2.0 * M_PI / NP) * fn;
-    const double2 *a = op + fp * FAC_OUT, *b = on + fn * FAC_OUT;
+  const int nphi = p.nphi;
+  const int2 en = p.ecan[iang];
+  for (int t = tid; t < nphi * nphi; t += NTC) {
+    const int fp = t / nphi, fn = t % nphi;
+    const double phip = (2.0 * M_PI / nphi) * fp;
+    const double phin = (2.0 * M_PI / nphi) * fn;
+    const GaugeClass gp = gauge_class(fp, nphi, p.self), gn = gauge_class(fn, nphi, p.self);
+    double2 a[8], b[8];  // the outputs of the two angles
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      a[k] = cconj_if(gp.conj, op[gp.c * FAC_OUT + k]);
+      b[k] = cconj_if(gn.conj, on[gn.c * FAC_OUT + k]);
+    }
+    const double2 epv = cconj_if(gn.conj, (gp.conj == gn.conj ? epn : epc)[gp.c * NP + gn.c]);
     const double2 zn = cmul(cscale(vac, cmul(a[0], b[0])),
                             cexpi(-phip * (p.pz ? p.pz[ip] : p.zval) - phin * (p.pn ? p.pn[ip] : p.nval)));
     const double2 ekin = cadd(a[2], b[2]);
-    const double2 e2s = cadd(cadd(a[1], b[1]), cadd(a[8], b[8]));
-    const double2 E = cadd(cadd(e2s, epn[fp * NP + fn]), cadd(ekin, make_double2(p.e0, 0.0)));
+    const double2 a8 = cconj_if(gp.conj, op[gp.c * FAC_OUT + 8]), b8 = cconj_if(gn.conj, on[gn.c * FAC_OUT + 8]);
+    const double2 e2s = cadd(cadd(a[1], b[1]), cadd(a8, b8));
+    const double2 E = cadd(cadd(e2s, epv), cadd(ekin, make_double2(p.e0, 0.0)));
     // <J^2> = A_p + A_n + (t_zp + t_zn)^2 + (t_+p + t_+n)(t_-p + t_-n)
     const double2 tzs = cadd(a[7], b[7]);
     const double2 J2 = cadd(cadd(cadd(a[4], b[4]), cmul(tzs, tzs)), cmul(cadd(a[5], b[5]), cadd(a[6], b[6])));
     const double2 o[NOBS] = {zn, cmul(zn, a[3]), cmul(zn, b[3]), cmul(zn, ekin), cmul(zn, E), cmul(zn, J2)};
     if (p.samples) {
-      double2 *sm = p.samples + (((size_t)ip * p.NE + iang) * NP * NP + t) * 2;
+      double2 *sm = p.samples + (((size_t)ip * p.nefull + en.x) * nphi * nphi + t) * 2;
       sm[0] = zn;
       sm[1] = E;
+      if (en.y >= 0) {  // the mirrored Euler point at -phi
+        const int tm = ((nphi - fp) % nphi) * nphi + (nphi - fn) % nphi;
+        sm = p.samples + (((size_t)ip * p.nefull + en.y) * nphi * nphi + tm) * 2;
+        sm[0] = cconj(zn);
+        sm[1] = cconj(E);
+      }
     }
 #pragma unroll
     for (int k = 0; k < NOBS; ++k) {
@@ -1131,8 +1198,8 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
     for (int k = 0; k < 2 * NOBS; ++k) red[wave * 2 * NOBS + k] = v[k];
   __syncthreads();
   if (tid == 0) {
-    const double inv = 1.0 / (double)(NP * NP);
-    double2 *z = p.zres + ((size_t)ip * p.NE + iang) * NOBS;
+    const double inv = 1.0 / (double)(nphi * nphi);
+    double2 *z = p.zres + ((size_t)ip * p.nefull + en.x) * NOBS;
     for (int k = 0; k < NOBS; ++k) {
       double re = 0, im = 0;
       for (int w = 0; w < (NTC + 63) / 64; ++w) {
@@ -1140,10 +1207,12 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
         im += red[w * 2 * NOBS + 2 * k + 1];
       }
       z[k] = make_double2(inv * re, inv * im);
+      if (en.y >= 0) p.zres[((size_t)ip * p.nefull + en.y) * NOBS + k] = make_double2(inv * re, -inv * im);
     }
     int st = 0;
     for (int q = 0; q < 2 * NP && !st; ++q) st = p.fstatus[base * NP + q];
-    p.status[(size_t)ip * p.NE + iang] = st;
+    p.status[(size_t)ip * p.nefull + en.x] = st;
+    if (en.y >= 0) p.status[(size_t)ip * p.nefull + en.y] = st;
   }
 }
 
@@ -1152,10 +1221,13 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
 // k_fac_phi wrote give, per species and gauge angle, tr_s(Q_mu rho_s(phi))
 // (ZQ2, Codes/PNAMP/PNAMP_ME1B.f90:52-75) and the orbit-pair traces
 // sum_m rho(k_a(m), k_b(m)) (ZRho1B_Angles, Codes/PNAMP/PNAMP_Rho1B.f90:13-33).
+// (the densities exist at the nd gauge angles evaluated, gauge_class names the rest)
 // A proton quantity depends on phi_p only, so its gauge sum weighs it with the
 // norm summed over phi_n (and a neutron one with the norm summed over phi_p).
 struct FacE2Params {
-  int n, h, NE, nphi, zval, nval, nob2;
+  int n, h, NE, nphi, nd, self, zval, nval, nob2;
+  int nefull;
+  const int2 *ecan;
   double vac_scale, snpfaf, sgn_h;
   const double *det;
   const int *q0, *q1;
@@ -1173,21 +1245,24 @@ __global__ __launch_bounds__(256) void k_fac_e2(FacE2Params p) {
   __shared__ double2 td[NPHI_MAX][NOB2_MAX];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int iang = blockIdx.x, ip = blockIdx.y;
-  const int h = p.h, hh = h * h, n = p.n, np = p.nphi;
+  const int h = p.h, hh = h * h, n = p.n, np = p.nphi, nd = p.nd;
   const size_t base = ((size_t)ip * p.NE + iang) * 2;
+  const int2 en = p.ecan[iang];
   const double vac = p.snpfaf * p.sgn_h * (p.det[p.q0[ip]] * p.vac_scale) * (p.det[p.q1[ip]] * p.vac_scale);
   for (int t = tid; t < np * np; t += blockDim.x) {
     const int fp = t / np, fn = t % np;
-    const double phip = (np == 1) ? 0.0 : (2.0 * M_PI / np) * fp;
-    const double phin = (np == 1) ? 0.0 : (2.0 * M_PI / np) * fn;
-    const double2 a = p.out[(base * np + fp) * FAC_OUT], b = p.out[((base + 1) * np + fn) * FAC_OUT];
+    const double phip = (2.0 * M_PI / np) * fp;
+    const double phin = (2.0 * M_PI / np) * fn;
+    const GaugeClass gp = gauge_class(fp, np, p.self), gn = gauge_class(fn, np, p.self);
+    const double2 a = cconj_if(gp.conj, p.out[(base * nd + gp.c) * FAC_OUT]),
+                  b = cconj_if(gn.conj, p.out[((base + 1) * nd + gn.c) * FAC_OUT]);
     zn[t] = cmul(cscale(vac, cmul(a, b)),
                  cexpi(-phip * (p.pz ? p.pz[ip] : p.zval) - phin * (p.pn ? p.pn[ip] : p.nval)));
   }
   // one wave per (species, phi): tr_s(Q_mu rho_s(phi)) for the five mu
-  for (int u = wave; u < 2 * np; u += blockDim.x / 64) {
-    const int sp = u / np, f = u % np;
-    const double2 *r = p.rho + ((base + sp) * np + f) * hh;
+  for (int u = wave; u < 2 * nd; u += blockDim.x / 64) {
+    const int sp = u / nd, f = u % nd;
+    const double2 *r = p.rho + ((base + sp) * nd + f) * hh;
     double q[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int e = lane; e < hh; e += 64) {
       const int a = e % h, b = e / h;
@@ -1202,10 +1277,10 @@ __global__ __launch_bounds__(256) void k_fac_e2(FacE2Params p) {
     for (int k = 0; k < 10; ++k) q[k] = wave_sum_dpp(q[k]);
     if (lane < 5) tq[sp][f][lane] = make_double2(q[2 * lane], q[2 * lane + 1]);
   }
-  for (int t = tid; t < np * p.nob2; t += blockDim.x) {
+  for (int t = tid; t < nd * p.nob2; t += blockDim.x) {
     const int f = t / p.nob2, k = t % p.nob2;
     const int4 op = p.orbp[k];
-    const double2 *r = p.rho + ((base + op.x) * np + f) * hh;
+    const double2 *r = p.rho + ((base + op.x) * nd + f) * hh;
     const int fa = op.y - op.x * h, fb = op.z - op.x * h;
     double2 acc = cz();
     for (int m = 0; m < op.w; ++m) acc = cadd(acc, r[(fa + m) + (fb + m) * h]);
@@ -1223,14 +1298,24 @@ __global__ __launch_bounds__(256) void k_fac_e2(FacE2Params p) {
   if (tid < 10) {
     const int sp = tid / 5, mu = tid % 5;
     double2 acc = cz();
-    for (int f = 0; f < np; ++f) acc = cadd(acc, cmul(wsum[sp][f], tq[sp][f][mu]));
-    p.ze2[((size_t)ip * p.NE + iang) * 10 + tid] = cscale(inv, acc);
+    for (int f = 0; f < np; ++f) {
+      const GaugeClass g = gauge_class(f, np, p.self);
+      acc = cadd(acc, cmul(wsum[sp][f], cconj_if(g.conj, tq[sp][g.c][mu])));
+    }
+    acc = cscale(inv, acc);
+    p.ze2[((size_t)ip * p.nefull + en.x) * 10 + tid] = acc;
+    if (en.y >= 0) p.ze2[((size_t)ip * p.nefull + en.y) * 10 + tid] = cconj(acc);
   }
   for (int k = tid; k < p.nob2; k += blockDim.x) {
     const int sp = p.orbp[k].x;
     double2 acc = cz();
-    for (int f = 0; f < np; ++f) acc = cadd(acc, cmul(wsum[sp][f], td[f][k]));
-    p.zrho[((size_t)ip * p.NE + iang) * p.nob2 + k] = cscale(inv, acc);
+    for (int f = 0; f < np; ++f) {
+      const GaugeClass g = gauge_class(f, np, p.self);
+      acc = cadd(acc, cmul(wsum[sp][f], cconj_if(g.conj, td[g.c][k])));
+    }
+    acc = cscale(inv, acc);
+    p.zrho[((size_t)ip * p.nefull + en.x) * p.nob2 + k] = acc;
+    if (en.y >= 0) p.zrho[((size_t)ip * p.nefull + en.y) * p.nob2 + k] = cconj(acc);
   }
 }
 
@@ -2147,6 +2232,12 @@ struct pnamp_ctx {
   std::vector<int> twom_h;
   // mesh
   int nalp = 0, nbet = 0, ngam = 0, nphi = 0, jmax = 0, fold = 0, NE = 0, npj = 0;
+  // Euler points evaluated (the others are their mirrors), and whether every
+  // point is its own mirror; the plain form's gauge pairs evaluated and the map
+  // of all nphi^2 onto them
+  int nec = 0, eself = 0, ngc = 0;
+  int2 *d_ecan = nullptr, *d_gcls = nullptr;
+  int *d_gmap = nullptr;
   double cscale = 1.0, vac_scale = 1.0, snpfaf = 1.0, e0 = 0.0;
   int nme = 0;
   int nstates = 0;
@@ -2390,6 +2481,54 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
   c->jmax = mesh->jmax;
   c->fold = mesh->fold;
   c->NE = mesh->nalp * mesh->nbet * mesh->ngam;
+  {
+    // mirrored Euler points: alpha' = -alpha and gamma' = -gamma modulo 2 pi to
+    // the rounding of the angles (2 ulp of 2 pi: Gauss-Legendre nodes on [0, 2
+    // pi] are symmetric, the one-point mesh is the angle 0); any other mesh
+    // keeps every point
+    auto mirrors = [](int m, const double *x) {
+      std::vector<int> r(m, -1);
+      for (int i = 0; i < m; ++i)
+        for (int j = 0; j < m && r[i] < 0; ++j) {
+          const double d = x[i] + x[j], t = std::fabs(d - 2.0 * M_PI * std::round(d / (2.0 * M_PI)));
+          if (t <= 2.0e-15 && std::fabs(d) <= 4.1 * M_PI) r[i] = j;
+        }
+      for (int i = 0; i < m; ++i)  // repeated angles: only a one-to-one pairing counts
+        if (r[i] >= 0 && r[r[i]] != i) return std::vector<int>(m, -1);
+      return r;
+    };
+    const std::vector<int> ma = mirrors(c->nalp, mesh->alp), mg = mirrors(c->ngam, mesh->gam);
+    std::vector<int2> ec;
+    int self = 1;
+    for (int e = 0; e < c->NE; ++e) {
+      const int ig = e % c->ngam, ia = (e / c->ngam) % c->nalp, ib = e / (c->ngam * c->nalp);
+      const int mi = (ma[ia] < 0 || mg[ig] < 0) ? -1 : (ib * c->nalp + ma[ia]) * c->ngam + mg[ig];
+      if (mi != e) self = 0;
+      if (mi < 0 || mi >= e) ec.push_back(make_int2(e, mi > e ? mi : -1));
+    }
+    c->nec = (int)ec.size();
+    c->eself = self;
+    // plain form: (phi_p, phi_n) ~ (phi_p + pi, phi_n + pi), and ~ (-phi_p,
+    // -phi_n) conjugated where every Euler point is its own mirror
+    const int f = std::min(c->nphi, NPHI_MAX);  // (the kernels refuse more)
+    std::vector<int2> gc;
+    std::vector<int> gm((size_t)f * f, -1);
+    for (int g = 0; g < f * f; ++g) {
+      if (gm[g] >= 0) continue;
+      const int lp = g / f, ln = g % f, k = (int)gc.size();
+      gc.push_back(make_int2(lp, ln));
+      for (int cj = 0; cj <= self; ++cj)
+        for (int sh = 0; sh < ((f & 1) ? 1 : 2); ++sh) {
+          const int a = ((cj ? f - lp : lp) + sh * (f / 2)) % f, b = ((cj ? f - ln : ln) + sh * (f / 2)) % f;
+          if (gm[a * f + b] < 0) gm[a * f + b] = k | (cj << 16);
+        }
+    }
+    c->ngc = (int)gc.size();
+    int re = 0;
+    if ((re = dupload(c, &c->d_ecan, ec.data(), ec.size())) || (re = dupload(c, &c->d_gcls, gc.data(), gc.size())) ||
+        (re = dupload(c, &c->d_gmap, gm.data(), gm.size())))
+      return bail(re, c->err);
+  }
   c->npj = 0;
   for (int J = 0; J <= c->jmax; ++J) c->npj += (2 * J + 1) * (2 * J + 1);
   c->cscale = mesh->cscale;
@@ -2963,6 +3102,7 @@ static PlainArgs plain_args(const pnamp_ctx *c, int zval, int nval, const int *q
                             int *status) {
   PlainArgs a{};
   a.n = c->n; a.h = c->h; a.nalp = c->nalp; a.nbet = c->nbet; a.ngam = c->ngam; a.NE = c->NE; a.nphi = c->nphi;
+  a.nec = c->nec; a.ngc = c->ngc; a.ecan = c->d_ecan; a.gcls = c->d_gcls; a.gmap = c->d_gmap;
   a.npack = c->npack; a.zval = zval; a.nval = nval;
   a.cscale = c->cscale; a.vac_scale = c->vac_scale; a.snpfaf = c->snpfaf; a.e0 = c->e0;
   a.q0 = q0; a.q1 = q1; a.pz = nullptr; a.pn = nullptr;
@@ -3042,14 +3182,16 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     if (hh > ((FAC_HMAX * FAC_HMAX + NTC - 1) / NTC) * NTC)
       return fail(c, PNAMP_E_SIZE, "h^2 exceeds the combine rows per workgroup");
     if (h > FAC_HMAX || (h & 1)) return fail(c, PNAMP_E_SIZE, "factored form: species size h must be even and <= 22");
-    // per pair: rho [NE][2][nphi][h^2], setup blocks [NE][2][5][h^2], per-phi scalars and status;
-    // mixed forms add the GEMM operands (4 x 2 NE nphi columns x kp, 4 bytes per element),
-    // A01 [NE][2][nphi][h^2] and G_pn [NE][nphi][h^2] (FP32 complex); chunks up to 24 GiB
-    const size_t rho_pp = (size_t)c->NE * 2 * c->nphi * hh, sb_pp = (size_t)c->NE * 2 * 5 * hh;
-    const size_t out_pp = (size_t)c->NE * 2 * c->nphi * FAC_OUT, st_pp = (size_t)c->NE * 2 * c->nphi;
-    const size_t cols_pp = (size_t)2 * c->NE * c->nphi;  // GEMM columns per pair and species
+    // per pair, with nec Euler points and nd gauge angles evaluated: rho
+    // [nec][2][nd][h^2], setup blocks [nec][2][5][h^2], per-phi scalars and status;
+    // mixed forms add the GEMM operands (4 x 2 nec nd columns x kp, 4 bytes per element),
+    // A01 [nec][2][nd][h^2] and G_pn [nec][nd][h^2] (FP32 complex); chunks up to 24 GiB
+    const int nd = gauge_classes(c->nphi, c->eself), nec = c->nec;
+    const size_t rho_pp = (size_t)nec * 2 * nd * hh, sb_pp = (size_t)nec * 2 * 5 * hh;
+    const size_t out_pp = (size_t)nec * 2 * nd * FAC_OUT, st_pp = (size_t)nec * 2 * nd;
+    const size_t cols_pp = (size_t)2 * nec * nd;  // GEMM columns per pair and species
     size_t bytes_pp = 16 * (rho_pp + sb_pp + out_pp) + 4 * st_pp;
-    if (mix != MIX_FP64) bytes_pp += 4 * 4 * cols_pp * kp + 16 * rho_pp + 8 * (size_t)c->NE * c->nphi * hh;
+    if (mix != MIX_FP64) bytes_pp += 4 * 4 * cols_pp * kp + 16 * rho_pp + 8 * (size_t)nec * nd * hh;
     const size_t chunk_max = std::max<size_t>(1, ((size_t)24 << 30) / bytes_pp);
     const size_t chunk_t = mix == MIX_FP64 ? std::max<size_t>(1, chunk_max / (size_t)std::max(1, c->tune.chunk_div)) : chunk_max;
     const int chunk = (int)std::min<size_t>((size_t)npairs, chunk_t);
@@ -3073,7 +3215,7 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
           HIPCHK(c, hipMemset(*bufs[b], 0, ncols_cap * kp * eb));
         }
       }
-      if ((r = dalloc(c, &c->d_a01, rho_pp * chunk)) || (r = dalloc(c, &c->d_gpn, (size_t)2 * c->NE * c->nphi * hh * chunk)))
+      if ((r = dalloc(c, &c->d_a01, rho_pp * chunk)) || (r = dalloc(c, &c->d_gpn, (size_t)2 * nec * nd * hh * chunk)))
         return r;
       c->mix_cap = chunk;
       c->mix_cap_mix = mix;
@@ -3083,15 +3225,16 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
         if ((r = upload_vmat(c, q, mix))) return r;
       c->va_mix = mix;
     }
-    if (!combine_attr(c->nphi, comb_lds)) return fail(c, PNAMP_E_SIZE, "factored form supports nphi <= 16");
+    const size_t comb_nd = sizeof(double2) * (size_t)nd * hh + sizeof(int) * (size_t)c->pn_ncol;
+    if (!combine_attr(nd, comb_nd)) return fail(c, PNAMP_E_SIZE, "factored form supports nphi <= 16");
     const size_t setup_lds = sizeof(double2) * 3 * (size_t)hh;
     SetupParams sp;
-    sp.n = c->n; sp.h = h; sp.nalp = c->nalp; sp.ngam = c->ngam; sp.npack = c->npack; sp.NE = c->NE;
+    sp.n = c->n; sp.h = h; sp.nalp = c->nalp; sp.ngam = c->ngam; sp.npack = c->npack; sp.NE = nec; sp.ecan = c->d_ecan;
     sp.alp = c->d_alp; sp.gam = c->d_gam; sp.Uf = c->d_Uf; sp.Vf = c->d_Vf; sp.Z = c->d_Z; sp.rtab = c->d_rtab;
     sp.pk_a = c->d_pk_a; sp.pk_b = c->d_pk_b; sp.blk_off = c->d_blk_off; sp.blk_sz = c->d_blk_sz;
     sp.blk_base = c->d_blk_base; sp.twom = c->d_twom; sp.sbuf = c->d_sbuf;
     PhiParams fp;
-    fp.n = c->n; fp.nphi = c->nphi; fp.NE = c->NE; fp.cscale = c->cscale; fp.sbuf = c->d_sbuf;
+    fp.n = c->n; fp.nphi = c->nphi; fp.nd = nd; fp.NE = nec; fp.cscale = c->cscale; fp.sbuf = c->d_sbuf;
     fp.UfT = c->d_UfT; fp.VfT = c->d_VfT; fp.Z = c->d_Z; fp.t1b = c->d_t1b; fp.mtab = c->d_mtab;
     fp.binv = c->d_binv; fp.pfb = c->d_pfb;
     const bool pfs = c->schur_allowed && c->pfs_any, both = pfs && !c->pfs_all && c->tune.pf_waves == 0;
@@ -3107,7 +3250,7 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     }
     fp.a01 = c->d_a01;
     VGemmParams vp;
-    vp.h = h; vp.nphi = c->nphi; vp.out = c->d_fout;
+    vp.h = h; vp.nphi = nd; vp.out = c->d_fout;
     for (int q = 0; q < NVPROB; ++q) {
       VProblem &P = vp.prob[q];
       const int spc = (q == 4) ? 1 : (q & 1);
@@ -3122,7 +3265,8 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
       P.ncols = 0;
     }
     CombParams cp;
-    cp.h = h; cp.NE = c->NE; cp.zval = zval; cp.nval = nval;
+    cp.h = h; cp.NE = nec; cp.nefull = c->NE; cp.nphi = c->nphi; cp.self = c->eself; cp.ecan = c->d_ecan;
+    cp.zval = zval; cp.nval = nval;
     cp.vac_scale = c->vac_scale; cp.snpfaf = c->snpfaf; cp.sgn_h = (h & 1) ? -1.0 : 1.0; cp.e0 = c->e0;
     cp.det = c->d_det; cp.pn_rows = c->d_pn_rows; cp.pn_blk = c->d_pn_blk; cp.pn_ycol = c->d_pn_ycol;
     cp.pn_w = c->d_pn_w; cp.pn_ncol = c->pn_ncol;
@@ -3134,7 +3278,8 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     const bool direct = samples != nullptr || e2 != nullptr;
     FacE2Params ep;
-    ep.n = c->n; ep.h = h; ep.NE = c->NE; ep.nphi = c->nphi; ep.zval = zval; ep.nval = nval; ep.nob2 = c->nob2;
+    ep.n = c->n; ep.h = h; ep.NE = nec; ep.nphi = c->nphi; ep.nd = nd; ep.self = c->eself;
+    ep.nefull = c->NE; ep.ecan = c->d_ecan; ep.zval = zval; ep.nval = nval; ep.nob2 = c->nob2;
     ep.vac_scale = c->vac_scale; ep.snpfaf = c->snpfaf; ep.sgn_h = (h & 1) ? -1.0 : 1.0; ep.det = c->d_det;
     ep.out = c->d_fout; ep.rho = c->d_frho; ep.q2 = c->d_q2; ep.orbp = c->d_orbp;
     if (direct || !c->fac_graph) {
@@ -3153,23 +3298,23 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
         cp.zres = c->d_zres + (size_t)p0 * c->NE * NOBS;
         cp.status = c->d_status + (size_t)p0 * c->NE;
         if (direct) cp.samples = samples + (size_t)p0 * c->NE * c->nphi * c->nphi * 2;
-        const size_t nwg = (size_t)np * c->NE * 2 * c->nphi;
+        const size_t nwg = (size_t)np * nec * 2 * nd;
         fp.nwg = (int)nwg;
-        hipLaunchKernelGGL(k_fac_setup, dim3(c->NE, np, 2), dim3(NTS), setup_lds, c->stream, sp);
+        hipLaunchKernelGGL(k_fac_setup, dim3(nec, np, 2), dim3(NTS), setup_lds, c->stream, sp);
         launch_phi_h(h, mix, c->tune, pfs ? (both ? 2 : 1) : 0, (unsigned)((nwg + 7) / 8 * 8), c->stream, fp);
         if (mix != MIX_FP64) {
           const int ncols = (int)(cols_pp * np);
           for (int q = 0; q < NVPROB; ++q) vp.prob[q].ncols = ncols;
           launch_vgemm(h, mix, dim3((ncols + 127) / 128, NVPROB), c->stream, vp);
         }
-        launch_combine_np(c->nphi, mix != MIX_FP64, dim3(c->NE, np), comb_lds, c->stream, cp);
+        launch_combine_np(nd, mix != MIX_FP64, dim3(nec, np), comb_nd, c->stream, cp);
         if (e2) {
           ep.q0 = c->d_q0 + p0; ep.q1 = c->d_q1 + p0;
           ep.pz = per_pair ? c->d_pz + p0 : nullptr;
           ep.pn = per_pair ? c->d_pn + p0 : nullptr;
           ep.ze2 = c->d_ze2 + (size_t)p0 * c->NE * 10;
           ep.zrho = c->d_zrho + (size_t)p0 * c->NE * c->nob2;
-          hipLaunchKernelGGL(k_fac_e2, dim3(c->NE, np), dim3(256), 0, c->stream, ep);
+          hipLaunchKernelGGL(k_fac_e2, dim3(nec, np), dim3(256), 0, c->stream, ep);
         }
       }
     }
@@ -3207,9 +3352,9 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     if (e2) {
       pa.q2 = c->d_q2; pa.orbp = c->d_orbp; pa.nob2 = c->nob2; pa.ze2 = c->d_ze2; pa.zrho = c->d_zrho;
     }
-    // units (pair, Euler point) in chunks whose work buffer stays under 4 GiB
-    const size_t ub = plain_unit_bytes(pa), units = (size_t)npairs * c->NE;
-    if (units > (size_t)INT32_MAX / 2) return fail(c, PNAMP_E_SIZE, "too many (pair, Euler point) units in one call");
+    // units (pair, Euler point evaluated) in chunks whose work buffer stays under 4 GiB
+    const size_t ub = plain_unit_bytes(pa), units = (size_t)npairs * c->nec;
+    if ((size_t)npairs * c->NE > (size_t)INT32_MAX / 2) return fail(c, PNAMP_E_SIZE, "too many (pair, Euler point) units in one call");
     const size_t cu = std::max<size_t>(1, std::min(units, ((size_t)4 << 30) / ub));
     if (c->pwork_bytes < cu * ub) {
       free_void(c, &c->d_pwork);
@@ -3417,11 +3562,14 @@ extern "C" int pnamp_kernels_batched_noalloc(pnamp_ctx *c, int npairs, const int
   int *spst = (int *)((char *)sk + al(sizeof(double2) * kper * chunk));
   void *swork = base + half;
   PlainArgs pa = plain_args(c, zval, nval, sq0, sq1, szr, sst);
-  const size_t ub = plain_unit_bytes(pa);
-  if (ub > half)
-    return fail(c, PNAMP_E_SIZE, "one (pair, Euler point) unit needs " + std::to_string(ub) + " bytes of work buffer; " +
-                                     std::to_string(half) + " available");
-  const size_t wu = std::max<size_t>(1, half / ub);  // units per launch
+  // the limit counts all nphi^2 gauge pairs, whatever number of them this
+  // mesh needs evaluated, so that it depends on n and nphi alone
+  PlainArgs pf = pa;
+  pf.ngc = (int)std::min<int64_t>((int64_t)c->nphi * c->nphi, INT32_MAX);
+  if (plain_unit_bytes(pf) > half)
+    return fail(c, PNAMP_E_SIZE, "one (pair, Euler point) unit needs " + std::to_string(plain_unit_bytes(pf)) +
+                                     " bytes of work buffer; " + std::to_string(half) + " available");
+  const size_t wu = std::max<size_t>(1, half / plain_unit_bytes(pa));  // units per launch
   std::vector<int> pst(chunk);
   for (int p0 = 0; p0 < npairs; p0 += chunk) {
     const int np = std::min(chunk, npairs - p0);
@@ -3431,7 +3579,7 @@ extern "C" int pnamp_kernels_batched_noalloc(pnamp_ctx *c, int npairs, const int
     // k_project every kernel and pair-status entry; each k_plain_gauge
     // workgroup writes its own gauge-point slots before k_plain_sum reads
     // them: nothing left by an earlier call is read
-    const size_t units = (size_t)np * c->NE;
+    const size_t units = (size_t)np * c->nec;
     for (size_t u0 = 0; u0 < units; u0 += wu)
       HIPCHK(c, plain_run(pa, (int)u0, (int)std::min(wu, units - u0), swork, c->stream));
     HIPCHK(c, launch_project(c, np, proj_params(c, szr, sst, sk, spst)));
@@ -3711,7 +3859,7 @@ extern "C" void pnamp_destroy(pnamp_ctx *c) {
                   c->d_lofs[0], c->d_lofs[1], c->d_Uf, c->d_Vf, c->d_binv, c->d_pfb, c->d_pfs_ok,
                   c->d_UfT, c->d_VfT, c->d_mtab, c->d_fout, c->d_frho,
                   c->d_sbuf, c->d_fstatus, c->d_pn_rows,
-                  c->d_pn_blk, c->d_pn_ycol, c->d_pn_w};
+                  c->d_pn_blk, c->d_pn_ycol, c->d_pn_w, c->d_ecan, c->d_gcls, c->d_gmap};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   for (int q = 0; q < NVPROB; ++q) {
