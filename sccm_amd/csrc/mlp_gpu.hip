@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs g) {
 // dW = sum over the splits of the partials, in split order; db[o] = sum_b
 // d[b][o] in the order of b.  The first nblk_w workgroups take a dW entry per
 // thread, the others 64 columns of d each: a column is one chain of B
-// dependent additions (14 us at B = 4096), so its values have to be at hand:
+// dependent additions, so its values have to be at hand:
 // the workgroup brings the next 128 rows into registers while one wave adds
 // the current 128 from LDS.  One load per addition straight from memory paid
 // its latency B times: 765 us per layer at B = 4096 (27.7 ms for two epochs

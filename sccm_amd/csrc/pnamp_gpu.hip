@@ -2076,12 +2076,256 @@ __device__ int block_jacobi(double *A, double *Vv, int dim, JacobiLds &L) {
   return sweep;
 }
 
-// (one workgroup of 1024 threads: the matrix streams through L2 every step,
-// so the workgroup's memory parallelism bounds it)
-__global__ __launch_bounds__(1024) void k_jacobi(double *A, double *Vv, int dim, int *nsweeps) {
-  __shared__ JacobiLds L;
-  const int sw = block_jacobi(A, Vv, dim, L);
+// The rotation (c, s) of pair (P, Q), P < Q, that annihilates a_PQ, and t = s /
+// c; (1, 0) and 0 for the pair with the dummy slot.  Every step waits for one
+// of these chains, so its divisions and roots are the hardware estimates
+// refined by Newton-Raphson steps (to an ulp or two: c and s stay a rotation
+// to that; t only has to annihilate a_PQ to its own rounding).
+__device__ __forceinline__ double rsq_nr(double d) {  // 1 / sqrt(d), d >= 1 and below 1e300
+  double r = __builtin_amdgcn_rsq(d);
+  r = fma(r * fma(-d * r, r, 1.0), 0.5, r);
+  return fma(r * fma(-d * r, r, 1.0), 0.5, r);
+}
+__device__ __forceinline__ double2 jacobi_angle(double app, double aqq, double apq, bool real, double &t) {
+  t = 0.0;
+  if (!real || !(fabs(apq) > 1e-300)) return make_double2(1.0, 0.0);
+  const double th = (aqq - app) / (2.0 * apq), h2 = fma(th, th, 1.0);
+  // sqrt(h2) = h2 rsq(h2); beyond 1e140 t = 1 / (2 |th|) to the last bit
+  const double ah = fabs(th), den = (ah < 1.0e140) ? ah + h2 * rsq_nr(h2) : 2.0 * ah;
+  t = (den < 1.0e300) ? rcp_nr(den) : 1.0 / den;
+  t = (th >= 0) ? t : -t;
+  const double c = rsq_nr(fma(t, t, 1.0));
+  return make_double2(c, t * c);
+}
+// Circle method: slots of pair k < m / 2 at a step < m - 1, m slots (even), slot 0 fixed.
+__device__ __forceinline__ int2 jacobi_pair(int k, int step, int m) {
+  int a = step + k, b = step - k;
+  a = (k == 0) ? 0 : 1 + (a >= m - 1 ? a - (m - 1) : a);
+  b = 1 + (b < 0 ? b + (m - 1) : b);
+  return make_int2(min(a, b), max(a, b));
+}
+
+// The same iteration (same pairs, same rotations) with the matrix in LDS: its
+// upper triangle packed, entry (i <= j) at j (j + 1) / 2 + i, dimension m =
+// dim rounded up to even (a dummy row of zeros), so a rotation step touches
+// each 2 x 2 block of a pair of pairs once instead of twice and nothing leaves
+// the CU.  Up to m = 200 (LDS_JACOBI_MAX; 202 would exceed the CU's 160 KB).
+// With the matrix streaming through L2 a solve of one workgroup took 87 ms at
+// dim 180, here 5.1 ms (the mean of a call's three solves), bound by
+// the LDS reads and writes of the blocks.  A thread keeps its blocks (a, b),
+// a < b, of pair indices for the whole run, consecutive threads take
+// consecutive a of one b (consecutive LDS words); the thread that computes a
+// pair's angle also updates its own 2 x 2 block (a_PP - t a_PQ, a_QQ + t a_PQ,
+// 0: no block of another pair reads it).  The rotations of the first logcap
+// sweeps go to log[(sweep (m - 1) + step) (m / 2) + pair]; the eigenvectors are
+// made from it (k_jacobi_vec, k_nos_vec).
+constexpr int JNT = 1024, LDS_JACOBI_MAX = 200, JBLK = 5;
+__host__ __device__ inline size_t jacobi_lds_bytes(int dim) {  // packed matrix, angles, sums
+  const size_t m = (size_t)dim + (dim & 1);
+  return 8 * ((m * (m + 1) / 2 + 1) & ~(size_t)1) + 16 * (m / 2) + 16 * (JNT / 64);
+}
+// jpk(i, j) = max(t_i + j, t_j + i), t_i = i (i + 1) / 2: the larger index's
+// triangle number wins
+// (24-bit products: full rate)
+__device__ __forceinline__ int jtri(int i) { return (int)(__umul24((unsigned)i, (unsigned)i + 1u) >> 1); }
+__device__ __forceinline__ int jpk(int i, int j) { return max(jtri(i) + j, jtri(j) + i); }
+
+__device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = dim + (dim & 1), hp = m / 2, ntri = m * (m + 1) / 2;
+  double *const A = sm;  // 16-byte aligned, as cs and red then are
+  double2 *const cs = (double2 *)(A + ((ntri + 1) & ~1));
+  double2 *const red = cs + hp;
+  // blocks of this thread: the triangle a < b of hp pairs, a <= b' = b - 1 of
+  // hb = hp - 1, folded into a rectangle of he / 2 columns (he = hb rounded up
+  // to even)
+  const int hb = hp - 1, he = hb + (hb & 1);
+  int ab[JBLK];
+#pragma unroll
+  for (int u = 0; u < JBLK; ++u) {
+    const int w = max(he / 2, 1), e = tid + u * JNT, i = e % w, j = e / w;
+    int a = i, b = j - 1;
+    if (j <= i) {
+      a = he - 1 - i;
+      b = he - 1 - j;
+    }
+    ab[u] = (hb > 0 && j <= he && a < hb && b < hb) ? (a | ((b + 1) << 16)) : -1;
+  }
+  int sweep = 0;
+  for (; sweep < 60; ++sweep) {
+    __syncthreads();
+    double off = 0.0, dg = 0.0;
+    for (int j = wave; j < m; j += JNT / 64)
+      for (int i = lane; i < j; i += 64) off = fma(A[jtri(j) + i], A[jtri(j) + i], off);
+    for (int i = tid; i < m; i += JNT) dg = fma(A[jtri(i) + i], A[jtri(i) + i], dg);
+    off = wave_sum_dpp(off);
+    dg = wave_sum_dpp(dg);
+    if (lane == 0) {
+      red[wave].x = off;
+      red[wave].y = dg;
+    }
+    __syncthreads();
+    off = dg = 0.0;
+    for (int w = 0; w < JNT / 64; ++w) {
+      off += red[w].x;
+      dg += red[w].y;
+    }
+    off *= 2.0;
+    if (off <= 1e-30 * (off + dg) || off == 0.0) break;  // uniform: every thread summed the same words
+    for (int step = 0; step < m - 1; ++step) {
+      if (tid < hp) {
+        const int2 p = jacobi_pair(tid, step, m);
+        const int ipp = jtri(p.x) + p.x, iqq = jtri(p.y) + p.y, ipq = jtri(p.y) + p.x;
+        const double app = A[ipp], aqq = A[iqq], apq = A[ipq];
+        double t;
+        const double2 r = jacobi_angle(app, aqq, apq, p.y < dim, t);
+        if (t != 0.0) {
+          A[ipp] = fma(-t, apq, app);
+          A[iqq] = fma(t, apq, aqq);
+          A[ipq] = 0.0;
+        }
+        cs[tid] = r;
+        if (sweep < logcap) log[((size_t)sweep * (m - 1) + step) * hp + tid] = r;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < JBLK; ++u) {
+        if (ab[u] < 0) continue;
+        const int a = ab[u] & 0xffff, b = ab[u] >> 16;
+        const int2 pa = jacobi_pair(a, step, m), pb = jacobi_pair(b, step, m);
+        const double2 ra = cs[a], rb = cs[b];
+        const double ca = ra.x, sa = ra.y, cb = rb.x, sb = rb.y;
+        const int ta = jtri(pa.x), ua = jtri(pa.y), tb = jtri(pb.x), ub = jtri(pb.y);
+        const int ipp = max(ta + pb.x, tb + pa.x), ipq = max(ta + pb.y, ub + pa.x);
+        const int iqp = max(ua + pb.x, tb + pa.y), iqq = max(ua + pb.y, ub + pa.y);
+        const double xpp = A[ipp], xpq = A[ipq], xqp = A[iqp], xqq = A[iqq];
+        const double ypp = cb * xpp - sb * xpq, ypq = sb * xpp + cb * xpq;  // columns: A J
+        const double yqp = cb * xqp - sb * xqq, yqq = sb * xqp + cb * xqq;
+        A[ipp] = ca * ypp - sa * yqp;  // rows: J^T (A J)
+        A[ipq] = ca * ypq - sa * yqq;
+        A[iqp] = sa * ypp + ca * yqp;
+        A[iqq] = sa * ypq + ca * yqq;
+      }
+      __syncthreads();
+    }
+  }
+  return sweep;
+}
+
+// One workgroup, the matrix in LDS; A (dim x dim) receives the eigenvalues on
+// its diagonal.
+__global__ __launch_bounds__(JNT) void k_jacobi_lds(double *A, int dim, double2 *log, int *nsweeps) {
+  extern __shared__ double jsm[];
+  const int m = dim + (dim & 1);
+  for (int j = threadIdx.x >> 6; j < m; j += JNT / 64)
+    for (int i = threadIdx.x & 63; i <= j; i += 64) jsm[j * (j + 1) / 2 + i] = j < dim ? A[i + (size_t)j * dim] : 0.0;
+  const int sw = lds_jacobi(jsm, dim, log, log ? 60 : 0);
+  for (int i = threadIdx.x; i < dim; i += JNT) A[i + (size_t)i * dim] = jsm[jtri(i) + i];
   if (threadIdx.x == 0) *nsweeps = sw;
+}
+
+// Eigenvectors from the logged rotations: V = J_1 J_2 ..., whose rows do not
+// mix, so a workgroup keeps JVR rows in LDS and applies every step to them
+// (thread = pair, the next step's angles in flight).  first: V starts as the
+// unit matrix, else as V (a later part of the log).
+constexpr int JVR = 4;
+__global__ __launch_bounds__(512) void k_jacobi_vec(double *V, int dim, const double2 *log, const int *nsweeps,
+                                                    int first) {
+  extern __shared__ double rows[];  // [JVR][m]
+  const int m = dim + (dim & 1), hp = m / 2, k = threadIdx.x, r0 = blockIdx.x * JVR;
+  for (int e = k; e < JVR * m; e += blockDim.x) {
+    const int r = r0 + e / m, c = e % m;
+    rows[e] = (r < dim && c < dim) ? (first ? (r == c ? 1.0 : 0.0) : V[r + (size_t)c * dim]) : 0.0;
+  }
+  const int ns = *nsweeps * (m - 1);
+  double2 cur = (k < hp && ns > 0) ? log[k] : make_double2(1.0, 0.0);
+  int step = 0;
+  for (int t = 0; t < ns; ++t) {
+    const double2 r = cur;
+    if (k < hp && t + 1 < ns) cur = log[(size_t)(t + 1) * hp + k];
+    __syncthreads();
+    if (k < hp) {
+      const int2 p = jacobi_pair(k, step, m);
+#pragma unroll
+      for (int i = 0; i < JVR; ++i) {
+        const double vp = rows[i * m + p.x], vq = rows[i * m + p.y];
+        rows[i * m + p.x] = r.x * vp - r.y * vq;
+        rows[i * m + p.y] = r.y * vp + r.x * vq;
+      }
+    }
+    step = (step + 1 == m - 1) ? 0 : step + 1;
+  }
+  __syncthreads();
+  for (int e = k; e < JVR * m; e += blockDim.x) {
+    const int r = r0 + e / m, c = e % m;
+    if (r < dim && c < dim) V[r + (size_t)c * dim] = rows[e];
+  }
+}
+
+// Larger matrices (dim > LDS_JACOBI_MAX): one launch per rotation step, A -> B, a 16 x 16 tile of
+// pair blocks per workgroup (its 32 angles computed from A by the workgroup
+// itself), so the step runs on every CU and needs no barrier across them;
+// the diagonal tiles log the angles.
+__global__ __launch_bounds__(256) void k_jacobi_step(const double *A, double *B, int dim, int step, double2 *log) {
+  __shared__ double2 cs[32];
+  __shared__ int2 pq[32];
+  const int m = dim + (dim & 1), hp = m / 2, tid = threadIdx.x;
+  if (tid < 32) {
+    const int k = (tid < 16 ? blockIdx.x : blockIdx.y) * 16 + (tid & 15);
+    if (k < hp) {
+      const int2 p = jacobi_pair(k, step, m);
+      const bool real = p.y < dim;
+      const int Q = real ? p.y : p.x;
+      double t;
+      const double2 r = jacobi_angle(A[p.x + (size_t)p.x * dim], A[Q + (size_t)Q * dim], A[p.x + (size_t)Q * dim], real, t);
+      cs[tid] = r;
+      pq[tid] = p;
+      if (blockIdx.x == blockIdx.y && tid < 16) log[(size_t)step * hp + k] = r;
+    }
+  }
+  __syncthreads();
+  const int ta = tid & 15, tb = 16 + (tid >> 4);
+  if (blockIdx.x * 16 + ta >= (unsigned)hp || blockIdx.y * 16 + (tb - 16) >= (unsigned)hp) return;
+  const int Pa = pq[ta].x, Qa = pq[ta].y, Pb = pq[tb].x, Qb = pq[tb].y;
+  const double ca = cs[ta].x, sa = cs[ta].y, cb = cs[tb].x, sb = cs[tb].y;
+  const bool qa = Qa < dim, qb = Qb < dim;
+  const double xpp = A[Pa + (size_t)Pb * dim];
+  const double xpq = qb ? A[Pa + (size_t)Qb * dim] : 0.0;
+  const double xqp = qa ? A[Qa + (size_t)Pb * dim] : 0.0;
+  const double xqq = (qa && qb) ? A[Qa + (size_t)Qb * dim] : 0.0;
+  const double ypp = cb * xpp - sb * xpq, ypq = sb * xpp + cb * xpq;  // columns: A J
+  const double yqp = cb * xqp - sb * xqq, yqq = sb * xqp + cb * xqq;
+  B[Pa + (size_t)Pb * dim] = ca * ypp - sa * yqp;  // rows: J^T (A J)
+  if (qb) B[Pa + (size_t)Qb * dim] = ca * ypq - sa * yqq;
+  if (qa) B[Qa + (size_t)Pb * dim] = sa * ypp + ca * yqp;
+  if (qa && qb) B[Qa + (size_t)Qb * dim] = sa * ypq + ca * yqq;
+}
+
+// flag = 1 when the off-diagonal norm is below 1e-30 of the total (one workgroup)
+__global__ __launch_bounds__(JNT) void k_jacobi_done(const double *A, int dim, int *flag) {
+  __shared__ double2 red[JNT / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double off = 0.0, dg = 0.0;
+  for (int j = wave; j < dim; j += JNT / 64)
+    for (int i = lane; i < dim; i += 64) {
+      const double x = A[i + (size_t)j * dim];
+      if (i == j) dg = fma(x, x, dg);
+      else off = fma(x, x, off);
+    }
+  for (int o = 32; o > 0; o >>= 1) {
+    off += __shfl_xor(off, o);
+    dg += __shfl_xor(dg, o);
+  }
+  if (lane == 0) red[wave] = make_double2(off, dg);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    off = dg = 0.0;
+    for (int w = 0; w < JNT / 64; ++w) {
+      off += red[w].x;
+      dg += red[w].y;
+    }
+    *flag = (off <= 1e-30 * (off + dg) || off == 0.0) ? 1 : 0;
+  }
 }
 
 // Natural-state scan of PreSolve_HWG (Codes/GCM/GCM_HWG.f90:2-100): block b
@@ -2091,81 +2335,167 @@ __global__ __launch_bounds__(1024) void k_jacobi(double *A, double *Vv, int dim,
 // block of G = R^T H R (M x M).  Per level k < min(kmax, nos): the energy
 // E_k (ascending), the amplitudes f = R(:, :nos) g_k (FF of HNDIAG) and the
 // variance q2 = sum_i [sum_j (H_ij - E_k N_ij) f_j]^2 of mean_variance
-// (:205-254).  work holds nos^2 + nos^2 doubles per block at offset
-// 2 sum_{i <= b} i^2; E and var are [M][kmax].
+// (:205-254).  E and var are [M][kmax].
+// Three launches: k_nos_scan the eigenvalues (LDS, rotations logged, nos <=
+// lim; else block_jacobi in work), k_nos_vec the kmax lowest eigenvectors from
+// the log, k_nos_var the amplitudes and the variance.
+constexpr int NOS_LOGCAP = 24;      // sweeps logged (about ten are needed; a block with more takes block_jacobi)
 struct NosParams {
-  int dim, M, kmax;
+  int dim, M, kmax, lim;
   const double *N, *H, *R, *G;
-  double *work, *E, *var;
+  double *work;                    // [2 nos^2] per block with nos > lim, from offset 0 for nos = lim + 1
+  double2 *log;                    // NOS_LOGCAP (m - 1) m / 2 per block with nos <= lim, m = nos rounded up to even
+  double *x;                       // [M][kmax][M]: eigenvectors g_k
+  int *ord, *sweeps;               // [M][kmax] column of level k; [M]
+  double *E, *var;
 };
+__host__ __device__ inline size_t nos_log_offset(int b) {  // sum over the blocks before b
+  size_t s = 0;
+  for (int i = 0; i < b; ++i) {
+    const size_t m = (size_t)(i + 1) + ((i + 1) & 1);
+    s += NOS_LOGCAP * (m - 1) * (m / 2);
+  }
+  return s;
+}
+__host__ __device__ inline size_t nos_work_offset(int b, int lim) {  // doubles, b >= lim
+  const size_t n = b, l = lim;
+  return 2 * (n * (n + 1) * (2 * n + 1) / 6 - l * (l + 1) * (2 * l + 1) / 6);
+}
 
-__global__ __launch_bounds__(256) void k_nos_scan(NosParams p) {
-  __shared__ JacobiLds L;
-  __shared__ int ord[1024];
-  __shared__ double f[1024], z[1024];
-  const int b = blockIdx.x, nos = b + 1, tid = threadIdx.x, nt = blockDim.x, dim = p.dim;
-  const size_t woff = 2 * ((size_t)b * (b + 1) * (2 * b + 1) / 6);
-  double *A = p.work + woff, *Vv = A + (size_t)nos * nos;
-  for (int e = tid; e < nos * nos; e += nt) A[e] = p.G[(e % nos) + (size_t)(e / nos) * p.M];
+__global__ __launch_bounds__(JNT) void k_nos_scan(NosParams p) {
+  extern __shared__ double jsm[];  // Jacobi part, then the eigenvalues [nos]
+  const int b = p.M - 1 - blockIdx.x;  // the largest blocks first
+  const int nos = b + 1, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool lds = nos <= p.lim;
+  double *const dg = jsm + (lds ? (jacobi_lds_bytes(nos) + 7) / 8 : (sizeof(JacobiLds) + 7) / 8);
+  double *A = nullptr, *Vv = nullptr;
+  int sw = 0;
+  if (lds) {
+    const int m = nos + (nos & 1);
+    for (int j = wave; j < m; j += JNT / 64)
+      for (int i = lane; i <= j; i += 64) jsm[jtri(j) + i] = j < nos ? p.G[i + (size_t)j * p.M] : 0.0;
+    sw = lds_jacobi(jsm, nos, p.log + nos_log_offset(b), NOS_LOGCAP);
+    for (int i = tid; i < nos; i += JNT) dg[i] = jsm[jtri(i) + i];
+  } else {
+    A = p.work + nos_work_offset(b, p.lim);
+    Vv = A + (size_t)nos * nos;
+    for (int e = tid; e < nos * nos; e += JNT) A[e] = p.G[(e % nos) + (size_t)(e / nos) * p.M];
+    __syncthreads();
+    block_jacobi(A, Vv, nos, *(JacobiLds *)jsm);
+    for (int i = tid; i < nos; i += JNT) dg[i] = A[i + (size_t)i * nos];
+  }
+  if (tid == 0) p.sweeps[b] = sw;
   __syncthreads();
-  block_jacobi(A, Vv, nos, L);
-  // ascending order of the eigenvalues (ties by index)
-  for (int i = tid; i < nos; i += nt) {
-    const double ei = A[i + (size_t)i * nos];
+  // ascending order of the eigenvalues (ties by index), zeros for k >= nos
+  for (int k = nos + tid; k < p.kmax; k += JNT) p.E[(size_t)b * p.kmax + k] = p.var[(size_t)b * p.kmax + k] = 0.0;
+  for (int i = tid; i < nos; i += JNT) {
+    const double ei = dg[i];
     int r = 0;
     for (int j = 0; j < nos; ++j) {
-      const double ej = A[j + (size_t)j * nos];
+      const double ej = dg[j];
       r += (ej < ei || (ej == ei && j < i)) ? 1 : 0;
     }
-    ord[r] = i;
-  }
-  __syncthreads();
-  const int kk = min(p.kmax, nos);
-  for (int k = 0; k < p.kmax; ++k) {
-    double *Eo = p.E + (size_t)b * p.kmax + k, *vo = p.var + (size_t)b * p.kmax + k;
-    if (k >= kk) {
-      if (tid == 0) { *Eo = 0.0; *vo = 0.0; }
-      continue;
+    if (r < p.kmax) {
+      p.E[(size_t)b * p.kmax + r] = ei;
+      p.ord[(size_t)b * p.kmax + r] = i;
+      if (!lds)
+        for (int l = 0; l < nos; ++l) p.x[((size_t)b * p.kmax + r) * p.M + l] = Vv[l + (size_t)i * nos];
     }
-    const int col = ord[k];
-    const double ek = A[col + (size_t)col * nos];
-    for (int i = tid; i < dim; i += nt) {
-      double s = 0.0;
-      for (int l = 0; l < nos; ++l) s = fma(p.R[i + (size_t)l * dim], Vv[l + (size_t)col * nos], s);
-      f[i] = s;
-    }
-    __syncthreads();
-    double q = 0.0;
-    for (int i = tid; i < dim; i += nt) {
-      double s = 0.0;
-      for (int j = 0; j < dim; ++j) s = fma(p.H[i + (size_t)j * dim] - ek * p.N[i + (size_t)j * dim], f[j], s);
-      z[i] = s;
-      q = fma(s, s, q);
-    }
-    L.red[tid] = q;
-    __syncthreads();
-    if (tid == 0) {
-      double t = 0.0;
-      for (int i = 0; i < nt; ++i) t += L.red[i];
-      *Eo = ek;
-      *vo = t;
-    }
-    __syncthreads();
   }
 }
 
-// W = R^T H R for R (dim x M) and symmetric H (dim x dim): one thread per (j, k)
-__global__ void k_congruence(const double *H, const double *R, double *W, int dim, int M) {
+// One wave per (block, level): x = J_1 (J_2 (... e_col)), the logged
+// rotations applied from the last to the first to one vector in LDS.
+__global__ __launch_bounds__(64) void k_nos_vec(NosParams p) {
+  __shared__ double x[LDS_JACOBI_MAX];
+  const int b = p.M - 1 - blockIdx.x, nos = b + 1, k = blockIdx.y, lane = threadIdx.x;
+  if (nos > p.lim || k >= nos || p.sweeps[b] > NOS_LOGCAP) return;
+  const int m = nos + (nos & 1), hp = m / 2;
+  const double2 *log = p.log + nos_log_offset(b);
+  const int col = p.ord[(size_t)b * p.kmax + k];
+  for (int i = lane; i < m; i += 64) x[i] = (i == col) ? 1.0 : 0.0;
+  constexpr int NP = (LDS_JACOBI_MAX / 2 + 63) / 64, AH = 8;  // pairs per lane, steps loaded ahead
+  const int ns = p.sweeps[b] * (m - 1);
+  double2 ahead[AH][NP];
+  auto load = [&](int t, double2 (&r)[NP]) {
+#pragma unroll
+    for (int u = 0; u < NP; ++u) r[u] = log[(size_t)max(t, 0) * hp + min(lane + 64 * u, hp - 1)];
+  };
+#pragma unroll
+  for (int i = 0; i < AH; ++i)
+    if (ns > 0) load(ns - 1 - i, ahead[i]);
+  int step = m - 2;
+  for (int t = ns - 1; t >= 0; t -= AH) {
+#pragma unroll
+    for (int i = 0; i < AH; ++i) {
+      if (t - i < 0) break;
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < NP; ++u) {
+        const int q = lane + 64 * u;
+        if (q < hp) {
+          const int2 pr = jacobi_pair(q, step, m);
+          const double xp = x[pr.x], xq = x[pr.y];
+          x[pr.x] = ahead[i][u].x * xp + ahead[i][u].y * xq;
+          x[pr.y] = ahead[i][u].x * xq - ahead[i][u].y * xp;
+        }
+      }
+      load(t - i - AH, ahead[i]);
+      step = step ? step - 1 : m - 2;
+    }
+  }
+  __syncthreads();
+  for (int l = lane; l < nos; l += 64) p.x[((size_t)b * p.kmax + k) * p.M + l] = x[l];
+}
+
+// f = R(:, :nos) g_k and var = sum_i [sum_j (H_ij - E_k N_ij) f_j]^2
+__global__ __launch_bounds__(256) void k_nos_var(NosParams p) {
+  extern __shared__ double f[];  // [dim], then the wave sums
+  const int b = p.M - 1 - blockIdx.x, nos = b + 1, k = blockIdx.y, tid = threadIdx.x, dim = p.dim;
+  if (k >= nos) return;
+  double *const red = f + dim;
+  const double ek = p.E[(size_t)b * p.kmax + k];
+  const double *g = p.x + ((size_t)b * p.kmax + k) * p.M;
+  for (int i = tid; i < dim; i += 256) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int l = 0; l < nos; ++l) s = fma(p.R[i + (size_t)l * dim], g[l], s);
+    f[i] = s;
+  }
+  __syncthreads();
+  double q = 0.0;
+  for (int i = tid; i < dim; i += 256) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int j = 0; j < dim; ++j) s = fma(p.H[i + (size_t)j * dim] - ek * p.N[i + (size_t)j * dim], f[j], s);
+    q = fma(s, s, q);
+  }
+  q = wave_sum_dpp(q);
+  if ((tid & 63) == 0) red[tid >> 6] = q;
+  __syncthreads();
+  if (tid == 0) p.var[(size_t)b * p.kmax + k] = red[0] + red[1] + red[2] + red[3];
+}
+
+// W = R^T H R for R (dim x M) and symmetric H (dim x dim) in two products:
+// X(l, k) = sum_i H(l, i) R(i, k), W(j, k) = sum_l R(l, j) X(l, k); one thread
+// per entry, consecutive threads on consecutive rows
+__global__ void k_congr_x(const double *H, const double *R, double *X, int dim, int M) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= dim * M) return;
+  const int l = e % dim, k = e / dim;
+  double hr = 0.0;
+#pragma unroll 8
+  for (int i = 0; i < dim; ++i) hr = fma(H[l + (size_t)i * dim], R[i + (size_t)k * dim], hr);
+  X[e] = hr;
+}
+__global__ void k_congr_w(const double *R, const double *X, double *W, int dim, int M) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= M * M) return;
   const int j = e % M, k = e / M;
   double s = 0.0;
-  for (int l = 0; l < dim; ++l) {
-    double hr = 0.0;
-    for (int i = 0; i < dim; ++i) hr = fma(H[l + i * dim], R[i + k * dim], hr);
-    s = fma(R[l + j * dim], hr, s);
-  }
-  W[j + k * M] = s;
+#pragma unroll 8
+  for (int l = 0; l < dim; ++l) s = fma(R[l + (size_t)j * dim], X[l + (size_t)k * dim], s);
+  W[j + (size_t)k * M] = s;
 }
 
 __global__ void k_scale_cols(const double *D, const double *w, double *R, int dim, int M) {
@@ -2220,7 +2550,16 @@ void *noalloc_scratch_ptr(int device, std::string &err) {
 }  // namespace
 
 // ====================================================================== host
+// Buffers of the Hill-Wheeler entry points, kept by the context up to HW_KEEP bytes each.
+struct HwSlot {
+  void *p = nullptr;
+  size_t cap = 0;
+};
+// (the rotation log of a scan over M = 200 natural states holds 0.5 GB)
+constexpr size_t HW_KEEP = (size_t)1 << 30;
+
 struct pnamp_ctx {
+  std::vector<HwSlot> hw_slot;
   int device = 0;
   void *scratch = nullptr;  // this device's scratch array (pnamp_kernels_batched_noalloc)
   hipStream_t stream = nullptr;
@@ -3596,20 +3935,92 @@ extern "C" int pnamp_kernels_batched_noalloc(pnamp_ctx *c, int npairs, const int
   return PNAMP_OK;
 }
 
-// Device buffers of one Hill-Wheeler solve, freed on scope exit.
+// Device buffers of one Hill-Wheeler solve: the context's slots, taken in
+// order and grown where too small; on scope exit the ones above HW_KEEP bytes
+// are given back (the others with the context).
 struct HwBufs {
-  std::vector<void *> p;
+  pnamp_ctx *c;
+  size_t next = 0;
+  explicit HwBufs(pnamp_ctx *ctx) : c(ctx) {}
   ~HwBufs() {
-    for (void *x : p)
-      if (x) (void)hipFree(x);
+    for (auto &s : c->hw_slot)
+      if (s.cap > HW_KEEP) {
+        (void)hipFree(s.p);
+        s = HwSlot{};
+      }
   }
   template <class T>
   bool alloc(T **q, size_t cnt) {
-    const hipError_t e = hipMalloc((void **)q, (cnt ? cnt : 1) * sizeof(T));
-    p.push_back(*q);
-    return e == hipSuccess;
+    const size_t bytes = (cnt ? cnt : 1) * sizeof(T);
+    if (next == c->hw_slot.size()) c->hw_slot.emplace_back();
+    HwSlot &s = c->hw_slot[next++];
+    if (s.cap < bytes) {
+      if (s.p) (void)hipFree(s.p);
+      s = HwSlot{};
+      if (hipMalloc(&s.p, bytes) != hipSuccess) {
+        s.p = nullptr;
+        return false;
+      }
+      s.cap = bytes;
+    }
+    *q = (T *)s.p;
+    return true;
   }
 };
+
+// Eigenvalues of the symmetric dA (dim x dim; on its diagonal afterwards) and,
+// where dV is not NULL, its eigenvectors.  Up to LDS_JACOBI_MAX the matrix
+// stays in one workgroup's LDS; beyond, one launch per step and a test of the
+// off-diagonal norm per sweep.
+static int hw_eig(pnamp_ctx *c, HwBufs &B, double *dA, double *dV, int dim) {
+  const int m = dim + (dim & 1), hp = m / 2;
+  const size_t sweep = (size_t)(m - 1) * hp;
+  const dim3 gv((dim + JVR - 1) / JVR), bv((hp + 63) / 64 * 64);
+  const size_t lv = sizeof(double) * JVR * m;
+  double2 *dlog = nullptr;
+  int *dns = nullptr;
+  if (!B.alloc(&dns, 1)) return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
+  if (dim <= LDS_JACOBI_MAX) {
+    if (dV && !B.alloc(&dlog, 60 * sweep)) return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
+    HIPCHK(c, hipFuncSetAttribute((const void *)k_jacobi_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)jacobi_lds_bytes(dim)));
+    hipLaunchKernelGGL(k_jacobi_lds, dim3(1), dim3(JNT), jacobi_lds_bytes(dim), c->stream, dA, dim, dlog, dns);
+    if (dV) hipLaunchKernelGGL(k_jacobi_vec, gv, bv, lv, c->stream, dV, dim, dlog, dns, 1);
+    HIPCHK(c, hipGetLastError());
+    return PNAMP_OK;
+  }
+  double *dB = nullptr;
+  if (!B.alloc(&dB, (size_t)dim * dim) || !B.alloc(&dlog, sweep))
+    return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
+  const int one = 1;
+  HIPCHK(c, hipMemcpyAsync(dns, &one, sizeof(int), hipMemcpyHostToDevice, c->stream));
+  int *dflag = nullptr;
+  if (!B.alloc(&dflag, 1)) return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
+  bool dV_set = false;
+  double *a = dA, *b = dB;
+  const int nt = (hp + 15) / 16;
+  for (int sw = 0; sw < 60; ++sw) {
+    int done = 0;
+    hipLaunchKernelGGL(k_jacobi_done, dim3(1), dim3(JNT), 0, c->stream, a, dim, dflag);
+    HIPCHK(c, hipMemcpyAsync(&done, dflag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (done) break;
+    for (int step = 0; step < m - 1; ++step) {
+      hipLaunchKernelGGL(k_jacobi_step, dim3(nt, nt), dim3(256), 0, c->stream, a, b, dim, step, dlog);
+      std::swap(a, b);
+    }
+    if (dV) hipLaunchKernelGGL(k_jacobi_vec, gv, bv, lv, c->stream, dV, dim, dlog, dns, sw == 0 ? 1 : 0);
+    HIPCHK(c, hipGetLastError());
+    if (sw == 0 && dV) dV_set = true;
+  }
+  if (dV && !dV_set) {  // diagonal from the start: the unit matrix
+    HIPCHK(c, hipMemsetAsync(dns, 0, sizeof(int), c->stream));
+    hipLaunchKernelGGL(k_jacobi_vec, gv, bv, lv, c->stream, dV, dim, dlog, dns, 1);
+  }
+  if (a != dA)
+    HIPCHK(c, hipMemcpyAsync(dA, a, sizeof(double) * (size_t)dim * dim, hipMemcpyDeviceToDevice, c->stream));
+  return PNAMP_OK;
+}
 
 // The first half of HNDIAG (Codes/GCM/GCM_HNDiag.f90:25-77): diagonalise -N
 // (EN descending), keep the M leading natural states with EN(i)/EN(1) >= eps
@@ -3618,17 +4029,16 @@ struct HwBufs {
 static int hw_prepare(pnamp_ctx *c, HwBufs &B, int dim, const double *N, const double *H, double eps, int nos,
                       double *EN, int *Mout, double **dN, double **dH, double **dR, double **dG) {
   const size_t dd = (size_t)dim * dim;
-  double *dA = nullptr, *dV = nullptr, *dD = nullptr, *dw = nullptr;
-  int *dsw = nullptr;
-  if (!B.alloc(&dA, dd) || !B.alloc(&dV, dd) || !B.alloc(dN, dd) || !B.alloc(dH, dd) || !B.alloc(&dsw, 1))
+  double *dA = nullptr, *dV = nullptr, *dD = nullptr, *dw = nullptr, *dX = nullptr;
+  if (!B.alloc(&dA, dd) || !B.alloc(&dV, dd) || !B.alloc(dN, dd) || !B.alloc(dH, dd))
     return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
   std::vector<double> negN(dd);
   for (size_t i = 0; i < dd; ++i) negN[i] = -N[i];
   HIPCHK(c, hipMemcpyAsync(dA, negN.data(), sizeof(double) * dd, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(*dN, N, sizeof(double) * dd, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(*dH, H, sizeof(double) * dd, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_jacobi, dim3(1), dim3(1024), 0, c->stream, dA, dV, dim, dsw);
-  HIPCHK(c, hipGetLastError());
+  const int re = hw_eig(c, B, dA, dV, dim);
+  if (re) return re;
   std::vector<double> A(dd), Vv(dd);
   HIPCHK(c, hipMemcpyAsync(A.data(), dA, sizeof(double) * dd, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(Vv.data(), dV, sizeof(double) * dd, hipMemcpyDeviceToHost, c->stream));
@@ -3648,12 +4058,14 @@ static int hw_prepare(pnamp_ctx *c, HwBufs &B, int dim, const double *N, const d
     w[k] = EN[k];
     for (int i = 0; i < dim; ++i) D[i + (size_t)k * dim] = Vv[i + (size_t)ord[k] * dim];
   }
-  if (!B.alloc(&dD, (size_t)dim * M) || !B.alloc(&dw, M) || !B.alloc(dR, (size_t)dim * M) || !B.alloc(dG, (size_t)M * M))
+  if (!B.alloc(&dD, (size_t)dim * M) || !B.alloc(&dw, M) || !B.alloc(dR, (size_t)dim * M) ||
+      !B.alloc(&dX, (size_t)dim * M) || !B.alloc(dG, (size_t)M * M))
     return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
   HIPCHK(c, hipMemcpyAsync(dD, D.data(), sizeof(double) * D.size(), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(dw, w.data(), sizeof(double) * M, hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL(k_scale_cols, dim3((dim * M + 255) / 256), dim3(256), 0, c->stream, dD, dw, *dR, dim, M);
-  hipLaunchKernelGGL(k_congruence, dim3((M * M + 255) / 256), dim3(256), 0, c->stream, *dH, *dR, *dG, dim, M);
+  hipLaunchKernelGGL(k_congr_x, dim3((dim * M + 255) / 256), dim3(256), 0, c->stream, *dH, *dR, dX, dim, M);
+  hipLaunchKernelGGL(k_congr_w, dim3((M * M + 255) / 256), dim3(256), 0, c->stream, *dR, dX, *dG, dim, M);
   HIPCHK(c, hipGetLastError());
   return PNAMP_OK;
 }
@@ -3663,21 +4075,20 @@ extern "C" int pnamp_hw_solve(pnamp_ctx *c, int dim, const double *N, const doub
   if (!c || dim <= 0 || !N || !H || !EN || !E || !nkept) return PNAMP_E_ARG;
   if (dim > 1022) return fail(c, PNAMP_E_SIZE, "HW dimension above 1022");
   HIPCHK(c, hipSetDevice(c->device));
-  HwBufs B;
+  HwBufs B(c);
   double *dN = nullptr, *dH = nullptr, *dR = nullptr, *dG = nullptr, *dV = nullptr, *dF = nullptr;
-  int *dsw = nullptr;
   int M = 0;
   const int r = hw_prepare(c, B, dim, N, H, eps, nos, EN, &M, &dN, &dH, &dR, &dG);
   if (r) return r;
   *nkept = M;
   if (M <= 0) return 1;
-  if (!B.alloc(&dV, (size_t)M * M) || !B.alloc(&dsw, 1) || (F && !B.alloc(&dF, (size_t)dim * M)))
+  if (F && (!B.alloc(&dV, (size_t)M * M) || !B.alloc(&dF, (size_t)dim * M)))
     return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in pnamp_hw_solve");
-  hipLaunchKernelGGL(k_jacobi, dim3(1), dim3(1024), 0, c->stream, dG, dV, M, dsw);
-  HIPCHK(c, hipGetLastError());
-  std::vector<double> G((size_t)M * M), gv((size_t)M * M);
+  const int re = hw_eig(c, B, dG, dV, M);
+  if (re) return re;
+  std::vector<double> G((size_t)M * M), gv(F ? (size_t)M * M : 0);
   HIPCHK(c, hipMemcpyAsync(G.data(), dG, sizeof(double) * G.size(), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(gv.data(), dV, sizeof(double) * gv.size(), hipMemcpyDeviceToHost, c->stream));
+  if (F) HIPCHK(c, hipMemcpyAsync(gv.data(), dV, sizeof(double) * gv.size(), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   std::vector<int> o2(M);
   for (int i = 0; i < M; ++i) o2[i] = i;
@@ -3703,7 +4114,7 @@ extern "C" int pnamp_hw_presolve(pnamp_ctx *c, int dim, const double *N, const d
     return PNAMP_E_ARG;
   if (dim > 1022) return fail(c, PNAMP_E_SIZE, "HW dimension above 1022");
   HIPCHK(c, hipSetDevice(c->device));
-  HwBufs B;
+  HwBufs B(c);
   double *dN = nullptr, *dH = nullptr, *dR = nullptr, *dG = nullptr, *dwork = nullptr, *dE = nullptr, *dvar = nullptr;
   int M = 0;
   const int r = hw_prepare(c, B, dim, N, H, eps, 0, EN, &M, &dN, &dH, &dR, &dG);
@@ -3714,15 +4125,42 @@ extern "C" int pnamp_hw_presolve(pnamp_ctx *c, int dim, const double *N, const d
     e_best[k] = 0.0;
   }
   if (M <= 0) return 1;
-  const size_t wsz = 2 * ((size_t)M * (M + 1) * (2 * M + 1) / 6);
-  if (!B.alloc(&dwork, wsz) || !B.alloc(&dE, (size_t)M * kmax) || !B.alloc(&dvar, (size_t)M * kmax))
+  int *dord = nullptr, *dsw = nullptr;
+  double *dx = nullptr;
+  double2 *dlog = nullptr;
+  const int kx = std::min(kmax, M);
+  if (!B.alloc(&dE, (size_t)M * kmax) || !B.alloc(&dvar, (size_t)M * kmax) || !B.alloc(&dord, (size_t)M * kmax) ||
+      !B.alloc(&dsw, M) || !B.alloc(&dx, (size_t)M * kmax * M))
     return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in pnamp_hw_presolve");
-  NosParams np{dim, M, kmax, dN, dH, dR, dG, dwork, dE, dvar};
-  hipLaunchKernelGGL(k_nos_scan, dim3(M), dim3(256), 0, c->stream, np);
-  HIPCHK(c, hipGetLastError());
-  HIPCHK(c, hipMemcpyAsync(E, dE, sizeof(double) * (size_t)M * kmax, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(var, dvar, sizeof(double) * (size_t)M * kmax, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  NosParams np{dim, M, kmax, 0, dN, dH, dR, dG, nullptr, nullptr, dx, dord, dsw, dE, dvar};
+  constexpr size_t LDS_CAP = 160 * 1024;
+  auto scan_lds = [](int nos) { return (jacobi_lds_bytes(nos) + 7) / 8 * 8 + sizeof(double) * nos; };
+  while (np.lim < std::min(M, LDS_JACOBI_MAX) && scan_lds(np.lim + 1) <= LDS_CAP) ++np.lim;
+  std::vector<int> sw(M);
+  for (int pass = 0; pass < 2; ++pass) {
+    size_t lds = scan_lds(np.lim);
+    if (M > np.lim) {
+      lds = std::max(lds, (sizeof(JacobiLds) + 7) / 8 * 8 + sizeof(double) * (size_t)M);
+      if (!B.alloc(&dwork, nos_work_offset(M, np.lim)))
+        return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in pnamp_hw_presolve");
+      np.work = dwork;
+    }
+    if (np.lim > 0 && !B.alloc(&dlog, nos_log_offset(np.lim)))
+      return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in pnamp_hw_presolve");
+    np.log = dlog;
+    HIPCHK(c, hipFuncSetAttribute((const void *)k_nos_scan, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_nos_scan, dim3(M), dim3(JNT), lds, c->stream, np);
+    if (np.lim > 0) hipLaunchKernelGGL(k_nos_vec, dim3(M, kx), dim3(64), 0, c->stream, np);
+    hipLaunchKernelGGL(k_nos_var, dim3(M, kx), dim3(256), sizeof(double) * ((size_t)dim + 4), c->stream, np);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipMemcpyAsync(E, dE, sizeof(double) * (size_t)M * kmax, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(var, dvar, sizeof(double) * (size_t)M * kmax, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(sw.data(), dsw, sizeof(int) * M, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    // a block that took more sweeps than the log holds: again without it
+    if (pass || *std::max_element(sw.begin(), sw.end()) <= NOS_LOGCAP) break;
+    np.lim = 0;
+  }
   // PreSolve_HWG's choice (Codes/GCM/GCM_HWG.f90:60-79): per level the NOS of
   // least variance, starting from the reference's initial value 100 and
   // updating on a strictly smaller variance; NOS > M repeat NOS = M
@@ -3874,6 +4312,8 @@ extern "C" void pnamp_destroy(pnamp_ctx *c) {
   void *e2b[] = {c->d_q2, c->d_t3j, c->d_orbscale, c->d_orbp, c->d_ze2, c->d_zrho, c->d_iproj, c->d_qred, c->d_rho1b};
   for (void *b : e2b)
     if (b) (void)hipFree(b);
+  for (auto &hs : c->hw_slot)
+    if (hs.p) (void)hipFree(hs.p);
   if (c->d_a01) (void)hipFree(c->d_a01);
   if (c->d_gpn) (void)hipFree(c->d_gpn);
   for (auto e : c->ev)
