@@ -14,18 +14,10 @@
 // k_plain_gauge then needs only O(n^2) phase work per gauge point before the
 // Pfaffian and the inverse.
 //
+// k_plain_pf: the Pfaffian of the 2n x 2n skew matrix (ZPfaffianF,
+// Codes/PNAMP/PNAMP_Proj.f90:218-350), see there.
 // k_plain_gauge, one workgroup of NTH = 64 ceil(3N/32) threads per gauge
 // point (N the size class of n):
-//   * Pfaffian of the 2n x 2n skew matrix by ZPfaffianF's algorithm
-//     (Codes/PNAMP/PNAMP_Proj.f90:218-350): full pivoting over the trailing
-//     upper triangle (largest |S(i,j)|, first in row-major order on ties),
-//     the two exchanges (NR I1), (NC I2), the rank-2 Schur update, Pf = 0 at
-//     a pivot of modulus <= 1e-13.  The strict upper triangle lives in
-//     registers, entry e in slot e / NTH of thread e % NTH, entries numbered
-//     from the bottom-right corner so the trailing matrix is always the first
-//     m(m-1)/2 entries.  The exchanges are not carried out: the trailing
-//     entries read the old rows NR, NC, I1, I2 (four vectors in LDS) through
-//     the composed transposition.  Two barriers per step.
 //   * T^{-1}: W = [A V1; A* U1] T^{-1} by Gauss-Jordan column operations on the
 //     stacked 3n x n matrix [T; A V1; A* U1] (pivot: largest |re|+|im| in the
 //     current row of T among unused columns, as IZAMAX; the solution columns
@@ -65,12 +57,8 @@ struct PlainCfg {
   static constexpr int NW = (3 * N + 31) / 32;     // waves: 32 stacked rows of [T; A V1; A* U1] each
   static constexpr int NTH = 64 * NW;
   static constexpr int HC = N / 2;                 // columns per thread (half a row)
-  static constexpr int NU = N * (2 * N - 1);       // strict upper entries of the 2N x 2N matrix
-  static constexpr int SL = (NU + NTH - 1) / NTH;  // Pfaffian slots per thread
-  // waves per SIMD the register budgets are fitted to: the Pfaffian kernel's
-  // slots grow as N^2 / NTH, the gauge kernel's register columns as N / 2;
-  // the gauge kernel of N = 64 (133 KB of LDS) runs one workgroup per CU
-  static constexpr int PF_WAVES = N <= 40 ? 4 : (N <= 48 ? 3 : 2);
+  // waves per SIMD the register budget is fitted to: the register columns
+  // grow as N / 2; N = 64 (133 KB of LDS) runs one workgroup per CU
   static constexpr int GAUGE_WAVES = N <= 48 ? 3 : 2;
 };
 
@@ -182,11 +170,6 @@ struct PGauge {
   double2 *gpf;   // [unit - u0][ngc]: Pfaffian of the gauge point's skew matrix
 };
 
-__device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int m) {
-  const unsigned lo = __shfl_xor((unsigned)(v & 0xffffffffull), m), hi = __shfl_xor((unsigned)(v >> 32), m);
-  return ((unsigned long long)hi << 32) | lo;
-}
-
 template <int N>
 __host__ __device__ constexpr size_t gauge_misc_bytes() {
   // wave keys [2][NW] (8 B), reductions [NW][20] (8 B), pivot order [N]
@@ -195,155 +178,215 @@ __host__ __device__ constexpr size_t gauge_misc_bytes() {
   return 16 * PlainCfg<N>::NW + 160 * PlainCfg<N>::NW + 4 * N;
 }
 
-// Pfaffian per gauge point, its own launch: little LDS (the four old rows,
-// 16 n complex) and ~100 VGPRs, so many workgroups per CU hide the serial
-// steps' barriers and reductions.
+// Pfaffian per gauge point: S = cscale [[D M0 D, -1], [1, -Z0]] (Pfaf_Over, 2n x
+// 2n skew) by Parlett-Reid elimination, the pivot of row r = 2k the largest
+// |S(r, c)|, c > r; index c exchanged with r + 1 (sign -1), rank-2 Schur update.
+// The zero rule is ZPfaffianF's: Pf = 0 where no entry left exceeds 1e-13 in
+// modulus.  ZPfaffianF pivots on the largest entry of the whole remaining
+// matrix, a search of every entry in every step; a pivot that is the largest
+// of its row bounds the multipliers S(j, r) / s by one as well.
+//
+// 2D block-cyclic layout over a G x G grid of threads (one wave for 2n <= 48,
+// four above): thread (a, b) holds S(a + G p, b + G q) in slot (p, q), p <= q < T
+// = ceil(2N / G); the diagonal slots hold the whole block (both triangles), so
+// a row or column of the matrix is T slots of one row or column of threads and
+// nothing is indexed at run time but the slot column of c (a uniform switch).
+// Step r: the wave that holds rows r, r + 1 finds c, and writes R = row r / s
+// and A = row r + 1; then every wave knows c and writes column c (C, below the
+// diagonal block from row c with the sign); then row and column c take the
+// place of r + 1 and the trailing slots get S(i, j) += R_i C_j - C_i R_j.  Two
+// barriers per step (none for one wave): R and A of the next step go to the
+// other half of their buffers while slow waves still update.  Entries that
+// left the trailing matrix are updated on with values nobody reads.
+// Bound by VALU issue (G = 8) and the wait of each step for its pivot chain (G =
+// 16, hidden by the other workgroups of the CU).  Against full pivoting with
+// the triangle spread entry by entry over 3n / 32 waves, per gauge point on the
+// whole card: n = 24 41 -> 15 ns, n = 40 168 -> 77 ns, n = 44 570 -> 97 ns, n =
+// 64 1,230 -> 300 ns.
 template <int N>
-__global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_eu(PlainCfg<N>::PF_WAVES))) void k_plain_pf(PGauge p) {
-  using C = PlainCfg<N>;
-  constexpr int NTH = C::NTH, NW = C::NW, SL = C::SL;
-  extern __shared__ double2 lds[];
+struct PfCfg {
+  static constexpr int G = (2 * N <= 48) ? 8 : 16;
+  static constexpr int NT = G * G;
+  static constexpr int T = (2 * N + G - 1) / G, NS = T * (T + 1) / 2;
+  // slots, held R and C, addresses: the waves per SIMD that fit
+  static constexpr int REGS = 4 * NS + 8 * T + 36;
+  static constexpr int WV = REGS <= 102 ? 5 : (REGS <= 128 ? 4 : (REGS <= 168 ? 3 : 2));
+};
+
+template <int N>
+__global__ __launch_bounds__(PfCfg<N>::NT) __attribute__((amdgpu_waves_per_eu(PfCfg<N>::WV))) void k_plain_pf(PGauge p) {
+  using C_ = PfCfg<N>;
+  constexpr int G = C_::G, T = C_::T, NS = C_::NS, KB = (2 * N <= 64) ? 6 : 7;
+  __shared__ double2 vR[2][G * T], vA[2][G * T], vC[G * T], sS[2];
+  __shared__ int sC[2];
   const int n = p.n, h = p.h, nn = n * n, N2 = 2 * n;
-  unsigned long long *const wkey = (unsigned long long *)(lds + 8 * N2);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int a = tid / G, b = tid % G;
   const unsigned L = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (L >= (unsigned)p.nwg) return;
   const int ng = p.ngc;
   const int g = (int)(L % (unsigned)ng), ul = (int)(L / (unsigned)ng), u = p.u0 + ul;
-  const int ip = u / p.NE;
-  const int q0 = p.q0[ip];
+  const int q0 = p.q0[u / p.NE];
   const int2 gl = p.gcls[g];
-  const double phip = (2.0 * M_PI / p.nphi) * gl.x;
-  const double phin = (2.0 * M_PI / p.nphi) * gl.y;
-  const double2 ep = cexpi(phip), en = cexpi(phin);
-  const double2 *const H = p.hoist + (size_t)ul * 7 * nn;
+  const double2 ep = cexpi((2.0 * M_PI / p.nphi) * gl.x), en = cexpi((2.0 * M_PI / p.nphi) * gl.y);
+  const double2 *const M0 = p.hoist + (size_t)ul * 7 * nn + 6 * nn;  // row-major
   const double *const Z0 = p.Z + (size_t)q0 * nn;
-  // ---------------------------------------------------------------- Pfaffian
-  // S = cscale [[D M0 D, -1], [1, -Z0]] (Pfaf_Over, strict upper triangle)
-  double2 pf = make_double2(1.0, 0.0);
+  auto SI = [](int pp, int qq) { return pp * T - pp * (pp - 1) / 2 + (qq - pp); };
+  double2 sv[NS];
   {
-    const int NU = n * (N2 - 1);
-    double2 sv[SL];
-    int sij[SL];
+    // every load unconditional (indices clamped into the blocks), the block chosen by selects
     const double2 e2p = cmul(ep, ep), epn = cmul(ep, en), e2n = cmul(en, en);
 #pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      const int e = s * NTH + tid;
-      double2 v = cz();
-      int ij = 0;
-      if (e < NU) {
-        // row from the bottom t: entries [t(t-1)/2, t(t+1)/2) are row N2-1-t
-        int t = (int)((1.0 + sqrt(1.0 + 8.0 * (double)e)) * 0.5);
-        while (t * (t - 1) / 2 > e) --t;
-        while (t * (t + 1) / 2 <= e) ++t;
-        const int i = N2 - 1 - t, j = i + 1 + (e - t * (t - 1) / 2);
-        ij = i | (j << 8);
-        if (j < n) {
-          const int sidx = (i >= h) + (j >= h);
-          v = cmul(sidx == 0 ? e2p : (sidx == 1 ? epn : e2n), H[6 * nn + (size_t)i * n + j]);
-        }
-        else if (i < n) v = make_double2((j - n == i) ? -1.0 : 0.0, 0.0);
-        else v = make_double2(-Z0[(i - n) + (size_t)(j - n) * n], 0.0);
-        v = cscale(p.cscale, v);
-      }
-      sv[s] = v;
-      sij[s] = ij;
-    }
-    bool zero = false;
-    double2 *const pbuf = lds;  // [2][4][N2]: old rows NR, NC, I1, I2 (R and AB are free here)
-    // pivot key of an entry: |S|^2 with the low 14 mantissa bits replaced by
-    // its row-major rank (largest magnitude, then the first in row-major order)
-    auto pkey = [&](double2 v, int i, int j) -> unsigned long long {
-      const double mag = v.x * v.x + v.y * v.y;
-      return ((unsigned long long)__double_as_longlong(mag) & ~0x3FFFull) | (unsigned long long)(0x3FFF - (i * N2 + j));
-    };
-    // step 0's key and old rows 0, 1 (later steps get theirs from the previous update sweep)
-    unsigned long long key = 0ull;
-    {
-      const int cnt = n * (N2 - 1);
-      double2 *const rNR = pbuf, *const rNC = pbuf + N2;
+    for (int pp = 0; pp < T; ++pp)
 #pragma unroll
-      for (int s = 0; s < SL; ++s) {
-        if (s * NTH < cnt && s * NTH + tid < cnt) {
-          const int i = sij[s] & 255, j = sij[s] >> 8;
-          const double2 v = sv[s];
-          const unsigned long long kk = pkey(v, i, j);
-          key = kk > key ? kk : key;
-          if (i == 0) rNR[j] = v;
-          if (i == 1) rNC[j] = v;
-          if (i == 0 && j == 1) rNC[0] = cneg(v);
-        }
+      for (int qq = pp; qq < T; ++qq) {
+        const int i = a + G * pp, j = b + G * qq, lo = min(i, j), hi = max(i, j);
+        const int ml = min(lo, n - 1), mh = min(hi, n - 1);
+        const double2 m0v = M0[(size_t)ml * n + mh];
+        const double z0v = Z0[min(max(lo - n, 0), n - 1) + (size_t)min(max(hi - n, 0), n - 1) * n];
+        const int sidx = (ml >= h) + (mh >= h);
+        double2 up = cmul(sidx == 0 ? e2p : (sidx == 1 ? epn : e2n), m0v);
+        if (hi >= n) up = (lo < n) ? make_double2((hi - n == lo) ? -1.0 : 0.0, 0.0) : make_double2(-z0v, 0.0);
+        up = (hi < N2 && lo != hi) ? cscale(p.cscale, up) : cz();
+        sv[SI(pp, qq)] = (i < j) ? up : cneg(up);
       }
-    }
-    for (int k = 0; k < n - 1; ++k) {
-      const int NR = 2 * k, NC = NR + 1, m = N2 - NR;
-      const int cnt = m * (m - 1) / 2, cnt2 = (m - 2) * (m - 3) / 2;
-      double2 *const rNR = pbuf + (k & 1) * 4 * N2, *const rNC = rNR + N2, *const rI1 = rNR + 2 * N2,
-                     *const rI2 = rNR + 3 * N2;
-      double2 *const nNR = pbuf + ((k + 1) & 1) * 4 * N2, *const nNC = nNR + N2;  // old rows of step k + 1
-      key = wave_umax64(key);
-      if (lane == 0) wkey[(k & 1) * NW + wave] = key;
-      __syncthreads();
-      unsigned long long best = wkey[(k & 1) * NW];
-      for (int w = 1; w < NW; ++w) {
-        const unsigned long long o = wkey[(k & 1) * NW + w];
-        best = o > best ? o : best;
-      }
-      const int lex = 0x3FFF - (int)(best & 0x3FFFull);
-      const int I1 = lex / N2, I2 = lex - (lex / N2) * N2;
-#pragma unroll
-      for (int s = 0; s < SL; ++s) {
-        if (s * NTH < cnt && s * NTH + tid < cnt) {
-          const int i = sij[s] & 255, j = sij[s] >> 8;
-          const double2 v = sv[s];
-          if (i == I1) rI1[j] = v;
-          if (j == I1) rI1[i] = cneg(v);
-          if (i == I2) rI2[j] = v;
-          if (j == I2) rI2[i] = cneg(v);
-        }
-      }
-      __syncthreads();
-      const double2 ss = rI1[I2];  // S(I1, I2), the pivot after the exchanges
-      if (!(ss.x * ss.x + ss.y * ss.y > 1.0e-26)) {  // |pivot| <= 1e-13
-        zero = true;
-        break;
-      }
-      const double phas = ((I1 == NR) ? -1.0 : 1.0) * ((I2 == NC) ? -1.0 : 1.0);
-      pf = cscale(phas, cmul(pf, ss));
-      const double2 inv = crecip(ss);
-      // composed transposition pi = (NR I1)(NC I2) on the trailing indices:
-      // pi(I1) = NR, pi(I2) = NC (NR if I1 = NC); S'(x, y) = S(pi x, pi y).
-      // The updated entries are step k + 1's trailing matrix: their key and
-      // its old rows NR + 2, NR + 3 are taken in the same sweep.
-      const int pI2 = (I1 == NC) ? NR : NC;
-      key = 0ull;
-#pragma unroll
-      for (int s = 0; s < SL; ++s) {
-        if (s * NTH < cnt2 && s * NTH + tid < cnt2) {
-          const int x = sij[s] & 255, y = sij[s] >> 8;
-          const int px = (x == I1) ? NR : ((x == I2) ? pI2 : x);
-          const int py = (y == I1) ? NR : ((y == I2) ? pI2 : y);
-          double2 base = sv[s];
-          if (px != x) base = (px == NR ? rNR : rNC)[py];
-          else if (py != y) base = cneg((py == NR ? rNR : rNC)[px]);
-          // S(i,j) += (S'(NC,i) S'(NR,j) - S'(NR,i) S'(NC,j)) / S'(NR,NC)
-          double2 t = cmul(rI2[px], rI1[py]);
-          cfms(t, rI1[px], rI2[py]);
-          cfma(base, t, inv);
-          sv[s] = base;
-          const unsigned long long kk = pkey(base, x, y);
-          key = kk > key ? kk : key;
-          if (x == NR + 2) nNR[y] = base;
-          if (x == NR + 3) nNC[y] = base;
-          if (x == NR + 2 && y == NR + 3) nNC[NR + 2] = cneg(base);
-        }
-      }
-    }
-    if (zero) pf = cz();
-    else if (tid == 0) pf = cmul(pf, sv[0]);  // entry 0 is S(2n-2, 2n-1)
-    if (tid == 0) p.gpf[L] = pf;
   }
-
+  double2 pf = make_double2(1.0, 0.0);
+  bool zero = false;
+#pragma unroll
+  for (int P = 0; P < T; ++P) {
+    if (zero || G * P >= N2 - 2) break;
+    for (int t = 0; t < G / 2 && G * P + 2 * t < N2 - 2; ++t) {
+      const int r = G * P + 2 * t, par = t & 1;  // (G / 2 is even: the halves alternate across P too)
+      double2 *const R = vR[par], *const A = vA[par];
+      if (wave == (2 * t * G) >> 6) {  // rows r (a = 2t) and r + 1 are this wave's
+        const int base = (2 * t * G) & 63;  // its lane of thread (2t, 0)
+        unsigned key = 0u;
+#pragma unroll
+        for (int q = P; q < T; ++q) {
+          const int j = b + G * q;
+          const double2 v = sv[SI(P, q)];
+          const unsigned kk = pivot_key_hi<KB>(v.x * v.x + v.y * v.y, j);
+          key = (j > r && j < N2) ? max(key, kk) : key;
+        }
+        key = oct_umax(key);
+        if (G == 16) key = dpp_umax<0x140, 0xF>(key);  // row_mirror
+        key = (unsigned)__builtin_amdgcn_readlane((int)key, base);
+        const int c = (1 << KB) - 1 - (int)(key & ((1u << KB) - 1u));
+        const int Q = c / G, src = base + c % G;
+        double2 s = cz();
+#pragma unroll
+        for (int qq = P; qq < T; ++qq) {
+          if (qq == Q) {
+            const double2 v = sv[SI(P, qq)];
+            const long long bx = __double_as_longlong(v.x), by = __double_as_longlong(v.y);
+            s.x = __longlong_as_double(((long long)__builtin_amdgcn_readlane((int)(bx >> 32), src) << 32) |
+                                       (unsigned)__builtin_amdgcn_readlane((int)bx, src));
+            s.y = __longlong_as_double(((long long)__builtin_amdgcn_readlane((int)(by >> 32), src) << 32) |
+                                       (unsigned)__builtin_amdgcn_readlane((int)by, src));
+          }
+        }
+        const double2 inv = crecip_nr(s);
+        if (a == 2 * t) {
+#pragma unroll
+          for (int q = P; q < T; ++q) {
+            const double2 v = cmul(sv[SI(P, q)], inv);
+            R[b + G * q] = v;
+          }
+          // position c takes index r + 1 (thread (2t, 2t + 1) holds it; after the row's own stores)
+          if (b == 2 * t + 1) R[c] = cmul(sv[SI(P, P)], inv);
+        }
+        if (a == 2 * t + 1) {
+#pragma unroll
+          for (int q = P; q < T; ++q) A[b + G * q] = sv[SI(P, q)];
+        }
+        if (a == 2 * t && b == 0) {
+          sC[par] = c;
+          sS[par] = s;
+        }
+      }
+      __syncthreads();
+      const int c = __builtin_amdgcn_readfirstlane(sC[par]);
+      const double2 s = sS[par];
+      const double s2 = s.x * s.x + s.y * s.y;
+      if (__builtin_amdgcn_readfirstlane((int)!(s2 > 1.0e-26))) {
+        // |pivot| <= 1e-13: Pf = 0 if no entry left is larger (or the row is zero)
+        bool big = false;
+#pragma unroll
+        for (int pp = P; pp < T; ++pp)
+#pragma unroll
+          for (int q = pp; q < T; ++q) {
+            const int i = a + G * pp, j = b + G * q;
+            const double2 v = sv[SI(pp, q)];
+            big = big || (i >= r && j > i && j < N2 && v.x * v.x + v.y * v.y > 1.0e-26);
+          }
+        const int any = __syncthreads_or(big ? 1 : 0);
+        if (!any || !(s2 > 1.0e-290)) {
+          zero = true;
+          break;
+        }
+      }
+      const bool swap = c != r + 1;
+      pf = cmul(pf, swap ? cneg(s) : s);
+      const int Q = c / G, cg = c % G;
+      // column c of the trailing matrix -> C (position c: the exchanged S(r + 1, c))
+      const double2 ac = A[c];
+#pragma unroll
+      for (int qq = P; qq < T; ++qq) {
+        if (qq == Q) {
+          if (b == cg) {
+#pragma unroll
+            for (int pp = P; pp <= qq; ++pp) {
+              double2 v = sv[SI(pp, qq)];
+              v.x = (a + G * pp == c) ? ac.x : v.x;
+              v.y = (a + G * pp == c) ? ac.y : v.y;
+              vC[a + G * pp] = v;
+            }
+          }
+          if (a == cg) {
+#pragma unroll
+            for (int q = qq + 1; q < T; ++q) vC[b + G * q] = cneg(sv[SI(qq, q)]);
+          }
+          // exchange: S'(x, c) = S(x, r + 1) = -A[x], S'(c, y) = A[y]
+          if (swap) {
+            if (b == cg) {
+#pragma unroll
+              for (int pp = P; pp <= qq; ++pp) sv[SI(pp, qq)] = cneg(A[a + G * pp]);
+            }
+            if (a == cg) {
+#pragma unroll
+              for (int q = qq; q < T; ++q) sv[SI(qq, q)] = A[b + G * q];
+            }
+          }
+        }
+      }
+      __syncthreads();
+      double2 Rj[T], Cj[T];
+#pragma unroll
+      for (int q = P; q < T; ++q) {
+        Rj[q] = R[b + G * q];
+        Cj[q] = vC[b + G * q];
+      }
+#pragma unroll
+      for (int pp = P; pp < T; ++pp) {
+        const double2 Ri = R[a + G * pp], Ci = vC[a + G * pp];
+#pragma unroll
+        for (int q = pp; q < T; ++q) {
+          cfms(sv[SI(pp, q)], Ci, Rj[q]);
+          cfma(sv[SI(pp, q)], Ri, Cj[q]);
+        }
+      }
+    }
+  }
+  // the last 2 x 2 block: S(2n - 2, 2n - 1)
+  const int lt = ((N2 - 2) % G) * G + (N2 - 1) % G;
+  if (tid == lt) {
+    double2 v = cz();
+#pragma unroll
+    for (int q = 0; q < T; ++q)
+      if (q == (N2 - 2) / G) v = sv[SI(q, q)];
+    p.gpf[L] = zero ? cz() : cmul(pf, v);
+  }
 }
 
 template <int N, bool E2>
@@ -721,11 +764,6 @@ size_t gauge_lds(int n) {
   return sizeof(double2) * ((size_t)n * (n + 1) + (size_t)n * n) + gauge_misc_bytes<N>();
 }
 
-template <int N>
-size_t pf_lds(int n) {
-  return sizeof(double2) * 16 * (size_t)n + 16 * PlainCfg<N>::NW;
-}
-
 template <int N, bool E2>
 hipError_t prepare_nc(int n) {
   return hipFuncSetAttribute((const void *)k_plain_gauge<N, E2>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -734,7 +772,7 @@ hipError_t prepare_nc(int n) {
 
 template <int N>
 hipError_t launch_gauge(bool e2, unsigned grid, hipStream_t s, const PGauge &gp) {
-  hipLaunchKernelGGL((k_plain_pf<N>), dim3(grid), dim3(PlainCfg<N>::NTH), pf_lds<N>(gp.n), s, gp);
+  hipLaunchKernelGGL((k_plain_pf<N>), dim3(grid), dim3(PfCfg<N>::NT), 0, s, gp);
   const size_t lds = gauge_lds<N>(gp.n);
   if (e2) hipLaunchKernelGGL((k_plain_gauge<N, true>), dim3(grid), dim3(PlainCfg<N>::NTH), lds, s, gp);
   else hipLaunchKernelGGL((k_plain_gauge<N, false>), dim3(grid), dim3(PlainCfg<N>::NTH), lds, s, gp);
