@@ -16,20 +16,17 @@
 //
 // k_plain_pf: the Pfaffian of the 2n x 2n skew matrix (ZPfaffianF,
 // Codes/PNAMP/PNAMP_Proj.f90:218-350), see there.
-// k_plain_gauge, one workgroup of NTH = 64 ceil(3N/32) threads per gauge
-// point (N the size class of n):
+// k_plain_gauge, one workgroup per gauge point:
 //   * T^{-1}: W = [A V1; A* U1] T^{-1} by Gauss-Jordan column operations on the
 //     stacked 3n x n matrix [T; A V1; A* U1] (pivot: largest |re|+|im| in the
 //     current row of T among unused columns, as IZAMAX; the solution columns
-//     come out permuted, the permutation is kept per register column).  Two
-//     threads per stacked row hold one half of its columns each in
-//     registers; one barrier per step (row k of T goes through LDS).
+//     come out permuted);
 //   * rho = W1 V0^T, kappa10 = W1 U0^T, kappa01 = -W2 V0^T
-//     (ROKAPPAphiomega, PNAMP_Proj.f90:459-551) straight from the registers;
-//     rho to LDS, kappa only as A01 = kappa01 - kappa01^T (strict upper) and
-//     A10 / 4 = (kappa10 - kappa10^T) / 4 (strict lower) of one n x n LDS
-//     block, each entry the sum of exactly two LDS atomic adds onto zero
-//     (so the result does not depend on their order).
+//     (ROKAPPAphiomega, PNAMP_Proj.f90:459-551) on the FP64 matrix units; rho
+//     to LDS, kappa only as A01 = kappa01 - kappa01^T (strict upper) and A10 /
+//     4 = (kappa10 - kappa10^T) / 4 (strict lower) of one n x n LDS block, each
+//     entry the sum of exactly two LDS atomic adds onto zero (so the result
+//     does not depend on their order).
 //   * the energy (HFB_Energy_COMPLEX, PNAMP_Energy_OpenMP.f90:5-100) from the
 //     regrouped list: (1/4) V [r_ijkl - r_jikl - r_ijlk + r_jilk + d (...)] =
 //     V [rho_ki rho_lj - rho_li rho_kj + A01_ij A10_kl / 4] + d (kl <-> ij),
@@ -52,14 +49,18 @@ using namespace pnamp_dev;
 constexpr int NOBS = PNAMP_NOBS;
 constexpr int NOG_E2 = NOBS + 10;  // per gauge point: observables, then tr_s(Q_mu rho), then orbit traces
 
+// k_plain_gauge's grid of GR x GC threads (see there) and its tiles.
 template <int N>
 struct PlainCfg {
-  static constexpr int NW = (3 * N + 31) / 32;     // waves: 32 stacked rows of [T; A V1; A* U1] each
-  static constexpr int NTH = 64 * NW;
-  static constexpr int HC = N / 2;                 // columns per thread (half a row)
-  // waves per SIMD the register budget is fitted to: the register columns
-  // grow as N / 2; N = 64 (133 KB of LDS) runs one workgroup per CU
-  static constexpr int GAUGE_WAVES = N <= 48 ? 3 : 2;
+  static constexpr int GC = N <= 24 ? 8 : 16, GR = N == 64 ? 32 : 16;
+  static constexpr int NTH = GR * GC, NW = NTH / 64;
+  static constexpr int TR = (3 * N + GR - 1) / GR, TC = (N + GC - 1) / GC, TP = (N + GR - 1) / GR;
+  // 16 x 16 output tiles of the densities: [W1; W2] V0^T and W1 U0^T
+  static constexpr int MT2 = (2 * N + 15) / 16, MT1 = (N + 15) / 16, NT = (N + 15) / 16;
+  static constexpr int JOBS = (MT2 + MT1) * NT, JW = (JOBS + NW - 1) / NW;
+  // waves per SIMD the registers are fitted to (LDS: 3 workgroups per CU at n =
+  // 40, 2 at n = 44, 1 at n = 64)
+  static constexpr int GAUGE_WAVES = N <= 32 ? 4 : (N <= 40 ? 3 : 2);
 };
 
 // ------------------------------------------------------------------ setup
@@ -172,11 +173,13 @@ struct PGauge {
 
 template <int N>
 __host__ __device__ constexpr size_t gauge_misc_bytes() {
-  // wave keys [2][NW] (8 B), reductions [NW][20] (8 B), pivot order [N]
-  // (4 B): 864 B at N = 40, so three workgroups of n = 40 (52.7 KB) share a
-  // CU's 160 KB
-  return 16 * PlainCfg<N>::NW + 160 * PlainCfg<N>::NW + 4 * N;
+  // pivots [2] (16 B), reductions [NW][20] (8 B), pivot columns [2] and the
+  // solution order [N] (4 B): 840 B at N = 40, so three workgroups of n = 40
+  // (52.7 KB) share a CU's 160 KB
+  return 32 + 160 * PlainCfg<N>::NW + 8 + 4 * N;
 }
+
+typedef double d4 __attribute__((ext_vector_type(4)));
 
 // Pfaffian per gauge point: S = cscale [[D M0 D, -1], [1, -Z0]] (Pfaf_Over, 2n x
 // 2n skew) by Parlett-Reid elimination, the pivot of row r = 2k the largest
@@ -389,21 +392,40 @@ __global__ __launch_bounds__(PfCfg<N>::NT) __attribute__((amdgpu_waves_per_eu(Pf
   }
 }
 
+// The stacked matrix [T; A V1; A* U1] is block-cyclic over the GR x GC threads:
+// thread (a, b) holds rows a + GR p, columns b + GC q in slot (p, q).  Step k
+// (row k of T: thread row k % GR, a compile-time slot row): the wave that holds
+// row k finds the pivot column c and writes R = row k / pivot (R_c = -1 /
+// pivot); then every wave knows c and writes column c (C), which starts again
+// from zero; then slot (p, q) -= C R, from TR + TC LDS reads for TR TC products.
+// Two barriers per step; R has two halves for the waves still updating.  Slot
+// rows of T above row k are left out.  (With a row per two lanes and its
+// columns in registers the pivot column was picked by selects over all register
+// columns and every lane read the whole of row k.)
+// The densities are products with the real V0, U0: W goes to LDS in solution
+// order and 16 x 16 tiles of [W1; W2] V0^T and W1 U0^T run on
+// v_mfma_f64_16x16x4 (its rate equals the vector units', but an operand is read
+// once per 16 results: the vector form read V0 once per result pair and thread).
+// Per gauge point on the whole card, with the list (a row per two lanes, vector
+// densities -> this): n = 24 70 -> 39 ns, n = 40 292 -> 182 ns, n = 44 688 -> 225
+// ns, n = 64 1,960 -> 830 ns.
 template <int N, bool E2>
 __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_eu(PlainCfg<N>::GAUGE_WAVES))) void k_plain_gauge(PGauge p) {
   using C = PlainCfg<N>;
-  constexpr int NTH = C::NTH, NW = C::NW, HC = C::HC;
+  constexpr int NTH = C::NTH, NW = C::NW, GR = C::GR, GC = C::GC, TR = C::TR, TC = C::TC, TP = C::TP, JW = C::JW;
   extern __shared__ double2 lds[];
   const int n = p.n, h = p.h, nn = n * n, ld = n + 1;
   double2 *const R = lds;              // rho, column-major with leading dimension n + 1
   double2 *const AB = lds + n * ld;    // A01 (i < j at i + j n), A10 / 4 (i < j at j + i n)
   char *const misc = (char *)(AB + nn);
-  unsigned long long *const wkey = (unsigned long long *)misc;
-  double *const red = (double *)(misc + 16 * NW);
-  unsigned *const kinv = (unsigned *)(red + 20 * NW);  // [N]: solution index of each pivot column, times 8 n
-  double2 *const rowb = AB;                        // Gauss-Jordan row buffers [2][N] (the A-block is free then)
+  double2 *const sS = (double2 *)misc;             // pivots [2]
+  double *const red = (double *)(misc + 32);
+  int *const sC = (int *)(red + 20 * NW);          // pivot columns [2]
+  int *const kinv = sC + 2;                        // [N]: solution index of each column
+  // Gauss-Jordan vectors, then W, at the front (rho and the A-block come later)
+  double2 *const vR = lds, *const vC = lds + 2 * GC * TC, *const W = lds;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // XCD-aware order: the ngc workgroups of one unit stay on one XCD (and
   // its L2, where the unit's setup matrices are); gridDim.x is a multiple of 8
   const unsigned L = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -411,149 +433,186 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
   const int ng = p.ngc;
   const int g = (int)(L % (unsigned)ng), ul = (int)(L / (unsigned)ng), u = p.u0 + ul;
   const int ip = u / p.NE;
-  const int q0 = p.q0[ip], q1 = p.q1[ip];
+  const int q0 = p.q0[ip];
   const int2 gl = p.gcls[g];
-  const double phip = (2.0 * M_PI / p.nphi) * gl.x;
-  const double phin = (2.0 * M_PI / p.nphi) * gl.y;
-  const double2 ep = cexpi(phip), en = cexpi(phin);
+  const double2 ep = cexpi((2.0 * M_PI / p.nphi) * gl.x), en = cexpi((2.0 * M_PI / p.nphi) * gl.y);
   const double2 *const H = p.hoist + (size_t)ul * 7 * nn;
-  const double *const Z0 = p.Z + (size_t)q0 * nn;
-
-  for (int a = tid; a < N; a += NTH) kinv[a] = 0u;  // padding columns (c >= n) read column 0
 
   // ---------------------------------------------------------------- Gauss-Jordan
-  // stacked row r: T (r < n), A V1 (n <= r < 2n), A* U1 (2n <= r < 3n); lanes
-  // l and l + 32 of a wave hold the two halves of one row
-  const int r = 32 * wave + (lane & 31), hf = lane >> 5;
-  const int kind = (r < n) ? 0 : (r < 2 * n) ? 1 : (r < 3 * n) ? 2 : 3;
-  const int ri = r - (kind < 3 ? kind : 0) * n;
-  double2 col[HC];
+  const int a = tid / GC, b = tid % GC;
+  double2 sv[TR][TC];
   {
     const double2 *Xp = H, *Xn = H + nn, *Yp = H + 2 * nn, *Yn = H + 3 * nn, *RV1 = H + 4 * nn, *RcU1 = H + 5 * nn;
-    const double2 es = (ri >= h) ? en : ep;
-    const double2 ph = (kind == 1) ? es : cconj(es);
 #pragma unroll
-    for (int cc = 0; cc < HC; ++cc) {
-      const int c = hf * HC + cc;
-      double2 v = cz();
-      if (c < n && kind < 3) {
-        const size_t o = (size_t)ri + (size_t)c * n;
-        if (kind == 0) {
-          v = cmul(ep, Xp[o]);
-          cfma(v, en, Xn[o]);
-          cfma(v, cconj(ep), Yp[o]);
-          cfma(v, cconj(en), Yn[o]);
-        } else {
-          v = cmul(ph, (kind == 1 ? RV1 : RcU1)[o]);
+    for (int pp = 0; pp < TR; ++pp) {
+      const int r = a + GR * pp;
+      const int kind = (r < n) ? 0 : (r < 2 * n) ? 1 : (r < 3 * n) ? 2 : 3;
+      const int ri = (kind < 3) ? r - kind * n : 0;
+      const double2 es = (ri >= h) ? en : ep;
+      const double2 ph = (kind == 1) ? es : cconj(es);
+#pragma unroll
+      for (int q = 0; q < TC; ++q) {
+        const int c = b + GC * q;
+        double2 v = cz();
+        if (c < n && kind < 3) {
+          const size_t o = (size_t)ri + (size_t)c * n;
+          if (kind == 0) {
+            v = cmul(ep, Xp[o]);
+            cfma(v, en, Xn[o]);
+            cfma(v, cconj(ep), Yp[o]);
+            cfma(v, cconj(en), Yn[o]);
+          } else {
+            v = cmul(ph, (kind == 1 ? RV1 : RcU1)[o]);
+          }
         }
+        sv[pp][q] = v;
       }
-      col[cc] = v;
     }
   }
   int info = 0;
   unsigned long long used = 0ull;
-  for (int k = 0; k < n; ++k) {
-    double2 *const b = rowb + (k & 1) * N;
-    if (r == k) {
 #pragma unroll
-      for (int cc = 0; cc < HC; ++cc) b[hf * HC + cc] = col[cc];
-    }
-    __syncthreads();
-    // pivot: largest |re| + |im| among unused columns, ties to the smaller
-    // column (one DPP maximum; a NaN entry counts as zero and still leaves an
-    // unused column as the pivot)
-    unsigned pk = 0u;
-    if (lane < n && !((used >> lane) & 1ull)) pk = pivot_key<6>(cabs1(b[lane]), lane);
-    pk = wave_umax(pk);
-    const int cs = 63 - (int)(pk & 63u);
-    used |= 1ull << cs;
-    const double2 piv = b[cs];
-    if (piv.x == 0.0 && piv.y == 0.0 && !info) info = k + 1;
-    const double2 ipv = crecip(piv);
-    const int hs = cs / HC, cl = cs - hs * HC;  // owner half and register column (uniform)
-    double2 x = cz();
+  for (int P = 0; P < TP; ++P) {
+    for (int t = 0; t < GR && GR * P + t < n; ++t) {
+      const int k = GR * P + t, par = t & 1;  // (GR is even: the halves alternate across P too)
+      double2 *const Rk = vR + par * GC * TC;
+      if (wave == (t * GC) >> 6) {
+        const int base = (t * GC) & 63;
+        // pivot: largest |re| + |im| among unused columns, ties to the smaller
+        // column (a NaN entry wins)
+        unsigned key = 0u;
 #pragma unroll
-    for (int cc = 0; cc < HC; ++cc)
-      if (cc == cl) x = col[cc];
-    double2 xlo, xhi;
-    halves2(x, xlo, xhi);
-    const double2 xp = cmul(hs ? xhi : xlo, ipv);  // pivot-column entry of this row (owner half), scaled
-    if (tid == 0) kinv[cs] = (unsigned)(k * n) * 8u;
+        for (int q = 0; q < TC; ++q) {
+          const int j = b + GC * q;
+          const unsigned kk = pivot_key_hi<6>(cabs1(sv[P][q]), j);
+          key = (j < n && !((used >> j) & 1ull)) ? max(key, kk) : key;
+        }
+        key = oct_umax(key);
+        if (GC == 16) key = dpp_umax<0x140, 0xF>(key);  // row_mirror
+        key = (unsigned)__builtin_amdgcn_readlane((int)key, base);
+        const int c = 63 - (int)(key & 63u), Q = c / GC, src = base + c % GC;
+        double2 s = cz();
 #pragma unroll
-    for (int cc = 0; cc < HC; ++cc) {
-      if (cc % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // bounds the LDS reads in flight
-      const double2 f = b[hf * HC + cc];
-      if (cc == cl && hf == hs) col[cc] = xp;
-      else cfms(col[cc], f, xp);
-    }
-  }
-  // solution W(row, k) = col[cc] for the register column cc with pivot order k
-
-  // ---------------------------------------------------------------- densities
-  __syncthreads();  // the row buffers in the A-block are read no more
-  for (int e = tid; e < nn; e += NTH) AB[e] = cz();
-  __syncthreads();
-  {
-    const double *V0 = p.V + (size_t)q0 * nn, *U0 = p.U + (size_t)q0 * nn;
-    const bool w1 = kind == 1, w2 = kind == 2;
-    // outputs in pairs of columns j (n is even); U0 only in waves with W1 rows
-    auto products = [&](auto withu) {
-      constexpr bool WU = decltype(withu)::value;
-#pragma unroll 1
-      for (int j0 = 0; j0 < n; j0 += 2) {
-        double2 a1[2] = {cz(), cz()}, a2[2] = {cz(), cz()};
-#pragma unroll
-        for (int cc = 0; cc < HC; ++cc) {
-          const double2 w = col[cc];
-          const unsigned o = kinv[hf * HC + cc] + (unsigned)j0 * 8u;
-          const double2 v01 = *(const double2 *)((const char *)V0 + o);
-          rfma(a1[0], v01.x, w);
-          rfma(a1[1], v01.y, w);
-          if constexpr (WU) {
-            const double2 u01 = *(const double2 *)((const char *)U0 + o);
-            rfma(a2[0], u01.x, w);
-            rfma(a2[1], u01.y, w);
-          }
-          // at most four columns' loads in flight: the accumulators pass
-          // through an empty asm that also orders memory, so the next
-          // columns' loads wait for these multiply-adds (the scheduler would
-          // otherwise issue all loads first and spill the W row)
-          if (cc % 4 == 3) {
-            __asm__ volatile("" : "+v"(a1[0].x), "+v"(a1[0].y), "+v"(a1[1].x), "+v"(a1[1].y) : : "memory");
-            if constexpr (WU) __asm__ volatile("" : "+v"(a2[0].x), "+v"(a2[0].y), "+v"(a2[1].x), "+v"(a2[1].y) : : "memory");
+        for (int qq = 0; qq < TC; ++qq) {
+          if (qq == Q) {
+            const double2 v = sv[P][qq];
+            const long long bx = __double_as_longlong(v.x), by = __double_as_longlong(v.y);
+            s.x = __longlong_as_double(((long long)__builtin_amdgcn_readlane((int)(bx >> 32), src) << 32) |
+                                       (unsigned)__builtin_amdgcn_readlane((int)bx, src));
+            s.y = __longlong_as_double(((long long)__builtin_amdgcn_readlane((int)(by >> 32), src) << 32) |
+                                       (unsigned)__builtin_amdgcn_readlane((int)by, src));
           }
         }
+        const double2 inv = crecip_nr(s);
+        if (a == t) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          double2 lo, hi;
-          halves2(a1[t], lo, hi);
-          a1[t] = cadd(lo, hi);
-          if constexpr (WU) {
-            halves2(a2[t], lo, hi);
-            a2[t] = cadd(lo, hi);
-          }
-          const int j = j0 + t;
-          if (hf == t) {
-            if (w1) {
-              R[ri + j * ld] = a1[t];  // rho
-              if (ri != j) {           // kappa10 -> A10 / 4
-                const double s = (ri < j) ? 0.25 : -0.25;
-                double *dst = (double *)&AB[(ri < j ? j : ri) + (ri < j ? ri : j) * n];
-                atomicAdd(dst, s * a2[t].x);
-                atomicAdd(dst + 1, s * a2[t].y);
-              }
-            } else if (w2 && ri != j) {  // kappa01 = -a1 -> A01
-              const double s = (ri < j) ? -1.0 : 1.0;
-              double *dst = (double *)&AB[(ri < j ? ri : j) + (ri < j ? j : ri) * n];
-              atomicAdd(dst, s * a1[t].x);
-              atomicAdd(dst + 1, s * a1[t].y);
-            }
+          for (int q = 0; q < TC; ++q) Rk[b + GC * q] = cmul(sv[P][q], inv);
+          if (b == 0) {  // (after the row's own stores)
+            Rk[c] = cneg(inv);
+            sC[par] = c;
+            sS[par] = s;
           }
         }
       }
-    };
-    if (__any(w1)) products(std::true_type{});
-    else if (__any(w2)) products(std::false_type{});
+      __syncthreads();
+      const int c = __builtin_amdgcn_readfirstlane(sC[par]), Q = c / GC, cg = c % GC;
+      used |= 1ull << c;
+      if (tid == 0) {
+        const double2 s = sS[par];
+        if (s.x == 0.0 && s.y == 0.0 && !info) info = k + 1;
+        kinv[c] = k;
+      }
+#pragma unroll
+      for (int qq = 0; qq < TC; ++qq) {
+        if (qq == Q && b == cg) {
+#pragma unroll
+          for (int pp = P; pp < TR; ++pp) {
+            vC[a + GR * pp] = sv[pp][qq];
+            sv[pp][qq] = cz();
+          }
+        }
+      }
+      __syncthreads();
+      double2 Rj[TC];
+#pragma unroll
+      for (int q = 0; q < TC; ++q) Rj[q] = Rk[b + GC * q];
+#pragma unroll
+      for (int pp = P; pp < TR; ++pp) {
+        const double2 Ci = vC[a + GR * pp];
+#pragma unroll
+        for (int q = 0; q < TC; ++q) cfms(sv[pp][q], Ci, Rj[q]);
+      }
+    }
+  }
+  __syncthreads();
+  // W(row, k) in solution order, rows of W1 then W2, column-major
+#pragma unroll
+  for (int pp = 0; pp < TR; ++pp) {
+    const int r = a + GR * pp - n;
+#pragma unroll
+    for (int q = 0; q < TC; ++q) {
+      const int c = b + GC * q;
+      if (r >= 0 && r < 2 * n && c < n) W[r + kinv[c] * 2 * n] = sv[pp][q];
+    }
+  }
+  __syncthreads();
+
+  // ---------------------------------------------------------------- densities
+  // tile jobs of this wave; lane l: A row l % 16, k = l / 16; B column l % 16
+  d4 tre[JW], tim[JW];
+  {
+    const double *V0 = p.V + (size_t)q0 * nn, *U0 = p.U + (size_t)q0 * nn;
+    const double *bp[JW];
+    int ar[JW];
+#pragma unroll
+    for (int w = 0; w < JW; ++w) {
+      const int jb = min(wave * JW + w, C::JOBS - 1), j2 = jb - C::MT2 * C::NT;
+      const int m = j2 < 0 ? jb % C::MT2 : j2 % C::MT1, nt = j2 < 0 ? jb / C::MT2 : j2 / C::MT1;
+      ar[w] = min(16 * m + (lane & 15), 2 * n - 1);
+      bp[w] = (j2 < 0 ? V0 : U0) + min(16 * nt + (lane & 15), n - 1);
+      tre[w] = tim[w] = d4{0.0, 0.0, 0.0, 0.0};
+    }
+    for (int k0 = 0; k0 < n; k0 += 4) {  // (n is a multiple of 4: every species has an even number of states)
+      const int k = k0 + (lane >> 4);
+#pragma unroll
+      for (int w = 0; w < JW; ++w) {
+        const double bv = bp[w][(size_t)k * n];
+        const double2 av = W[ar[w] + k * 2 * n];
+        tre[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, bv, tre[w], 0, 0, 0);
+        tim[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, bv, tim[w], 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();  // W is read no more
+  for (int e = tid; e < nn; e += NTH) AB[e] = cz();
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < JW; ++w) {
+    const int jb = wave * JW + w, j2 = jb - C::MT2 * C::NT;
+    const int m = j2 < 0 ? jb % C::MT2 : j2 % C::MT1, nt = j2 < 0 ? jb / C::MT2 : j2 / C::MT1;
+    const int j = 16 * nt + (lane & 15);
+    if (jb >= C::JOBS || j >= n) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = 16 * m + 4 * v + (lane >> 4);  // D: row 4 v + l / 16, column l % 16
+      const double2 x = make_double2(tre[w][v], tim[w][v]);
+      if (j2 < 0) {
+        if (r < n) {
+          R[r + j * ld] = x;  // rho
+        } else if (r < 2 * n && r - n != j) {  // kappa01 = -x -> A01
+          const int i = r - n;
+          const double sg = (i < j) ? -1.0 : 1.0;
+          double *dst = (double *)&AB[min(i, j) + max(i, j) * n];
+          atomicAdd(dst, sg * x.x);
+          atomicAdd(dst + 1, sg * x.y);
+        }
+      } else if (r < n && r != j) {  // kappa10 -> A10 / 4
+        const double sg = (r < j) ? 0.25 : -0.25;
+        double *dst = (double *)&AB[max(r, j) + min(r, j) * n];
+        atomicAdd(dst, sg * x.x);
+        atomicAdd(dst + 1, sg * x.y);
+      }
+    }
   }
   __syncthreads();
 
