@@ -46,6 +46,8 @@ namespace {
 
 using namespace pnamp_dev;
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+
 constexpr int NOBS = PNAMP_NOBS;
 constexpr int NOG_E2 = NOBS + 10;  // per gauge point: observables, then tr_s(Q_mu rho), then orbit traces
 
@@ -76,33 +78,44 @@ struct PSetup {
 
 constexpr int RPK = 256;  // packed rotation entries (per species) held in LDS
 
+// One workgroup per (unit, 16 columns): R~ V1, R~* U1 and X, Y of its columns, M0
+// of the rows of the same numbers, so a few units still fill the card.  X_s =
+// V0^T P_s (R~ V1) and Y_s run on v_mfma_f64_16x16x4, a wave per 16 rows (a V0
+// element is read once per 16 columns instead of once per column, the columns
+// from LDS).  With one workgroup per unit and a thread per element, 45 units of
+// n = 64 took 224 us and 432 units of n = 40 83 us; now 28 and 46 us.
+constexpr int SC = 16, SLD = SC + 1;
+__host__ __device__ constexpr size_t setup_lds(int n) { return sizeof(double2) * (2 * (size_t)n * SLD + SC * ((size_t)n + 1)); }
+
 __global__ __launch_bounds__(256) void k_plain_setup(PSetup p) {
   extern __shared__ double2 lds[];
-  __shared__ double2 sR[RPK];
+  __shared__ double2 sR[RPK], ea[32], eg[32];
   __shared__ short m_off[32], m_sz[32], m_base[32];
   const int tid = threadIdx.x, n = p.n, h = p.h, nn = n * n;
   const int ul = blockIdx.x, u = p.u0 + ul, ip = u / p.NE, iang = p.ecan[u - ip * p.NE].x;
+  const int c0 = blockIdx.y * SC, cw = min(SC, n - c0);
   const int ig = iang % p.ngam, ia = (iang / p.ngam) % p.nalp, ib = iang / (p.ngam * p.nalp);
   const double alp = p.alp[ia], gam = p.gam[ig];
   const int q0 = p.q0[ip], q1 = p.q1[ip];
   const double *V0 = p.V + (size_t)q0 * nn, *U0 = p.U + (size_t)q0 * nn;
   const double *V1 = p.V + (size_t)q1 * nn, *U1 = p.U + (size_t)q1 * nn, *Z1 = p.Z + (size_t)q1 * nn;
   double2 *out = p.hoist + (size_t)ul * 7 * nn;
-  double2 *sA = lds, *sB = lds + nn;  // R~V1, R~*U1; later R~ Z1 in sA
+  double2 *const sA = lds, *const sB = lds + n * SLD, *const sZ = lds + 2 * n * SLD;  // R~V1, R~*U1 (row * SLD + column), rows of R~ Z1
+  // R(a, b) = exp(-i alp m_a) d(beta)_{ab} exp(-i gam m_b) (ROTATION_MAT, PNAMP_Proj.f90:83-136)
   for (int i = tid; i < h; i += 256) {
     m_off[i] = (short)p.blk_off[i];
     m_sz[i] = (short)p.blk_sz[i];
     m_base[i] = (short)p.blk_base[i];
-  }
-  // R(a, b) = exp(-i alp m_a) d(beta)_{ab} exp(-i gam m_b) (ROTATION_MAT, PNAMP_Proj.f90:83-136)
-  for (int e = tid; e < p.npack; e += 256) {
-    const int a = p.pk_a[e], b = p.pk_b[e];
-    sR[e] = cscale(p.rtab[(size_t)ib * p.npack + e], cexpi(-alp * 0.5 * p.twom[a] - gam * 0.5 * p.twom[b]));
+    ea[i] = cexpi(-alp * 0.5 * p.twom[i]);
+    eg[i] = cexpi(-gam * 0.5 * p.twom[i]);
   }
   __syncthreads();
-  // R~ V1, R~* U1 (block-sparse rows)
-  for (int e = tid; e < nn; e += 256) {
-    const int i = e % n, j = e / n;
+  for (int e = tid; e < p.npack; e += 256)
+    sR[e] = cscale(p.rtab[(size_t)ib * p.npack + e], cmul(ea[p.pk_a[e]], eg[p.pk_b[e]]));
+  __syncthreads();
+  // R~ V1, R~* U1 (block-sparse rows), 16 columns
+  for (int e = tid; e < n * cw; e += 256) {
+    const int jl = e / n, i = e - jl * n, j = c0 + jl;
     const int sp = i >= h, il = i - sp * h;
     const int off = m_off[il], sz = m_sz[il], base = m_base[il];
     double2 a = cz(), b = cz();
@@ -112,44 +125,57 @@ __global__ __launch_bounds__(256) void k_plain_setup(PSetup p) {
       rfma(a, V1[row + j * n], r);
       rfma(b, U1[row + j * n], cconj(r));
     }
-    sA[e] = a;
-    sB[e] = b;
-    out[4 * nn + e] = a;
-    out[5 * nn + e] = b;
+    sA[i * SLD + jl] = a;
+    sB[i * SLD + jl] = b;
+    out[4 * nn + i + j * n] = a;
+    out[5 * nn + i + j * n] = b;
   }
-  __syncthreads();
-  // X_s(a, c) = sum_{i in s} V0(i, a) (R~V1)(i, c), Y_s likewise with U0, R~*U1
-  for (int e = tid; e < nn; e += 256) {
-    const int a = e % n, c = e / n;
-    double2 x[2] = {cz(), cz()}, y[2] = {cz(), cz()};
-    for (int s = 0; s < 2; ++s)
-      for (int i = s * h; i < (s + 1) * h; ++i) {
-        rfma(x[s], V0[i + a * n], sA[i + c * n]);
-        rfma(y[s], U0[i + a * n], sB[i + c * n]);
-      }
-    out[e] = x[0];
-    out[nn + e] = x[1];
-    out[2 * nn + e] = y[0];
-    out[3 * nn + e] = y[1];
-  }
-  __syncthreads();
-  // M0 = (R~ Z1) R~^T
-  for (int e = tid; e < nn; e += 256) {
-    const int i = e % n, j = e / n;
+  // rows c0 .. of R~ Z1
+  for (int e = tid; e < n * SC; e += 256) {
+    const int il0 = e & (SC - 1), j = e >> 4, i = c0 + il0;
+    if (il0 >= cw) continue;
     const int sp = i >= h, il = i - sp * h;
     const int off = m_off[il], sz = m_sz[il], base = m_base[il];
     double2 a = cz();
     for (int k = 0; k < sz; ++k) rfma(a, Z1[(sp * h + off + k) + j * n], sR[base + (il - off) + k * sz]);
-    sA[e] = a;
+    sZ[il0 * (n + 1) + j] = a;
   }
   __syncthreads();
-  for (int e = tid; e < nn; e += 256) {
-    const int j = e % n, i = e / n;  // row-major output: consecutive threads, consecutive j
+  // M0 = (R~ Z1) R~^T, row-major output: consecutive threads, consecutive j
+  for (int e = tid; e < n * cw; e += 256) {
+    const int il0 = e / n, j = e - il0 * n;
     const int sp = j >= h, jl = j - sp * h;
     const int off = m_off[jl], sz = m_sz[jl], base = m_base[jl];
     double2 a = cz();
-    for (int k = 0; k < sz; ++k) cfma(a, sA[i + (sp * h + off + k) * n], sR[base + (jl - off) + k * sz]);
-    out[6 * nn + (size_t)i * n + j] = a;
+    for (int k = 0; k < sz; ++k) cfma(a, sZ[il0 * (n + 1) + sp * h + off + k], sR[base + (jl - off) + k * sz]);
+    out[6 * nn + (size_t)(c0 + il0) * n + j] = a;
+  }
+  // X_s(a, c) = sum_{i in s} V0(i, a) (R~V1)(i, c), Y_s likewise with U0, R~*U1:
+  // lane l: A row a = l % 16, B column c = l % 16, both i = l / 16 of the step
+  const int lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+  for (int m = tid >> 6; m < (n + 15) / 16; m += 4) {
+    const int ar = min(16 * m + l16, n - 1);
+    for (int s = 0; s < 2; ++s) {
+      d4 xr = {0.0, 0.0, 0.0, 0.0}, xi = xr, yr = xr, yi = xr;
+      for (int k0 = 0; k0 < h; k0 += 4) {
+        const int k = k0 + lk, i = s * h + min(k, h - 1);
+        const double z = (k < h) ? 1.0 : 0.0;
+        const double av = z * V0[i + ar * n], au = z * U0[i + ar * n];
+        const double2 bv = sA[i * SLD + min(l16, cw - 1)], bu = sB[i * SLD + min(l16, cw - 1)];
+        xr = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv.x, xr, 0, 0, 0);
+        xi = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv.y, xi, 0, 0, 0);
+        yr = __builtin_amdgcn_mfma_f64_16x16x4f64(au, bu.x, yr, 0, 0, 0);
+        yi = __builtin_amdgcn_mfma_f64_16x16x4f64(au, bu.y, yi, 0, 0, 0);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {  // D: row 4 v + l / 16, column l % 16
+        const int r = 16 * m + 4 * v + lk;
+        if (r < n && l16 < cw) {
+          out[s * nn + r + (c0 + l16) * n] = make_double2(xr[v], xi[v]);
+          out[(2 + s) * nn + r + (c0 + l16) * n] = make_double2(yr[v], yi[v]);
+        }
+      }
+    }
   }
 }
 
@@ -173,13 +199,19 @@ struct PGauge {
 
 template <int N>
 __host__ __device__ constexpr size_t gauge_misc_bytes() {
-  // pivots [2] (16 B), reductions [NW][20] (8 B), pivot columns [2] and the
-  // solution order [N] (4 B): 840 B at N = 40, so three workgroups of n = 40
-  // (52.7 KB) share a CU's 160 KB
-  return 32 + 160 * PlainCfg<N>::NW + 8 + 4 * N;
+  // pivots [2] (16 B), reductions [NW][20], ladder table [N] (8 B), pivot
+  // columns [2] and the solution order [N] (4 B): 1,160 B at N = 40, so three
+  // workgroups of n = 40 (53,640 B) share a CU's 160 KB
+  return 32 + 160 * PlainCfg<N>::NW + 8 * N + 8 + 4 * N;
 }
 
-typedef double d4 __attribute__((ext_vector_type(4)));
+template <int CTRL>
+__device__ __forceinline__ double dpp_quad_f64(double v) {  // DPP move of a double
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
 
 // Pfaffian per gauge point: S = cscale [[D M0 D, -1], [1, -Z0]] (Pfaf_Over, 2n x
 // 2n skew) by Parlett-Reid elimination, the pivot of row r = 2k the largest
@@ -202,10 +234,11 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 // other half of their buffers while slow waves still update.  Entries that
 // left the trailing matrix are updated on with values nobody reads.
 // Bound by VALU issue (G = 8) and the wait of each step for its pivot chain (G =
-// 16, hidden by the other workgroups of the CU).  Against full pivoting with
-// the triangle spread entry by entry over 3n / 32 waves, per gauge point on the
-// whole card: n = 24 41 -> 15 ns, n = 40 168 -> 77 ns, n = 44 570 -> 97 ns, n =
-// 64 1,230 -> 300 ns.
+// 16, hidden by the other workgroups of the CU: n = 40 at three waves per SIMD
+// 77 ns, at four, spilling 20 bytes, 64 ns).  Against full pivoting with the
+// triangle spread entry by entry over 3n / 32 waves, per gauge point on the whole
+// card: n = 24 41 -> 15 ns, n = 40 168 -> 64 ns, n = 44 570 -> 97 ns, n = 64 1,230 ->
+// 300 ns.
 template <int N>
 struct PfCfg {
   static constexpr int G = (2 * N <= 48) ? 8 : 16;
@@ -213,7 +246,7 @@ struct PfCfg {
   static constexpr int T = (2 * N + G - 1) / G, NS = T * (T + 1) / 2;
   // slots, held R and C, addresses: the waves per SIMD that fit
   static constexpr int REGS = 4 * NS + 8 * T + 36;
-  static constexpr int WV = REGS <= 102 ? 5 : (REGS <= 128 ? 4 : (REGS <= 168 ? 3 : 2));
+  static constexpr int WV = REGS <= 102 ? 5 : (REGS <= 136 ? 4 : (REGS <= 168 ? 3 : 2));
 };
 
 template <int N>
@@ -407,8 +440,10 @@ __global__ __launch_bounds__(PfCfg<N>::NT) __attribute__((amdgpu_waves_per_eu(Pf
 // v_mfma_f64_16x16x4 (its rate equals the vector units', but an operand is read
 // once per 16 results: the vector form read V0 once per result pair and thread).
 // Per gauge point on the whole card, with the list (a row per two lanes, vector
-// densities -> this): n = 24 70 -> 39 ns, n = 40 292 -> 182 ns, n = 44 688 -> 225
-// ns, n = 64 1,960 -> 830 ns.
+// densities -> this): n = 24 70 -> 34 ns, n = 40 292 -> 163 ns, n = 44 688 -> 211
+// ns, n = 64 1,960 -> 785 ns; of n = 40's, loads 15 %, Gauss-Jordan 38 % (VALU
+// issue, half of it multiply-adds, and the barriers), densities 12 %, the list
+// and the sums 27 % (LDS gathers).
 template <int N, bool E2>
 __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_eu(PlainCfg<N>::GAUGE_WAVES))) void k_plain_gauge(PGauge p) {
   using C = PlainCfg<N>;
@@ -416,11 +451,12 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
   extern __shared__ double2 lds[];
   const int n = p.n, h = p.h, nn = n * n, ld = n + 1;
   double2 *const R = lds;              // rho, column-major with leading dimension n + 1
-  double2 *const AB = lds + n * ld;    // A01 (i < j at i + j n), A10 / 4 (i < j at j + i n)
-  char *const misc = (char *)(AB + nn);
+  double2 *const AB = lds + n * ld;    // A01 (i < j at i + j (n + 1)), A10 / 4 (i < j at j + i (n + 1))
+  char *const misc = (char *)(AB + n * ld);
   double2 *const sS = (double2 *)misc;             // pivots [2]
   double *const red = (double *)(misc + 32);
-  int *const sC = (int *)(red + 20 * NW);          // pivot columns [2]
+  double *const mt = red + 20 * NW;                // [2][N / 2]: m, <m+1|J+|m> per species-local state
+  int *const sC = (int *)(mt + N);                 // pivot columns [2]
   int *const kinv = sC + 2;                        // [N]: solution index of each column
   // Gauss-Jordan vectors, then W, at the front (rho and the A-block come later)
   double2 *const vR = lds, *const vC = lds + 2 * GC * TC, *const W = lds;
@@ -438,35 +474,45 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
   const double2 ep = cexpi((2.0 * M_PI / p.nphi) * gl.x), en = cexpi((2.0 * M_PI / p.nphi) * gl.y);
   const double2 *const H = p.hoist + (size_t)ul * 7 * nn;
 
+  for (int i = tid; i < 2 * h; i += NTH) mt[i] = p.mtab[i];
   // ---------------------------------------------------------------- Gauss-Jordan
   const int a = tid / GC, b = tid % GC;
   double2 sv[TR][TC];
   {
-    const double2 *Xp = H, *Xn = H + nn, *Yp = H + 2 * nn, *Yn = H + 3 * nn, *RV1 = H + 4 * nn, *RcU1 = H + 5 * nn;
+    const double2 *Xp = H, *Xn = H + nn, *Yp = H + 2 * nn, *Yn = H + 3 * nn, *RV1 = H + 4 * nn;  // (R~* U1 after R~ V1)
+    // unconditional loads (indices clamped, the value chosen by selects), so a
+    // slot row's loads are in flight together; slot rows below n / GR hold rows
+    // of T only, those from (n - 1) / GR + 1 on none
 #pragma unroll
     for (int pp = 0; pp < TR; ++pp) {
       const int r = a + GR * pp;
-      const int kind = (r < n) ? 0 : (r < 2 * n) ? 1 : (r < 3 * n) ? 2 : 3;
-      const int ri = (kind < 3) ? r - kind * n : 0;
+      const int kind = (r < n) ? 0 : (r < 2 * n) ? 1 : 2;
+      const int ri = min(r - kind * n, n - 1);
+      const bool ok = r < 3 * n;
       const double2 es = (ri >= h) ? en : ep;
       const double2 ph = (kind == 1) ? es : cconj(es);
 #pragma unroll
       for (int q = 0; q < TC; ++q) {
         const int c = b + GC * q;
-        double2 v = cz();
-        if (c < n && kind < 3) {
-          const size_t o = (size_t)ri + (size_t)c * n;
-          if (kind == 0) {
-            v = cmul(ep, Xp[o]);
-            cfma(v, en, Xn[o]);
-            cfma(v, cconj(ep), Yp[o]);
-            cfma(v, cconj(en), Yn[o]);
-          } else {
-            v = cmul(ph, (kind == 1 ? RV1 : RcU1)[o]);
-          }
+        const unsigned o = (unsigned)(ri + min(c, n - 1) * n) * 16u;  // (a 32-bit offset to uniform bases)
+        auto at = [&](const double2 *m) { return *(const double2 *)((const char *)m + o); };
+        auto atw = [&](unsigned x) { return *(const double2 *)((const char *)RV1 + (o + x)); };
+        double2 t = cz(), w = cz();
+        if (GR * pp < n) {  // (uniform)
+          t = cmul(ep, at(Xp));
+          cfma(t, en, at(Xn));
+          cfma(t, cconj(ep), at(Yp));
+          cfma(t, cconj(en), at(Yn));
         }
-        sv[pp][q] = v;
+        if (GR * pp + GR > n) w = cmul(ph, atw(kind == 2 ? 16u * (unsigned)nn : 0u));
+        const bool in = ok && c < n;
+        sv[pp][q].x = in ? (kind == 0 ? t.x : w.x) : 0.0;
+        sv[pp][q].y = in ? (kind == 0 ? t.y : w.y) : 0.0;
       }
+      // a row's values are made before the next row's loads are issued (the
+      // scheduler would otherwise issue all loads first and spill)
+#pragma unroll
+      for (int q = 0; q < TC; ++q) __asm__ volatile("" : "+v"(sv[pp][q].x), "+v"(sv[pp][q].y) : : "memory");
     }
   }
   int info = 0;
@@ -545,14 +591,15 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
     }
   }
   __syncthreads();
-  // W(row, k) in solution order, rows of W1 then W2, column-major
+  // W(row, k) in solution order, rows of W1 then W2, column-major with an odd
+  // leading dimension (a row of threads writes 16 columns at once)
 #pragma unroll
   for (int pp = 0; pp < TR; ++pp) {
     const int r = a + GR * pp - n;
 #pragma unroll
     for (int q = 0; q < TC; ++q) {
       const int c = b + GC * q;
-      if (r >= 0 && r < 2 * n && c < n) W[r + kinv[c] * 2 * n] = sv[pp][q];
+      if (r >= 0 && r < 2 * n && c < n) W[r + kinv[c] * (2 * n + 1)] = sv[pp][q];
     }
   }
   __syncthreads();
@@ -577,14 +624,14 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int w = 0; w < JW; ++w) {
         const double bv = bp[w][(size_t)k * n];
-        const double2 av = W[ar[w] + k * 2 * n];
+        const double2 av = W[ar[w] + k * (2 * n + 1)];
         tre[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, bv, tre[w], 0, 0, 0);
         tim[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, bv, tim[w], 0, 0, 0);
       }
     }
   }
   __syncthreads();  // W is read no more
-  for (int e = tid; e < nn; e += NTH) AB[e] = cz();
+  for (int e = tid; e < n * ld; e += NTH) AB[e] = cz();
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < JW; ++w) {
@@ -602,13 +649,13 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
         } else if (r < 2 * n && r - n != j) {  // kappa01 = -x -> A01
           const int i = r - n;
           const double sg = (i < j) ? -1.0 : 1.0;
-          double *dst = (double *)&AB[min(i, j) + max(i, j) * n];
+          double *dst = (double *)&AB[min(i, j) + max(i, j) * ld];
           atomicAdd(dst, sg * x.x);
           atomicAdd(dst + 1, sg * x.y);
         }
       } else if (r < n && r != j) {  // kappa10 -> A10 / 4
         const double sg = (r < j) ? 0.25 : -0.25;
-        double *dst = (double *)&AB[max(r, j) + min(r, j) * n];
+        double *dst = (double *)&AB[max(r, j) + min(r, j) * ld];
         atomicAdd(dst, sg * x.x);
         atomicAdd(dst + 1, sg * x.y);
       }
@@ -623,17 +670,22 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
   // (c_a = <m_a+1|J+|m_a>, 0 for the first state of an orbit, m = j .. -j);
   // traces t_z = sum m_a rho_aa, t_+ = sum c_a rho(a, a-1), t_- = sum c_{a+1} rho(a, a+1)
   double2 ek = cz(), aj = cz(), tz = cz(), tpl = cz(), tmi = cz(), zp = cz(), zn = cz();
-  auto a01 = [&](int x, int y) -> double2 {
-    return x < y ? AB[x + y * n] : (x > y ? cneg(AB[y + x * n]) : cz());
+  auto a01 = [&](int x, int y) -> double2 {  // branch-free: the stored triangle with the sign, 0 on the diagonal
+    const double2 v = AB[min(x, y) + max(x, y) * ld];
+    const double sg = (x < y) ? 1.0 : (x > y ? -1.0 : 0.0);
+    return cscale(sg, v);
   };
-  for (int e = tid; e < nn; e += NTH) {
-    const int a = e % n, b = e / n;
+  // b fastest (t1(b, a) contiguous, rho at an odd leading dimension)
+  for (int e = tid, x = tid / n, y = tid - x * n; e < nn; e += NTH) {
+    const int a = x, b = y;
     const double2 rab = R[a + b * ld], rba = R[b + a * ld];
     const int al = a >= h ? a - h : a, bl = b >= h ? b - h : b;
-    const double ma = p.mtab[al], mb = p.mtab[bl], ca = p.mtab[h + al], cb = p.mtab[h + bl];
+    const double ma = mt[al], mb = mt[bl], ca = mt[h + al], cb = mt[h + bl];  // c = 0 at the first state of an orbit
+    const double ca1 = (a + 1 < n) ? mt[h + (a + 1 >= h ? a + 1 - h : a + 1)] : 0.0;
+    const double cb1 = (b + 1 < n) ? mt[h + (b + 1 >= h ? b + 1 - h : b + 1)] : 0.0;
     rfma(ek, p.t1b[b + (size_t)a * n], rab);
     double2 q = cscale(ma * mb, rba);
-    if (ca != 0.0 && cb != 0.0) rfma(q, ca * cb, R[(b - 1) + (a - 1) * ld]);
+    rfma(q, ca * cb, R[max(b - 1, 0) + max(a - 1, 0) * ld]);
     cfms(aj, rab, q);
     if (a == b) {
       rfma(aj, p.mtab[2 * h + al], rab);
@@ -643,18 +695,19 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
     }
     if (a == b + 1) rfma(tpl, ca, rab);
     if (b == a + 1) rfma(tmi, cb, rab);
-    if (a != b) {
-      const double2 l4 = (a < b) ? AB[b + a * n] : cneg(AB[a + b * n]);
-      double2 s = cscale(ma * mb, a01(a, b));
-      if (ca != 0.0 && b + 1 < n) {
-        const double cb1 = p.mtab[h + (b + 1 >= h ? b + 1 - h : b + 1)];
-        if (cb1 != 0.0) rfma(s, 0.5 * ca * cb1, a01(a - 1, b + 1));
-      }
-      if (cb != 0.0 && a + 1 < n) {
-        const double ca1 = p.mtab[h + (a + 1 >= h ? a + 1 - h : a + 1)];
-        if (ca1 != 0.0) rfma(s, 0.5 * ca1 * cb, a01(a + 1, b - 1));
-      }
-      cfma(aj, l4, s);
+    {
+      double2 l4 = AB[max(a, b) + min(a, b) * ld];  // (A10 / 4)(a, b) up to the sign; a = b: never used
+      l4 = cscale((a < b) ? 1.0 : (a > b ? -1.0 : 0.0), l4);
+      double2 w = cscale(ma * mb, a01(a, b));
+      rfma(w, 0.5 * ca * cb1, a01(max(a - 1, 0), min(b + 1, n - 1)));
+      rfma(w, 0.5 * ca1 * cb, a01(min(a + 1, n - 1), max(b - 1, 0)));
+      cfma(aj, l4, w);
+    }
+    x += NTH / n;
+    y += NTH % n;
+    if (y >= n) {
+      y -= n;
+      ++x;
     }
   }
   // two-body energy, regrouped list
@@ -672,20 +725,36 @@ __global__ __launch_bounds__(PlainCfg<N>::NTH) __attribute__((amdgpu_waves_per_e
       rfma(e2, me, t);
     }
   }
+  // the 16 sums: quad sums by DPP, those of each value through LDS (the A-block
+  // is free after the list), thread k < 16 adds value k's
   double v[16] = {e2.x, e2.y, ek.x, ek.y, aj.x, aj.y, tz.x, tz.y, tpl.x, tpl.y, tmi.x, tmi.y, zp.x, zp.y, zn.x, zn.y};
 #pragma unroll
-  for (int k = 0; k < 16; ++k)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off);
-  if (lane == 0)
+  for (int k = 0; k < 16; ++k) {
+    v[k] += dpp_quad_f64<0xB1>(v[k]);  // quad_perm [1,0,3,2]
+    v[k] += dpp_quad_f64<0x4E>(v[k]);  // quad_perm [2,3,0,1]
+  }
+  __syncthreads();
+  double *const qs = (double *)AB;
+  int NQ = NTH / 4 < 64 ? NTH / 4 : 64;  // quads through LDS at a time: 17 doubles each in the A-block's 16 n (n + 1) bytes
+  while (NQ * 17 * 8 > 16 * n * ld) NQ >>= 1;
+  double tot = 0.0;
+#pragma unroll 1
+  for (int q0 = 0; q0 < NTH / 4; q0 += NQ) {
+    const int qd = (tid >> 2) - q0;
+    if ((tid & 3) == 0 && qd >= 0 && qd < NQ) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) red[wave * 20 + k] = v[k];
+      for (int k = 0; k < 16; ++k) qs[qd * 17 + k] = v[k];
+    }
+    __syncthreads();
+    if (tid < 16)
+      for (int i = 0; i < NQ; ++i) tot += qs[i * 17 + tid];
+    __syncthreads();
+  }
+  if (tid < 16) red[tid] = tot;
   __syncthreads();
   double2 *const go = p.gout + (size_t)L * p.nog;
   if (tid == 0) {
-    double t[16];
-    for (int k = 0; k < 16; ++k) t[k] = 0.0;
-    for (int w = 0; w < NW; ++w)
-      for (int k = 0; k < 16; ++k) t[k] += red[w * 20 + k];
+    const double *t = red;
     const double2 E2v = make_double2(t[0], t[1]), EK = make_double2(t[2], t[3]), A = make_double2(t[4], t[5]);
     const double2 TZ = make_double2(t[6], t[7]), TP = make_double2(t[8], t[9]), TM = make_double2(t[10], t[11]);
     const double2 ZP = make_double2(t[12], t[13]), ZN = make_double2(t[14], t[15]);
@@ -806,9 +875,9 @@ __global__ __launch_bounds__(64) void k_plain_sum(PSum p) {
 
 // ------------------------------------------------------------------ host
 // Size classes of the kernels (n <= N): sd 24, pf 40, f5pg9 44 -> 48,
-// sdpf 64.  The gauge kernel's LDS is 16 (2 n^2 + n) bytes plus ~1 KB:
-// 52.7 KB at n = 40 (three workgroups per CU), 62.6 KB at n = 44 (two),
-// 133 KB at n = 64 (one).
+// sdpf 64.  The gauge kernel's LDS is 32 n (n + 1) bytes plus ~1 KB:
+// 53.6 KB at n = 40 (three workgroups per CU), 64.6 KB at n = 44 (two),
+// 136 KB at n = 64 (one).
 constexpr int NCLASS = 6;
 constexpr int CLASSES[NCLASS] = {16, 24, 32, 40, 48, 64};
 
@@ -820,7 +889,7 @@ int class_of(int n) {
 
 template <int N>
 size_t gauge_lds(int n) {
-  return sizeof(double2) * ((size_t)n * (n + 1) + (size_t)n * n) + gauge_misc_bytes<N>();
+  return sizeof(double2) * 2 * (size_t)n * (n + 1) + gauge_misc_bytes<N>();
 }
 
 template <int N, bool E2>
@@ -853,7 +922,7 @@ size_t plain_unit_bytes(const PlainArgs &a) {
 
 hipError_t plain_prepare(int n, bool e2) {
   const hipError_t e = hipFuncSetAttribute((const void *)k_plain_setup, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)(sizeof(double2) * 2 * (size_t)n * n));
+                                           (int)setup_lds(n));
   if (e != hipSuccess) return e;
   switch (class_of(n)) {
     case 16: return e2 ? prepare_nc<16, true>(n) : prepare_nc<16, false>(n);
@@ -885,7 +954,7 @@ hipError_t plain_run(const PlainArgs &a, int u0, int nu, void *work, hipStream_t
   sp.alp = a.alp; sp.gam = a.gam; sp.rtab = a.rtab; sp.pk_a = a.pk_a; sp.pk_b = a.pk_b;
   sp.blk_off = a.blk_off; sp.blk_sz = a.blk_sz; sp.blk_base = a.blk_base; sp.twom = a.twom;
   sp.q0 = a.q0; sp.q1 = a.q1; sp.U = a.U; sp.V = a.V; sp.Z = a.Z; sp.hoist = hoist;
-  hipLaunchKernelGGL(k_plain_setup, dim3(nu), dim3(256), sizeof(double2) * 2 * nn, s, sp);
+  hipLaunchKernelGGL(k_plain_setup, dim3(nu, (a.n + SC - 1) / SC), dim3(256), setup_lds(a.n), s, sp);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
 

@@ -2925,14 +2925,14 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
   // and, when a + b != c + d, its (cd)(ab) partner; an entry with a = b or
   // c = d adds exactly zero to the eight-term sum of HFB_Energy_COMPLEX and is
   // dropped.  Operands by LDS offset (rho at leading dimension n + 1, then
-  // the A-block: A01(a,b) at a + b n, A10(c,d) / 4 at d + c n): bytes when
+  // the A-block: A01(a,b) at a + b (n + 1), A10(c,d) / 4 at d + c (n + 1)): bytes when
   // they fit 16 bits, else elements.
   {
     const unsigned ldr = n + 1, abase = n * ldr;
-    c->pl_bytes = (16u * (abase + (unsigned)n * n) <= 65535u) ? 1 : 0;
+    c->pl_bytes = (16u * (abase + (unsigned)n * ldr) <= 65535u) ? 1 : 0;
     const unsigned sc = c->pl_bytes ? 16u : 1u;
     auto rb = [&](int row, int col) { return sc * ((unsigned)row + (unsigned)col * ldr); };
-    auto ab = [&](int row, int col) { return sc * (abase + (unsigned)row + (unsigned)col * n); };
+    auto ab = [&](int row, int col) { return sc * (abase + (unsigned)row + (unsigned)col * ldr); };
     std::vector<uint4> lo;
     std::vector<double> lm;
     auto term = [&](int i, int j, int k, int l, double me) {
