@@ -31,6 +31,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pnamp_gpu.h"
@@ -223,11 +224,12 @@ struct VEntry {
 // Four launches per chunk of pairs:
 //   k_fac_setup    one workgroup per (pair, Euler point, species): the
 //                  gauge-independent X, Y, R V1s, R* U1s, M0 = R Z1s R^T -> HBM;
-//   k_fac_phi<h>   one wavefront per (pair, Euler point, species, phi), twice
-//                  over the same grid: the Pfaffian (the skew matrix in a 2D
-//                  block-cyclic register layout), then Gauss-Jordan (one
-//                  column per lane) and the densities, rho / kappa in LDS for
-//                  the list; no workgroup barriers;
+//   k_fac_phi<h>   one wavefront per (pair, Euler point, species, phi): the
+//                  Pfaffian (the skew matrix in a 2D block-cyclic register
+//                  layout);
+//   k_fac_dens<h>  one wavefront per (pair, Euler point, species, group of
+//                  angles): Gauss-Jordan (one column per lane), the densities
+//                  and the species lists on 4 x 4 matrix tiles;
 //   k_fac_combine  one workgroup per (pair, Euler point): the p-n bilinear form
 //                  and the nphi^2 gauge sum.
 constexpr int NTS = 256;     // threads of the setup workgroup
@@ -277,7 +279,7 @@ struct SetupParams {
   const double *rtab;               // [nbet][npack]
   const int *pk_a, *pk_b, *blk_off, *blk_sz, *blk_base, *twom;
   const int *q0, *q1;
-  double2 *sbuf;                    // [npairs][NE][2][5][h*h]: X, Y, R V1s, R* U1s, M0 (column-major)
+  double2 *sbuf;                    // [npairs][NE][2][5][h*h]: X, Y (column-major), R V1s, R* U1s (row-major), M0 (column-major)
 };
 
 __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
@@ -326,10 +328,13 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
     RV1[e] = a;
     RcU1[e] = b;
     RZ1[e] = c;
-    out[2 * hh + e] = a;
-    out[3 * hh + e] = b;
   }
   __syncthreads();
+  for (int e = tid; e < hh; e += NTS) {  // row-major (k_fac_dens reads rows as wave-uniform operands)
+    const int j = e % h, i = e / h;
+    out[2 * hh + e] = RV1[i + j * h];
+    out[3 * hh + e] = RcU1[i + j * h];
+  }
   // X = V0s^T RV1, Y = U0s^T RcU1, M0 = (R Z1s) R^T
   for (int e = tid; e < hh; e += NTS) {
     const int i = e % h, j = e / h;
@@ -349,6 +354,19 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
   }
 }
 
+// Bilinear form sum_xy C(x, y) a_x b_y as tiles of v_mfma_f64_4x4x4_4b (D_b +=
+// A_b B_b for four b): groups of four row tiles (four rows x each, b = 0..3),
+// every tile with columns of its own, four per step.  A is the table's 4 x 4
+// entries of each tile, B the tiles' column elements of up to two complex
+// vectors (B column = 2 vector + re / im), gathered from LDS by offset.
+struct BilForm {
+  const double *v;   // [2 pairs][64]: A of lane 16 k + 4 b + i = C(row i of tile b, column k of the step)
+  const uint4 *ofs;  // [pairs][16], LDS byte offsets, entry 4 k + b: column k of tile b in both steps of the
+                     // pair, row k of tile b, and 1 in the last pair of a group
+  int np;            // pairs of steps, a multiple of BIL_RING (BIL_RING more, all zero, follow)
+};
+constexpr int BIL_RING = 8;
+
 struct PhiParams {
   int n, nphi, nd, NE, nwg;         // nphi gauge angles, nd of them evaluated
   double cscale;
@@ -359,14 +377,11 @@ struct PhiParams {
   const int *pfs_ok;                // both Pfaffian kernels launched: [nstates] route of bra state q0, else NULL
   const double *t1b;                // n x n
   const double *mtab;               // [3][h]: m, <m+1|J_+|m> (0 at m = j), j(j+1) per species-local state
-  const double2 *jtab;              // [2][h^2][4]: coefficients of rho(a,b) in Ekin and the <J^2> pieces (see pnamp_create)
-  // species lists (p, n), one term per entry, nl entries padded with zero
-  // terms to a multiple of 256: entry q is lofs[q] = LDS byte offsets of
-  // rho(k,i), rho(l,j), rho(l,i), rho(k,j) and lofs[nl + q] = those of
-  // A01(i,j), A10(k,l)/4 and the matrix element (low, high word); full
-  // 32-bit offsets, so the loop unpacks nothing
-  const uint4 *lofs[2];
-  int nl[2];
+  int ngrp, geff;                   // k_fac_dens: groups of geff gauge angles, one wave each
+  // species lists (p, n): rho (sum over x <= y of C(x, y) rho_x rho_y, offsets
+  // in a rho block, leading dimension h + 1) and kappa (sum of V A01_x A10_y /
+  // 4, offsets in an A-block, leading dimension h)
+  BilForm frho[2], fkap[2];
   const int *q0, *q1;
   double2 *out;                     // [npairs][NE][2][nphi][FAC_OUT]
   double2 *rho;                     // [npairs][NE][2][nphi][h*h], column-major
@@ -439,50 +454,7 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-// Gauss-Jordan on an H-row system held one column per lane of the wavefront:
-// col[r] is row r of this lane's column, lanes 0..H-1 hold the coefficient
-// matrix M, the other lanes right-hand sides.  Step k pivots on row k and the
-// unused coefficient column q with the largest |M(k, q)| (|re| + |im| to
-// 2^-15 relative, ties to the smallest q): for M = T^T this is the row
-// pivoting of T by ZGETRF's IZAMAX.  The row index is static, so nothing is picked out of registers by
-// a run-time index; column q reaches every lane by v_readlane from lane q (a
-// wave-uniform operand of the update; through LDS the 64-lane broadcast reads
-// made the step LDS-bound).  On return the unknown q_k = qmap[k] is row k of
-// each right-hand-side column; INFO as LAPACK for an exactly-zero pivot.  The
-// workgroup is this one wavefront, so __syncthreads() only orders LDS.
-template <int H>
-__device__ int wave_gauss_jordan(double2 (&col)[H], int *qmap) {
-  const int lane = threadIdx.x;
-  unsigned used = 0u;
-  int info = 0;
-#pragma unroll
-  for (int k = 0; k < H; ++k) {
-    unsigned key = 0u;
-    if (lane < H && !((used >> lane) & 1u)) key = pivot_key_hi<5>(cabs1(col[k]), lane);
-    key = wave_umax(key);
-    const int q = 31 - (int)(key & 31u);
-    used |= 1u << q;
-    if (lane == 0) qmap[k] = q;
-    auto rl = [&](double x) {
-      const long long bb = __double_as_longlong(x);
-      return __longlong_as_double(((long long)__builtin_amdgcn_readlane((int)(bb >> 32), q) << 32) |
-                                  (long long)(unsigned)__builtin_amdgcn_readlane((int)bb, q));
-    };
-    const double2 pv = make_double2(rl(col[k].x), rl(col[k].y));
-    // tested here (uniform) rather than at the INFO store: a test sunk to
-    // the use keeps every pivot alive in registers
-    if (__builtin_amdgcn_readfirstlane((pv.x == 0.0 && pv.y == 0.0) ? 1 : 0) && info == 0) info = k + 1;
-    const double2 prow = cmul(col[k], crecip_nr(pv));
-#pragma unroll
-    for (int r = 0; r < H; ++r)
-      if (r != k) cfms(col[r], make_double2(rl(col[r].x), rl(col[r].y)), prow);
-    col[k] = prow;
-  }
-  __syncthreads();
-  return info;
-}
-
-// One wavefront per (pair, Euler point, species, gauge angle phi).
+// The Pfaffian part: one wavefront per (pair, Euler point, species, gauge angle phi).
 //
 // Pfaffian of S(phi) (2H x 2H skew) by Parlett-Reid elimination with partial
 // pivoting: at step k the pivot of row r = 2k is the largest |S(r, c)|, c > r,
@@ -494,34 +466,7 @@ __device__ int wave_gauss_jordan(double2 (&col)[H], int *qmap) {
 // block-cyclic layout (lane 8a + b holds S(a + 8p, b + 8q), slot rows p <=
 // slot columns q); rows r, r + 1 and row / column c of the step go through
 // LDS, and the update covers the slot rows that still hold trailing entries.
-//
-// T = e^{i phi} X + e^{-i phi} Y, W1 = e^{i phi} R V1s T^-1 and
-// W2 = e^{-i phi} R* U1s T^-1 solve T^T [W1 W2]^T = [e^{i phi} RV1, e^{-i phi} RcU1]^T
-// (Gauss-Jordan on lanes: T^T in lanes 0..H-1, right-hand sides in lanes
-// H..3H-1, or in two passes when 3H > 64), then rho = W1 V0s^T,
-// kappa10 = W1 U0s^T, kappa01 = -W2 V0s^T (ROKAPPAphiomega,
-// Codes/PNAMP/PNAMP_Proj.f90:459-551) with V0s, U0s read as wave-uniform
-// operands.
-//
-// <J^2> pieces (ZJ2_0, Codes/PNAMP/PNAMP_ME2B.f90:1-152) from the ladder form
-// sum_k J_k (x) J_k = J_z (x) J_z + (J_+ (x) J_- + J_- (x) J_+) / 2 with J_z
-// diagonal and J_+ one off-diagonal inside each orbit:
-//   A = sum_a j_a(j_a+1) rho_aa - sum_k Tr(J_k rho J_k rho) + sum_k Tr(J_k kappa10 J_k^T kappa01^T),
-//   t_+ = Tr(J_+ rho), t_- = Tr(J_- rho), t_z = Tr(J_z rho),
-// so <J^2> = A_p + A_n + (t_zp + t_zn)^2 + (t_+p + t_+n)(t_-p + t_-n).
-//
-// The eight-term list sum of HFB_Energy_COMPLEX
-// (Codes/PNAMP/PNAMP_Energy_OpenMP.f90:5-100) is regrouped exactly: with
-// A01 = kappa01 - kappa01^T and A10 = kappa10 - kappa10^T,
-//   (1/4) V [r_ijkl - r_jikl - r_ijlk + r_jilk + d (r_klij - r_klji - r_lkij + r_lkji)]
-//   = V [rho_ki rho_lj - rho_li rho_kj + A01_ij A10_kl / 4
-//        + d (rho_ik rho_jl - rho_jk rho_il + A01_kl A10_ij / 4)].
-//
-// The work is split in two launches over the same grid: PART_PF the Pfaffian
-// (a few KB of LDS and ~100 VGPRs, so many waves per SIMD hide its serial
-// steps), PART_REST the rest (13 KB of LDS for rho and one kappa / A block at
-// h = 20, so three waves per SIMD).
-constexpr int PART_PF = 1, PART_REST = 2;
+constexpr int PART_PF = 1;
 // PART_PFS: the Pfaffian by the Schur complement of the state block,
 //   Pf([[A, -1], [1, B]]) = Pf(B) Pf(A + B^-1),  A = e^{2i phi} M0, B = -Z_s,
 // an h x h Pfaffian per (pair, Euler point, species, phi) with B^-1 and
@@ -536,35 +481,17 @@ constexpr int pf_hold_vgprs(int h) {
   return 4 * (((2 * h + 7) / 8) * ((2 * h + 7) / 8 + 1) / 2) + 8 * ((2 * h + 7) / 8) + 8 + 20;
 }
 // Waves per SIMD the register budget is fitted to (the autotuner's knob;
-// these are the defaults): the Pfaffian part four where the held column
-// values fit 128 VGPRs (h <= 20), else three; the rest three while one
-// Gauss-Jordan pass fits the wavefront, else two.
+// these are the defaults): four where the held column values fit 128 VGPRs (h
+// <= 20), else three.
 constexpr int pf_default_waves(int h) { return pf_hold_vgprs(h) <= 128 ? 4 : 3; }
 template <int H, int PART>
 constexpr int fac_default_waves() {
-  return PART == PART_PF ? pf_default_waves(H) : PART == PART_PFS ? pf_default_waves(H / 2) : (3 * H <= 64 ? 3 : 2);
+  return PART == PART_PF ? pf_default_waves(H) : pf_default_waves(H / 2);
 }
 
-template <int H, int MIX, int PART, int WV = fac_default_waves<H, PART>()>
+template <int H, int PART, int WV = fac_default_waves<H, PART>()>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k_fac_phi(PhiParams p) {
-  constexpr int N2 = 2 * H, NU = N2 * (N2 - 1) / 2, SL = (NU + 63) / 64, HH = H * H;
-  constexpr int KP = (HH + 31) / 32 * 32;  // V-contraction K padded to the MFMA tile
-  constexpr int PASSES = (3 * H <= 64) ? 1 : 2;
-  constexpr int HP = H + 1, MS = H * HP;  // LDS leading dimension h + 1: transposed reads avoid bank conflicts
-  // B0 = sA[0, MS): rho (ld h + 1; transposed reads avoid bank conflicts);
-  // B1 = sA[MS, MS + h^2) (ld h): Gauss-Jordan unknown map (one pass),
-  // kappa01, kappa10, then the A-block A01 (strict upper) and A10 / 4
-  // (strict lower triangle); 13 KB at h = 20, twelve waves per CU.  The
-  // closing reduction reuses sA for 16 quad sums of 14 values (112 double2),
-  // more than MS + h^2 below h = 8: LDS stores past the allocation are
-  // dropped, so sA is never smaller than that.
-  constexpr int RED2 = 16 * 14 / 2;
-  __shared__ double2 sA[(MS + HH > RED2) ? MS + HH : RED2];
-  // in two passes kappa01 of pass 0 holds B1 through pass 1
-  constexpr bool GJ_IN_SA = (PASSES == 1);
-  __shared__ int qmap_sep[GJ_IN_SA ? 1 : H];
-  double2 *const B0 = sA, *const B1 = sA + MS;
-  int *qmap = GJ_IN_SA ? (int *)B1 : qmap_sep;
+  constexpr int N2 = 2 * H, HH = H * H;
   const int lane = threadIdx.x;
   // XCD-aware order: consecutive logical indices (the nphi waves of one setup
   // block) stay on one XCD and its L2; gridDim.x is a multiple of 8.
@@ -578,14 +505,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k
   const int iang = (int)(t % (unsigned)p.NE), ip = (int)(t / (unsigned)p.NE);
   const size_t g = ((size_t)ip * p.NE + iang) * 2 + sp;
   const size_t obase = g * nphi + f;
-  const double2 *X = p.sbuf + g * 5 * HH, *Y = X + HH, *RV1 = X + 2 * HH, *RcU1 = X + 3 * HH, *M0 = X + 4 * HH;
+  const double2 *M0 = p.sbuf + g * 5 * HH + 4 * HH;
   const int q0 = p.q0[ip];
-  const auto V0T = ro_const(p.VfT + ((size_t)q0 * 2 + sp) * HH), U0T = ro_const(p.UfT + ((size_t)q0 * 2 + sp) * HH);
   const double *Z0 = p.Z + (size_t)q0 * n * n + (size_t)sp * H * (n + 1);  // species block, ld n
-  const double phi = (2.0 * M_PI / p.nphi) * f;
-  const double2 e1 = cexpi(phi), e2 = cexpi(2.0 * phi);
+  const double2 e2 = cexpi((4.0 * M_PI / p.nphi) * f);
 
-  if constexpr (PART == PART_PF || PART == PART_PFS) {
   // ---- Pfaffian (PART_PF: of the 2h x 2h S; PART_PFS: of A + B^-1, h x h)
   // With both kernels launched over the grid, each keeps the pairs whose bra
   // state takes its route (one pair per wave: the test is wave-uniform)
@@ -764,213 +688,478 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k
 
   if constexpr (PART == PART_PFS) pf = cscale(p.pfb[(size_t)q0 * 2 + sp], pf);  // Pf(cscale B)
   if (lane == 0) p.out[obase * FAC_OUT] = pf;
-  } else {
-  // ---- Gauss-Jordan and the density products
-  // One pass: T^T in lanes 0..H-1, RV1 (-> W1) in H..2H-1, RcU1 (-> W2) in
-  // 2H..3H-1.  Two passes: pass 0 RcU1 (-> W2), pass 1 RV1 (-> W1), both in
-  // lanes H..2H-1.  W1 rows give rho (B0) and kappa10, W2 rows kappa01 (B1).
-  int info = 0;
-  constexpr int K01L = (PASSES == 1) ? 2 * H : H;  // first lane of the W2 rows
-  const bool w1lane = lane >= H && lane < 2 * H;
-  const int irow = (lane >= K01L && lane < K01L + H && PASSES == 1) ? lane - K01L : lane - H;
-  double2 *rho_out = p.rho + obase * HH;
-  const size_t mcol = ((size_t)ip * p.NE + iang) * nphi + f;  // GEMM column pair of this phi in species sp
-  constexpr int NE64 = (HH + 63) / 64;
-  double2 a01r[NE64];  // A01 = kappa01 - kappa01^T, strict upper triangle
-  double2 ajk = cz();  // kappa part of <J^2>
-  const auto mz = ro_const(p.mtab), cp = ro_const(p.mtab + H);
+}
+
+// acc[t] += this lane's part of a^T C b for vectors 2 t, 2 t + 1 of nv (blocks of
+// bstride bytes in LDS; vectors past nv repeat the last): columns of tile t are
+// (re, im) of the two, so the lanes of either half of bit 1 sum to a vector's
+// form.  A ring of BIL_RING pairs of steps holds the table loads in flight and
+// a ring of two the LDS operands; each slot is loaded again where it was used,
+// so no load is waited for by a register copy.
+template <int NC>
+__device__ __forceinline__ void bil_sum(const BilForm &t, const char *lds, int bstride, int nv, int lane, double2 *acc) {
+  constexpr int D = NC <= 2 ? BIL_RING : BIL_RING / 2;  // (registers)
+  auto mac = [](double a, double b, double d) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, d, 0, 0, 0); };
+  const char *bv[NC];  // (this lane's vector and component)
+  const int im = (lane & 1) * 8;
 #pragma unroll
-  for (int pass = 0; pass < PASSES; ++pass) {
-    const bool isW1 = w1lane && (PASSES == 1 || pass == 1);
-    const bool isW2 = (PASSES == 1) ? (lane >= K01L && lane < K01L + H) : (pass == 0 && w1lane);
-    double2 col[H];
-    if (lane < H) {
+  for (int c = 0; c < NC; ++c) bv[c] = lds + min(2 * c + ((lane >> 1) & 1), nv - 1) * bstride + im;
+  const double *vp = t.v + lane;
+  const uint4 *cp = t.ofs + (lane >> 2);
+  double v[D][2], b[2][NC][2], d[NC][2];
+  uint4 o[D];
 #pragma unroll
-      for (int r = 0; r < H; ++r)
-        col[r] = cadd(cmul(e1, X[lane + r * H]), cmul(cconj(e1), Y[lane + r * H]));
-    } else if (isW1 || isW2) {
-      const double2 *src = isW2 ? RcU1 : RV1;
-      const double2 ph = isW2 ? cconj(e1) : e1;
+  for (int u = 0; u < D; ++u) {
+    o[u] = cp[16 * u];
+    v[u][0] = vp[128 * u];
+    v[u][1] = vp[128 * u + 64];
+  }
 #pragma unroll
-      for (int r = 0; r < H; ++r) col[r] = cmul(ph, src[irow + r * H]);
-    } else {
+  for (int c = 0; c < NC; ++c) {
+    d[c][0] = d[c][1] = 0.0;
 #pragma unroll
-      for (int r = 0; r < H; ++r) col[r] = cz();
+    for (int u = 0; u < 2; ++u) {
+      b[u][c][0] = *(const double *)(bv[c] + o[u].x);
+      b[u][c][1] = *(const double *)(bv[c] + o[u].y);
     }
-    const int inf = wave_gauss_jordan<H>(col, qmap);
-    if (inf && !info) info = inf;
-    // solution rows in unknown order through B0, h rows at a time (unknown
-    // qmap[k] is row k), back into col: w[k] is W(irow, k) on the W lanes
+  }
+#pragma unroll 1
+  for (int q = 0; q < t.np; q += D) {
+    vp += 128 * D;
+    cp += 16 * D;
 #pragma unroll
-    for (int g = 0; g < ((PASSES == 1) ? 2 : 1); ++g) {
-      const bool gl = lane >= H * (g + 1) && lane < H * (g + 2);
-      if (gl) {
+    for (int u = 0; u < D; ++u) {
 #pragma unroll
-        for (int r = 0; r < H; ++r) B0[(lane - H * (g + 1)) * HP + qmap[r]] = col[r];
+      for (int c = 0; c < NC; ++c) {
+        d[c][0] = mac(v[u][0], b[u & 1][c][0], d[c][0]);
+        d[c][1] = mac(v[u][1], b[u & 1][c][1], d[c][1]);
       }
-      __syncthreads();
-      if (gl) {
+      // the group's rows: D row lk of tile lb, column li (no global loads in the
+      // branch: the wait counts of the ring stay exact)
+      if (__builtin_amdgcn_readfirstlane((int)o[u].w)) {
 #pragma unroll
-        for (int k = 0; k < H; ++k) col[k] = B0[(lane - H * (g + 1)) * HP + k];
-      }
-      __syncthreads();
-    }
-    const double2 (&w)[H] = col;
-    // V0s sweep: rho (W1 rows) -> B0 and HBM, kappa01 (W2 rows) -> B1
-#pragma unroll 2
-    for (int j = 0; j < H; ++j) {
-      double2 acc = cz();
-#pragma unroll
-      for (int k = 0; k < H; ++k) rfma(acc, V0T[j * H + k], w[k]);
-      if (isW1) {
-        B0[irow + j * HP] = acc;
-        rho_out[irow + j * H] = acc;
-        if (MIX != MIX_FP64) {
-          put_b<MIX, KP>(p.brho[sp], p.brho_lo[sp], irow + j * H, 2 * mcol, acc.x);
-          put_b<MIX, KP>(p.brho[sp], p.brho_lo[sp], irow + j * H, 2 * mcol + 1, acc.y);
+        for (int c = 0; c < NC; ++c) {
+          const double2 a = *(const double2 *)(bv[c] - im + o[u].z);
+          const double x = d[c][0] + d[c][1];
+          acc[c].x = fma(im ? -a.y : a.x, x, acc[c].x);
+          acc[c].y = fma(im ? a.x : a.y, x, acc[c].y);
+          d[c][0] = d[c][1] = 0.0;
         }
       }
-      if (isW2) B1[irow + j * H] = cneg(acc);
+      const uint4 on = o[(u + 2) % D];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        b[u & 1][c][0] = *(const double *)(bv[c] + on.x);
+        b[u & 1][c][1] = *(const double *)(bv[c] + on.y);
+      }
+      o[u] = cp[16 * u];
+      v[u][0] = vp[128 * u];
+      v[u][1] = vp[128 * u + 64];
+    }
+  }
+}
+
+// Densities, energies and <J^2> pieces, one wavefront per (pair, Euler point,
+// species, group of up to G = 64 / H gauge angles): lane (g, c) = (lane / H, lane
+// % H) works on column c or row c of angle g, so nearly all lanes are in use.
+//
+// S = T^-T of every angle by in-place Gauss-Jordan (T = e^{i phi} X + e^{-i phi}
+// Y; lane (g, c) holds column c of T^T in registers).  Step k pivots on row k
+// and the unused column q with the largest |re| + |im| (to 2^-15 relative, ties
+// to the smallest q: the row pivoting of T by ZGETRF's IZAMAX).  The row index
+// is static, so nothing is picked out of registers by a run-time index; column q
+// of each angle goes from its lane through LDS to the angle's lanes (a broadcast
+// read of G addresses).  Then, as the reference (T inverted, then ZGEMMs), W1 =
+// e^{i phi} R V1s T^-1 and W2 = e^{-i phi} R* U1s T^-1, rho = W1 V0s^T, kappa10 =
+// W1 U0s^T, kappa01 = -W2 V0s^T (ROKAPPAphiomega,
+// Codes/PNAMP/PNAMP_Proj.f90:459-551), on v_mfma_f64_4x4x4_4b: its four blocks
+// take four-row strips of T^-T or W (of any of the wave's angles, so h = 20 wastes
+// nothing, h = 22 a sixth) and share the tile of the right operand, which comes
+// from memory one tile column ahead.  All strips of the left operand are in
+// registers, so a product is written over it in LDS: one block per angle, and
+// the LDS holds eight waves per CU at h = 20.
+//
+// Bound by latency at those two waves per SIMD.  At h = 20 (15 pairs x 1000 Euler
+// points, 9 angles; the FP64 rate alone would take 0.46 ms): inversion 1.45 ms,
+// products, <J^2> and traces 1.5 ms, lists 1.2 ms, 4.3 ms in all.  One angle per
+// wave with T^T and both right-hand sides in 60 lanes, the pivot column by four
+// v_readlane per multiplier, took 5.40 ms (8,148 VALU instructions per angle);
+// this grouping with the products as scalar-operand FMAs 6.0 ms, with the
+// lists as gathered terms (four rho reads a term, 12 per step) 4.63 ms.  h = 12 (21
+// x 384 points, 7 angles): 910 -> 555 us, h = 22 (28 x 567, 4 angles): 4.8 -> 3.05 ms.
+//
+// <J^2> pieces (ZJ2_0, Codes/PNAMP/PNAMP_ME2B.f90:1-152) from the ladder form
+// sum_k J_k (x) J_k = J_z (x) J_z + (J_+ (x) J_- + J_- (x) J_+) / 2 with J_z
+// diagonal and J_+ one off-diagonal inside each orbit:
+//   A = sum_a j_a(j_a+1) rho_aa - sum_k Tr(J_k rho J_k rho) + sum_k Tr(J_k kappa10 J_k^T kappa01^T),
+//   t_+ = Tr(J_+ rho), t_- = Tr(J_- rho), t_z = Tr(J_z rho),
+// so <J^2> = A_p + A_n + (t_zp + t_zn)^2 + (t_+p + t_+n)(t_-p + t_-n).
+//
+// The eight-term list sum of HFB_Energy_COMPLEX
+// (Codes/PNAMP/PNAMP_Energy_OpenMP.f90:5-100) is regrouped exactly: with
+// A01 = kappa01 - kappa01^T and A10 = kappa10 - kappa10^T,
+//   (1/4) V [r_ijkl - r_jikl - r_ijlk + r_jilk + d (r_klij - r_klji - r_lkij + r_lkji)]
+//   = V [rho_ki rho_lj - rho_li rho_kj + A01_ij A10_kl / 4
+//        + d (rho_ik rho_jl - rho_jk rho_il + A01_kl A10_ij / 4)].
+// The kappa part runs first (A-blocks of all angles in LDS: A01 in the strict
+// upper, A10 / 4 in the strict lower triangle), then the rho part in the same
+// LDS, both as bilinear forms (bil_sum).
+constexpr int dens_angles(int h) { return 64 / h < 8 ? 64 / h : 8; }
+constexpr int dens_strips(int h) { return (dens_angles(h) * ((h + 3) / 4) + 3) / 4; }
+// T^-1 and W in strips in registers, and ~60 for the rest
+constexpr int dens_default_waves(int h) { return h > 4 && 8 * ((h + 3) / 4) * dens_strips(h) + 60 <= 168 ? 3 : 2; }
+
+template <int H, int MIX>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(dens_default_waves(H)))) void k_fac_dens(PhiParams p) {
+  constexpr int HH = H * H, G = dens_angles(H), LD = H + 1, BS = H * LD;  // (odd LD: rows and columns without bank conflicts)
+  constexpr int KP = (HH + 31) / 32 * 32;  // V-contraction K padded to the MFMA tile
+  constexpr int NPU = H / 2;               // index pairs a < b per lane: (c, c + u mod H), u = 1 .. H / 2
+  constexpr int HK = (H + 3) & ~3;         // pivot keys per angle, padded for 16-byte reads
+  // one block of LD x H per angle: pivot columns and keys, T^-1, W2, kappa01,
+  // W1, kappa10, the A-block (ld H), rho; the closing sums take 12 values per
+  // lane
+  constexpr int RED2 = 64 * 13 / 2, GJ2 = G * H + (G * HK + 3) / 4;
+  constexpr int SH2 = G * BS > RED2 ? (G * BS > GJ2 ? G * BS : GJ2) : (RED2 > GJ2 ? RED2 : GJ2);
+  __shared__ double2 sh[SH2];
+  __shared__ double mt[2 * H];  // m, <m+1|J_+|m> per state (20 KB of LDS in all at h = 20: eight waves per CU)
+  const int lane = threadIdx.x;
+  // XCD-aware order: consecutive logical indices (the waves of one setup
+  // block) stay on one XCD and its L2; gridDim.x is a multiple of 8.
+  const unsigned L = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (L >= (unsigned)p.nwg) return;
+  const int n = p.n, nd = p.nd;
+  const int grp = (int)(L % (unsigned)p.ngrp);
+  unsigned t0 = L / (unsigned)p.ngrp;
+  const int sp = (int)(t0 & 1u);
+  t0 >>= 1;
+  const int iang = (int)(t0 % (unsigned)p.NE), ip = (int)(t0 / (unsigned)p.NE);
+  const size_t blk = ((size_t)ip * p.NE + iang) * 2 + sp;
+  const bool act = lane / H < p.geff;                  // lanes past the group's angles repeat angle 0 and store nothing
+  const int gg = act ? lane / H : 0, c = lane % H;
+  const int f = min(grp * p.geff + gg, nd - 1);        // (a last group with fewer angles repeats the last one)
+  const double2 *X = p.sbuf + blk * 5 * HH, *Y = X + HH;
+  const double2 *E1 = X + 2 * HH, *E2 = X + 3 * HH;
+  const int q0 = p.q0[ip];
+  const double *V0 = p.VfT + ((size_t)q0 * 2 + sp) * HH, *U0 = p.UfT + ((size_t)q0 * 2 + sp) * HH;
+  const double2 e1 = cexpi((2.0 * M_PI / p.nphi) * f);
+  double2 *const B = sh + gg * BS;  // this angle's block
+  for (int i = lane; i < 2 * H; i += 64) mt[i] = p.mtab[i];
+
+  // ---- S = T^-T
+  int info = 0;
+  {
+    double2 col[H];
+#pragma unroll
+    for (int r = 0; r < H; ++r) col[r] = cadd(cmul(e1, X[c + r * H]), cmul(cconj(e1), Y[c + r * H]));
+    double2 *const pc = sh + gg * H;                           // pivot column of the angle
+    unsigned *const keys = (unsigned *)(sh + G * H) + gg * HK;  // pivot keys of its columns
+    if (act && c == 0)
+      for (int k = H; k < HK; ++k) keys[k] = 0u;
+    if (act) keys[c] = pivot_key_hi<5>(cabs1(col[0]), c);
+    bool used = false;
+    int myj = 0;
+    unsigned qp[(H + 3) / 4];
+#pragma unroll
+    for (int k = 0; k < (H + 3) / 4; ++k) qp[k] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      unsigned best = 0u;
+#pragma unroll
+      for (int w = 0; w < HK / 4; ++w) {
+        const uint4 kk = ((const uint4 *)keys)[w];
+        best = max(max(best, max(kk.x, kk.y)), max(kk.z, kk.w));
+      }
+      const int q = 31 - (int)(best & 31u);
+      qp[k / 4] |= (unsigned)q << (8 * (k % 4));
+      const bool piv = c == q;
+      if (piv) {
+        used = true;
+        myj = k;
+        if (act) {
+#pragma unroll
+          for (int r = 0; r < H; ++r) pc[r] = col[r];
+        }
+        // the pivot column starts again from zero (its new entries are -m / pivot)
+#pragma unroll
+        for (int r = 0; r < H; ++r)
+          if (r != k) col[r] = cz();
+      }
+      __syncthreads();
+      const double2 pv = pc[k];
+      if (pv.x == 0.0 && pv.y == 0.0 && info == 0) info = k + 1;
+      __asm__ volatile("" : "+v"(info));  // (a test sunk to the INFO store would keep every pivot in registers)
+      const double2 inv = crecip_nr(pv);
+      double2 pr = cmul(col[k], inv);
+      pr.x = piv ? inv.x : pr.x;
+      pr.y = piv ? inv.y : pr.y;
+      // row k + 1 first: its keys are the next step's
+#pragma unroll
+      for (int rr = 1; rr < H; ++rr) {
+        if (rr % 4 == 1) __builtin_amdgcn_sched_barrier(0);  // bounds the LDS reads in flight (registers)
+        const int r = (k + rr) % H;
+        cfms(col[r], pc[r], pr);
+        if (rr == 1 && k + 1 < H && act) keys[c] = used ? 0u : pivot_key_hi<5>(cabs1(col[r]), c);
+      }
+      col[k] = pr;
+      __syncthreads();
+    }
+    // column c was pivoted at step myj: col[k] = S(q_k, myj) = T^-1(myj, q_k); lane q_k
+    // takes column q_k of T^-1
+    if (act) {
+#pragma unroll
+      for (int k = 0; k < H; ++k) B[(int)((qp[k / 4] >> (8 * (k % 4))) & 255u) * LD + myj] = col[k];
+    }
+    if (act && c == 0) B[H] = e1;  // (a padding entry of the block)
+    __syncthreads();
+  }
+  // ---- products on 4 x 4 tiles of the FP64 matrix units (v_mfma_f64_4x4x4_4b:
+  // D_b += A_b B_b for four b at once): A_b are four strips of four rows of the
+  // left matrices (NT strips an angle, so strips of several angles share an
+  // instruction), B the same tile of the shared right operand in all four
+  constexpr int NT = (H + 3) / 4, NS = dens_strips(H);
+  const int li = lane & 3, lb = (lane >> 2) & 3, lk = lane >> 4;  // A: row li, k lk of b = lb; B: k lk, column li; D: row lk, column li
+  const int ns = p.geff * NT;
+  auto kk = [&](int kt) { return H % 4 == 0 ? 4 * kt + lk : min(4 * kt + lk, H - 1); };
+  unsigned sid[NS];  // strip of block lb in group g: angle, strip << 8
+#pragma unroll
+  for (int g = 0; g < NS; ++g) sid[g] = min(4 * g + lb, ns - 1) / NT + ((min(4 * g + lb, ns - 1) % NT) << 8);
+  auto strip = [&](int g, int &a, int &st) {
+    unsigned x = sid[g];
+    __asm__ volatile("" : "+v"(x));  // (offsets are made at each use, not kept over the loops)
+    a = (int)(x & 255u);
+    st = (int)(x >> 8);
+  };
+  // strips from the blocks: lane (li, lb, lk) takes entries (4 st + li, 4 kt + lk), row stride LD
+  auto load = [&](double2 (&x)[NS][NT]) {
+#pragma unroll
+    for (int g = 0; g < NS; ++g) {
+      int a, st;
+      strip(g, a, st);
+      const double2 *r = sh + a * BS + min(4 * st + li, H - 1) * LD;
+#pragma unroll
+      for (int kt = 0; kt < NT; ++kt) x[g][kt] = r[kk(kt)];
     }
     __syncthreads();
-    if (PASSES == 1 || pass == 1) {
+  };
+  auto mac = [](double a, double b, double d) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, d, 0, 0, 0); };
+  // columns 4 jt .. 4 jt + 3 of the right operand F^T (row-major F, zero past H)
+  auto tiles = [&](auto F, int jt, auto (&x)[NT]) {
+    const auto *r = F + min(4 * jt + li, H - 1) * H;
 #pragma unroll
-      for (int u = 0; u < NE64; ++u) {
-        const int e = lane + 64 * u, a = e % H, b = e / H;
-        a01r[u] = (e < HH && a < b) ? csub(B1[a + b * H], B1[b + a * H]) : cz();
+    for (int kt = 0; kt < NT; ++kt) {
+      x[kt] = r[kk(kt)];
+      if (H % 4 != 0 && kt == NT - 1 && 4 * kt + lk >= H) x[kt] = {};
+    }
+  };
+  // x F^T for all strips: f(angle, row, column, value)
+  auto product = [&](auto F, const double2 (&x)[NS][NT], auto &&f) {
+    typedef typename std::remove_cv<typename std::remove_reference<decltype(*F)>::type>::type T;
+    constexpr bool AHEAD = NT * sizeof(T) <= 80;  // (registers)
+    T cur[NT], nxt[NT];
+    if (AHEAD) tiles(F, 0, cur);
+#pragma unroll 1
+    for (int jt = 0; jt < NT; ++jt) {
+      if (AHEAD) {
+        tiles(F, min(jt + 1, NT - 1), nxt);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        tiles(F, jt, cur);
       }
-      // U0s sweep: kappa10 (W1 rows) with the kappa part of <J^2>,
-      //   sum_ab kappa10(a,b) [m_a m_b kappa01(a,b) + c_a c_{b+1} kappa01(a-1,b+1) / 2
-      //                        + c_{a+1} c_b kappa01(a+1,b-1) / 2]
-      // (c_a = <m_a + 1|J_+|m_a>, 0 at m_a = j_a, so a - 1 is in a's orbit
-      // when c_a != 0); kappa10(a, b - 1) replaces kappa01(a, b - 1) in B1 one
-      // column late, after the last read of that column
-      const int a = w1lane ? irow : 0;
-      const double ma = mz[a], ca = cp[a], ca1 = (a + 1 < H) ? cp[a + 1] : 0.0;
-      const int am = (a > 0) ? a - 1 : 0, ap = (a + 1 < H) ? a + 1 : a;
-      double2 prev = cz();
-#pragma unroll 2
-      for (int j = 0; j < H; ++j) {
-        double2 acc = cz();
 #pragma unroll
-        for (int k = 0; k < H; ++k) rfma(acc, U0T[j * H + k], w[k]);
-        if (w1lane) {
-          double2 x = cscale(ma * mz[j], B1[a + j * H]);
-          if (j + 1 < H) x = cadd(x, cscale(0.5 * ca * cp[j + 1], B1[am + (j + 1) * H]));
-          if (j > 0) x = cadd(x, cscale(0.5 * ca1 * cp[j], B1[ap + (j - 1) * H]));
-          cfma(ajk, acc, x);
-          if (j > 0) B1[a + (j - 1) * H] = prev;
-          prev = acc;
+      for (int g = 0; g < NS; ++g) {
+        if (4 * g >= ns) continue;
+        double d0 = 0.0, d1 = 0.0, d2 = 0.0, d3 = 0.0;
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt) {
+          if constexpr (sizeof(T) == 16) {
+            d0 = mac(x[g][kt].x, cur[kt].x, d0);
+            d1 = mac(x[g][kt].x, cur[kt].y, d1);
+            d2 = mac(x[g][kt].y, cur[kt].y, d2);
+            d3 = mac(x[g][kt].y, cur[kt].x, d3);
+          } else if (kt % 2 == 0) {
+            d0 = mac(x[g][kt].x, cur[kt], d0);
+            d1 = mac(x[g][kt].y, cur[kt], d1);
+          } else {
+            d2 = mac(x[g][kt].x, cur[kt], d2);
+            d3 = mac(x[g][kt].y, cur[kt], d3);
+          }
         }
+        int a, st;
+        strip(g, a, st);
+        const int r = 4 * st + lk, j = 4 * jt + li;
+        if (4 * g + lb < ns && r < H && j < H)
+          f(a, r, j, sizeof(T) == 16 ? make_double2(d0 - d2, d1 + d3) : make_double2(d0 + d2, d1 + d3));
       }
-      if (w1lane) B1[a + (H - 1) * H] = prev;
-      __syncthreads();
-    }
-  }
-
-  // ---- traces, the rho part of <J^2>, kinetic energy
-  // per element rho(a, b): Ekin t1(b, a); <J^2> -m_a m_b rho(b, a) - c_a c_b
-  // rho(b-1, a-1) + j_a(j_a+1) d_ab; traces d_ab, m_a d_ab, c_a d_{a,b+1},
-  // c_b d_{b,a+1} -- eight coefficients tabled per element, no branches
-  double2 tr = cz(), ek = cz(), aj = ajk, tp = cz(), tm = cz(), tz = cz();
-  const double2 *jt = p.jtab + (size_t)sp * HH * 4;
-  for (int e = lane; e < HH; e += 64) {
-    const int a = e % H, b = e / H;
-    const double2 c01 = jt[4 * e], c23 = jt[4 * e + 1], c45 = jt[4 * e + 2], c67 = jt[4 * e + 3];
-    const double2 rab = B0[a + b * HP];
-    const double2 rba = B0[b + a * HP];
-    const double2 rl = B0[(b > 0 ? b - 1 : 0) + (a > 0 ? a - 1 : 0) * HP];
-    rfma(ek, c01.x, rab);
-    rfma(aj, -c01.y, cmul(rab, rba));
-    rfma(aj, -c23.x, cmul(rab, rl));
-    rfma(tr, c23.y, rab);
-    rfma(tz, c45.x, rab);
-    rfma(aj, c45.y, rab);
-    rfma(tp, c67.x, rab);
-    rfma(tm, c67.y, rab);
-  }
-  // A10 / 4 = (kappa10 - kappa10^T) / 4, then the A-block
-  double2 a10r[NE64];
 #pragma unroll
-  for (int u = 0; u < NE64; ++u) {
-    const int e = lane + 64 * u, a = e % H, b = e / H;
-    a10r[u] = (e < HH && a < b) ? cscale(0.25, csub(B1[a + b * H], B1[b + a * H])) : cz();
+      for (int kt = 0; kt < NT && AHEAD; ++kt) cur[kt] = nxt[kt];
+    }
+    __syncthreads();
+  };
+  // pair u of the lane: a < b of {c, c + u + 1 mod H}; the last u counts each pair twice: c < H / 2 only
+  // (c passes through an empty asm: the pairs are made again at each use instead
+  // of being kept in registers over the products)
+  auto pair_ab = [&](int u, int &a, int &b) -> bool {
+    int x = c;
+    __asm__ volatile("" : "+v"(x));
+    const int d = (x + u + 1 >= H) ? x + u + 1 - H : x + u + 1;
+    a = min(x, d);
+    b = max(x, d);
+    return u + 1 < NPU || x < NPU;
+  };
+  double2 a01[NPU], a10[NPU], w[NS][NT];
+  {
+    double2 t[NS][NT];
+    load(t);  // rows of T^-T: block entry r + c LD is T^-1(r, c)
+    // W2^T = T^-T E2^T e^{-i phi}; its rows j (of E) are stored with stride LD
+    product(E2, t, [&](int a, int r, int j, double2 v) { sh[a * BS + j * LD + r] = cmul(cconj(sh[a * BS + H]), v); });
+    load(w);
+    product(V0, w, [&](int a, int r, int j, double2 v) { sh[a * BS + r + j * LD] = make_double2(-v.x, -v.y); });  // kappa01
+#pragma unroll
+    for (int u = 0; u < NPU; ++u) {
+      if (u % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // (bounds the reads in flight: registers)
+      int a, b;
+      pair_ab(u, a, b);
+      a01[u] = csub(B[a + b * LD], B[b + a * LD]);
+    }
+    __syncthreads();
+    product(E1, t, [&](int a, int r, int j, double2 v) { sh[a * BS + j * LD + r] = cmul(sh[a * BS + H], v); });
+  }
+  load(w);
+  product(U0, w, [&](int a, int r, int j, double2 v) { sh[a * BS + r + j * LD] = v; });  // kappa10
+#pragma unroll
+  for (int u = 0; u < NPU; ++u) {
+    if (u % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    int a, b;
+    pair_ab(u, a, b);
+    a10[u] = cscale(0.25, csub(B[a + b * LD], B[b + a * LD]));
   }
   __syncthreads();
+  // the A-blocks, leading dimension H (diagonals are never read with a weight)
+  double2 *const AB = sh + gg * HH;
 #pragma unroll
-  for (int u = 0; u < NE64; ++u) {
-    const int e = lane + 64 * u, a = e % H, b = e / H;
-    if (e < HH && a < b) {
-      B1[a + b * H] = a01r[u];
-      B1[b + a * H] = a10r[u];
+  for (int u = 0; u < NPU; ++u) {
+    int a, b;
+    if (pair_ab(u, a, b) && act) {
+      AB[a + b * H] = a01[u];
+      AB[b + a * H] = a10[u];
     }
   }
+  if (act) AB[c + c * H] = cz();
   __syncthreads();
-  double2 e2b = cz();
+  // ---- kappa part of <J^2>: sum_{a != b} (A10 / 4)(a, b) [m_a m_b A01(a, b) +
+  // c_a c_{b+1} A01(a-1, b+1) / 2 + c_{a+1} c_b A01(a+1, b-1) / 2], twice the sum
+  // over a < b (c_a = <m_a + 1|J_+|m_a>, 0 at m_a = j_a, so a - 1 is in a's orbit
+  // when c_a != 0)
+  const double *const mz = mt, *const cp = mt + H;
+  double2 aj = cz();
+#pragma unroll
+  for (int u = 0; u < NPU; ++u) {
+    __builtin_amdgcn_sched_barrier(0);
+    int a, b;
+    const double on = pair_ab(u, a, b) ? 2.0 : 0.0;
+    const int am = max(a - 1, 0), bp = min(b + 1, H - 1), ap = a + 1, bm = b - 1;  // am < bp; ap, bm cross at b = a + 1
+    double2 x = cscale(mz[a] * mz[b], a01[u]);
+    rfma(x, (b + 1 < H) ? 0.5 * cp[a] * cp[bp] : 0.0, AB[am + bp * H]);
+    const double s3 = (ap < bm) ? 0.5 : (ap > bm ? -0.5 : 0.0);
+    rfma(x, s3 * cp[ap] * cp[b], AB[min(ap, bm) + max(ap, bm) * H]);
+    cfma(aj, cscale(on, a10[u]), x);
+    __asm__ volatile("" : "+v"(aj.x), "+v"(aj.y));  // (summed here, not after all operands are loaded)
+  }
+  // ---- species list, kappa part: V A01_ij A10_kl / 4
+  constexpr int NC = (G + 1) / 2;  // B column tiles of two angles
+  double2 e2b[NC];
+#pragma unroll
+  for (int g = 0; g < NC; ++g) e2b[g] = cz();
   if (MIX != MIX_FP64) {
     // the species list moves to k_vgemm: A01 (dot vector) and A10 (operand)
-    double2 *a01 = p.a01 + obase * HH;
-    for (int e = lane; e < HH; e += 64) {
-      const int a = e % H, b = e / H;
-      const double2 x01 = (a < b) ? B1[a + b * H] : (a > b ? cneg(B1[b + a * H]) : cz());
-      const double2 x10 = (a < b) ? cscale(4.0, B1[b + a * H]) : (a > b ? cscale(-4.0, B1[a + b * H]) : cz());
-      a01[e] = x01;
-      put_b<MIX, KP>(p.ba10[sp], p.ba10_lo[sp], e, 2 * mcol, x10.x);
-      put_b<MIX, KP>(p.ba10[sp], p.ba10_lo[sp], e, 2 * mcol + 1, x10.y);
+    for (int e = lane; e < G * HH; e += 64) {
+      const int g = e / HH, x = e % HH, a = x % H, b = x / H;
+      const int fg = grp * p.geff + g;
+      if (g >= p.geff || fg >= nd) continue;
+      const double2 *A = sh + g * HH;
+      const size_t mcol = ((size_t)ip * p.NE + iang) * nd + fg;  // GEMM column pair of this phi in species sp
+      const double2 v01 = A[min(a, b) + max(a, b) * H], v10 = A[max(a, b) + min(a, b) * H];
+      const double sg = (a < b) ? 1.0 : (a > b ? -1.0 : 0.0);
+      p.a01[(blk * nd + fg) * HH + x] = cscale(sg, v01);
+      put_b<MIX, KP>(p.ba10[sp], p.ba10_lo[sp], x, 2 * mcol, 4.0 * sg * v10.x);
+      put_b<MIX, KP>(p.ba10[sp], p.ba10_lo[sp], x, 2 * mcol + 1, 4.0 * sg * v10.y);
     }
   } else {
-    // ---- species list: V [rho_ki rho_lj - rho_li rho_kj + A01_ij A10_kl / 4]
-    const uint4 *lo = p.lofs[sp];
-    const int nl = p.nl[sp];
-    const char *lds = (const char *)sA;
-    auto ld = [&](unsigned off) { return *(const double2 *)(lds + off); };
-    for (int q0 = lane; q0 < nl; q0 += 4 * 64) {
-      uint4 o[4], w[4];  // four entries loaded ahead of their LDS reads
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        o[u] = lo[q0 + 64 * u];
-        w[u] = lo[nl + q0 + 64 * u];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const double2 r1 = ld(o[u].x), r2 = ld(o[u].y), r3 = ld(o[u].z), r4 = ld(o[u].w), x = ld(w[u].x),
-                      y = ld(w[u].y);
-        const double me = __hiloint2double((int)w[u].w, (int)w[u].z);
-        double2 t = cmul(r1, r2);
-        cfms(t, r3, r4);
-        cfma(t, x, y);
-        rfma(e2b, me, t);
+    if (p.geff <= 2) bil_sum<1>(p.fkap[sp], (const char *)sh, HH * 16, p.geff, lane, e2b);
+    else bil_sum<NC>(p.fkap[sp], (const char *)sh, HH * 16, p.geff, lane, e2b);
+  }
+  __syncthreads();
+  // ---- rho, E_kin, traces
+  product(V0, w, [&](int a, int r, int j, double2 v) {
+    sh[a * BS + r + j * LD] = v;
+    const int fa = grp * p.geff + a;
+    if (fa < nd) {
+      p.rho[(blk * nd + fa) * HH + r + j * H] = v;
+      if (MIX != MIX_FP64) {
+        const size_t mc = ((size_t)ip * p.NE + iang) * nd + fa;
+        put_b<MIX, KP>(p.brho[sp], p.brho_lo[sp], r + j * H, 2 * mc, v.x);
+        put_b<MIX, KP>(p.brho[sp], p.brho_lo[sp], r + j * H, 2 * mc + 1, v.y);
       }
     }
+  });
+  const double2 tr = B[c + c * LD];
+  const double mc_ = mz[c], cc = cp[c], cc1 = (c + 1 < H) ? cp[c + 1] : 0.0;
+  const double2 tz = cscale(mc_, tr);
+  const double2 tp = cscale(cc, B[c + max(c - 1, 0) * LD]);                    // J_+: rho(c, c - 1)
+  const double2 tm = cscale(cc1, B[c + min(c + 1, H - 1) * LD]);               // J_-: rho(c, c + 1)
+  rfma(aj, p.mtab[2 * H + c], tr);
+  // E_kin = sum_b t1(b, c) rho(c, b), and - sum_b rho(c, b) [m_c m_b rho(b, c) +
+  // c_c c_b rho(b - 1, c - 1)]
+  double2 ek = cz();
+  const double *const t1 = p.t1b + (size_t)(sp * H) + (size_t)(sp * H + c) * n;
+  const auto umz = ro_const(p.mtab), ucp = ro_const(p.mtab + H);
+#pragma unroll 4
+  for (int b = 0; b < H; ++b) {
+    double2 x = cscale(mc_ * umz[b], B[b + c * LD]);
+    rfma(x, cc * ucp[b], B[max(b - 1, 0) + max(c - 1, 0) * LD]);
+    const double2 rcb = B[c + b * LD];
+    cfms(aj, rcb, x);
+    rfma(ek, t1[b], rcb);
   }
-  // the 14 sums: quad sums by DPP, the 16 quad sums of each value through
-  // LDS (sA is free after the list), lane q < 14 adds those of value q and
-  // writes it (Re, Im of output slots 1..7)
-  double v[14] = {e2b.x, e2b.y, ek.x, ek.y, tr.x, tr.y, aj.x, aj.y, tp.x, tp.y, tm.x, tm.y, tz.x, tz.y};
+  // ---- species list, rho part: V [rho_ki rho_lj - rho_li rho_kj]
+  if (MIX == MIX_FP64) {
+    if (p.geff <= 2) bil_sum<1>(p.frho[sp], (const char *)sh, BS * 16, p.geff, lane, e2b);
+    else bil_sum<NC>(p.frho[sp], (const char *)sh, BS * 16, p.geff, lane, e2b);
+  }
+  // ---- sums: the list over the wavefront, the others over an angle's H lanes
+  double2 el = cz();  // lane (g, c): the list sum of angle g, columns 2 (g % 2), + 1 of tile g / 2
 #pragma unroll
-  for (int q = 0; q < 14; ++q) {
-    v[q] += dpp_f64<0xB1, 0xF>(v[q]);  // quad_perm [1,0,3,2]
-    v[q] += dpp_f64<0x4E, 0xF>(v[q]);  // quad_perm [2,3,0,1]
+  for (int g = 0; g < G; ++g) {
+    if (g < p.geff) {
+      const bool in = ((lane >> 1) & 1) == (g & 1);
+      const double x = wave_sum_dpp(in ? e2b[g / 2].x : 0.0), y = wave_sum_dpp(in ? e2b[g / 2].y : 0.0);
+      if (g == gg) el = make_double2(x, y);
+    }
   }
-  double *red = (double *)sA;
-  static_assert(sizeof(sA) >= 16 * 14 * sizeof(double), "sA holds the closing reduction");
+  const double v[12] = {ek.x, ek.y, tr.x, tr.y, aj.x, aj.y, tp.x, tp.y, tm.x, tm.y, tz.x, tz.y};
   __syncthreads();
-  if ((lane & 3) == 0) {
+  double *const red = (double *)sh;
 #pragma unroll
-    for (int q = 0; q < 14; ++q) red[(lane >> 2) * 14 + q] = v[q];
-  }
+  for (int q = 0; q < 12; ++q) red[lane * 13 + q] = v[q];
   __syncthreads();
-  double2 *o = p.out + obase * FAC_OUT;
-  if (lane < 14) {
+  for (int e = lane; e < G * 12; e += 64) {
+    const int g = e / 12, q = e % 12, fg = grp * p.geff + g;
+    if (g >= p.geff || fg >= nd) continue;
     double tot = 0.0;
-#pragma unroll
-    for (int qd = 0; qd < 16; ++qd) tot += red[qd * 14 + lane];
-    ((double *)o)[2 + lane] = tot;
+#pragma unroll 4
+    for (int i = 0; i < H; ++i) tot += red[(g * H + i) * 13 + q];
+    ((double *)(p.out + (blk * nd + fg) * FAC_OUT))[4 + q] = tot;  // slots 2 .. 7: E_kin, Tr rho, A, t_+, t_-, t_z
   }
-  if (lane == 0) {
+  int le = lane;
+  __asm__ volatile("" : "+v"(le));  // (made again, not kept in registers)
+  const int fe = grp * p.geff + le / H;
+  if (le % H == 0 && le / H < p.geff && fe < nd) {
+    const size_t ob = blk * nd + fe;
+    double2 *const o = p.out + ob * FAC_OUT;
+    o[1] = el;
     o[8] = cz();
-    p.status[obase] = info;
-  }
+    p.status[ob] = info;
   }
 }
 
@@ -1669,44 +1858,54 @@ static bool launch_vgemm(int h, int mix, dim3 grid, hipStream_t s, const VGemmPa
 
 // Occupancy variants of the FP64 factored form that the autotuner times
 // (species sizes h >= 8; smaller spaces take the defaults): Pfaffian part at
-// three, four or five waves per SIMD, the rest at its default or, for
-// h <= 16, four (a tighter register cap).  0 = the default.
+// three, four or five waves per SIMD (0 = the default), and the chunk size.
+// The densities have one variant: their LDS allows no more waves than the
+// default.
 struct FacTune {
-  int pf_waves = 0, rest_waves = 0, chunk_div = 1;
+  int pf_waves = 0, chunk_div = 1;
 };
 
 // route: 0 the 2h x 2h Pfaffian, 1 the Schur route for every state, 2 both
-// kernels (pp.pfs_ok names each pair's); a pf_waves choice takes the 2h x 2h one
+// kernels (pp.pfs_ok names each pair's); a pf_waves choice takes the 2h x 2h one.
+// blocks: (pair, Euler point, species) blocks of the chunk
 template <int H>
-static void launch_phi(int mix, const FacTune &t, int route, unsigned grid, hipStream_t s, const PhiParams &pp) {
-  const dim3 g(grid), b(64);
-  if (route >= 1 && t.pf_waves == 0) hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_PFS>), g, b, 0, s, pp);
+static void launch_phi(int mix, const FacTune &t, int route, size_t blocks, hipStream_t s, PhiParams pp) {
+  const dim3 b(64);
+  auto grid = [](size_t nwg) { return dim3((unsigned)((nwg + 7) / 8 * 8)); };
+  pp.nwg = (int)(blocks * pp.nd);
+  const dim3 g = grid(blocks * pp.nd);
+  if (route >= 1 && t.pf_waves == 0) hipLaunchKernelGGL((k_fac_phi<H, PART_PFS>), g, b, 0, s, pp);
   if (route == 1 && t.pf_waves == 0) {
-  } else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 3) hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_PF, 3>), g, b, 0, s, pp);
-  else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 4) hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_PF, 4>), g, b, 0, s, pp);
-  else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 5) hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_PF, 5>), g, b, 0, s, pp);
-  else hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_PF>), g, b, 0, s, pp);
-  if (mix == MIX_FP32) hipLaunchKernelGGL((k_fac_phi<H, MIX_FP32, PART_REST>), g, b, 0, s, pp);
-  else if (mix == MIX_BF16) hipLaunchKernelGGL((k_fac_phi<H, MIX_BF16, PART_REST>), g, b, 0, s, pp);
-  else if (H >= 8 && H <= 16 && t.rest_waves == 4)
-    hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_REST, 4>), g, b, 0, s, pp);
-  else hipLaunchKernelGGL((k_fac_phi<H, MIX_FP64, PART_REST>), g, b, 0, s, pp);
+  } else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 3) hipLaunchKernelGGL((k_fac_phi<H, PART_PF, 3>), g, b, 0, s, pp);
+  else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 4) hipLaunchKernelGGL((k_fac_phi<H, PART_PF, 4>), g, b, 0, s, pp);
+  else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 5) hipLaunchKernelGGL((k_fac_phi<H, PART_PF, 5>), g, b, 0, s, pp);
+  else hipLaunchKernelGGL((k_fac_phi<H, PART_PF>), g, b, 0, s, pp);
+  // the fewest groups of angles, of equal size; more groups while all waves
+  // still run at once, one per SIMD (one sd pair, 10 Euler points, 4 angles:
+  // 31 us in groups of five, 23 us one by one)
+  pp.ngrp = (pp.nd + dens_angles(H) - 1) / dens_angles(H);
+  pp.geff = (pp.nd + pp.ngrp - 1) / pp.ngrp;
+  while (pp.geff > 1 && blocks * (size_t)((pp.nd + pp.geff - 2) / (pp.geff - 1)) <= 1024) --pp.geff;
+  pp.ngrp = (pp.nd + pp.geff - 1) / pp.geff;
+  pp.nwg = (int)(blocks * pp.ngrp);
+  const dim3 gd = grid(blocks * pp.ngrp);
+  if (mix == MIX_FP32) hipLaunchKernelGGL((k_fac_dens<H, MIX_FP32>), gd, b, 0, s, pp);
+  else if (mix == MIX_BF16) hipLaunchKernelGGL((k_fac_dens<H, MIX_BF16>), gd, b, 0, s, pp);
+  else hipLaunchKernelGGL((k_fac_dens<H, MIX_FP64>), gd, b, 0, s, pp);
 }
 
 // Scratch (register spill) bytes per lane of the FP64 variant kernels a
 // tuning choice launches; the autotuner only takes spill-free variants.
 template <int H>
 static size_t phi_scratch(const FacTune &t, bool schur) {
-  const void *pf = (const void *)k_fac_phi<H, MIX_FP64, PART_PF>;
-  if (schur && t.pf_waves == 0) pf = (const void *)k_fac_phi<H, MIX_FP64, PART_PFS>;
-  if (H >= 8 && t.pf_waves == 3) pf = (const void *)k_fac_phi<H, MIX_FP64, PART_PF, 3>;
-  if (H >= 8 && t.pf_waves == 4) pf = (const void *)k_fac_phi<H, MIX_FP64, PART_PF, 4>;
-  if (H >= 8 && t.pf_waves == 5) pf = (const void *)k_fac_phi<H, MIX_FP64, PART_PF, 5>;
-  const void *rest = (const void *)k_fac_phi<H, MIX_FP64, PART_REST>;
-  if (H >= 8 && H <= 16 && t.rest_waves == 4) rest = (const void *)k_fac_phi<H, MIX_FP64, PART_REST, 4>;
-  hipFuncAttributes a{}, b{};
-  if (hipFuncGetAttributes(&a, pf) != hipSuccess || hipFuncGetAttributes(&b, rest) != hipSuccess) return (size_t)-1;
-  return a.localSizeBytes + b.localSizeBytes;
+  const void *pf = (const void *)k_fac_phi<H, PART_PF>;
+  if (schur && t.pf_waves == 0) pf = (const void *)k_fac_phi<H, PART_PFS>;
+  if (H >= 8 && t.pf_waves == 3) pf = (const void *)k_fac_phi<H, PART_PF, 3>;
+  if (H >= 8 && t.pf_waves == 4) pf = (const void *)k_fac_phi<H, PART_PF, 4>;
+  if (H >= 8 && t.pf_waves == 5) pf = (const void *)k_fac_phi<H, PART_PF, 5>;
+  hipFuncAttributes a{};
+  if (hipFuncGetAttributes(&a, pf) != hipSuccess) return (size_t)-1;
+  return a.localSizeBytes;
 }
 
 static size_t phi_scratch_h(int h, const FacTune &t, bool schur) {
@@ -1728,20 +1927,20 @@ static size_t phi_scratch_h(int h, const FacTune &t, bool schur) {
 
 // Species sizes h = n / 2 with an instantiated k_fac_phi (every h is even:
 // an orbit holds 2j + 1 states).
-static bool launch_phi_h(int h, int mix, const FacTune &t, int route, unsigned grid, hipStream_t s,
+static bool launch_phi_h(int h, int mix, const FacTune &t, int route, size_t blocks, hipStream_t s,
                          const PhiParams &pp) {
   switch (h) {
-    case 2: launch_phi<2>(mix, t, route, grid, s, pp); return true;
-    case 4: launch_phi<4>(mix, t, route, grid, s, pp); return true;
-    case 6: launch_phi<6>(mix, t, route, grid, s, pp); return true;
-    case 8: launch_phi<8>(mix, t, route, grid, s, pp); return true;
-    case 10: launch_phi<10>(mix, t, route, grid, s, pp); return true;
-    case 12: launch_phi<12>(mix, t, route, grid, s, pp); return true;
-    case 14: launch_phi<14>(mix, t, route, grid, s, pp); return true;
-    case 16: launch_phi<16>(mix, t, route, grid, s, pp); return true;
-    case 18: launch_phi<18>(mix, t, route, grid, s, pp); return true;
-    case 20: launch_phi<20>(mix, t, route, grid, s, pp); return true;
-    case 22: launch_phi<22>(mix, t, route, grid, s, pp); return true;
+    case 2: launch_phi<2>(mix, t, route, blocks, s, pp); return true;
+    case 4: launch_phi<4>(mix, t, route, blocks, s, pp); return true;
+    case 6: launch_phi<6>(mix, t, route, blocks, s, pp); return true;
+    case 8: launch_phi<8>(mix, t, route, blocks, s, pp); return true;
+    case 10: launch_phi<10>(mix, t, route, blocks, s, pp); return true;
+    case 12: launch_phi<12>(mix, t, route, blocks, s, pp); return true;
+    case 14: launch_phi<14>(mix, t, route, blocks, s, pp); return true;
+    case 16: launch_phi<16>(mix, t, route, blocks, s, pp); return true;
+    case 18: launch_phi<18>(mix, t, route, blocks, s, pp); return true;
+    case 20: launch_phi<20>(mix, t, route, blocks, s, pp); return true;
+    case 22: launch_phi<22>(mix, t, route, blocks, s, pp); return true;
     default: return false;
   }
 }
@@ -2595,7 +2794,6 @@ struct pnamp_ctx {
   void *d_pwork = nullptr;
   size_t pwork_bytes = 0;
   double *d_t1b = nullptr;
-  double *d_jtab = nullptr;
   double *d_U = nullptr, *d_V = nullptr, *d_Z = nullptr, *d_det = nullptr;
   int *d_state_status = nullptr;
   int *d_q0 = nullptr, *d_q1 = nullptr, *d_pz = nullptr, *d_pn = nullptr;
@@ -2614,8 +2812,8 @@ struct pnamp_ctx {
   int form = PNAMP_FORM_PLAIN;
   bool separable = false;
   int nme_s[3] = {0, 0, 0};
-  uint4 *d_lofs[2] = {nullptr, nullptr};            // species lists of k_fac_phi (p, n)
-  int nl[2] = {0, 0};
+  BilForm frho[2] = {}, fkap[2] = {};               // species lists of k_fac_dens (p, n), in d_bil
+  double *d_bil = nullptr;
   bool fac_list_ok = false;
   std::string fac_reason;
   double *d_Uf = nullptr, *d_Vf = nullptr, *d_UfT = nullptr, *d_VfT = nullptr;
@@ -2739,6 +2937,101 @@ static int dupload(pnamp_ctx *c, T **p, const T *src, size_t count) {
   if (r) return r;
   if (count) HIPCHK(c, hipMemcpy(*p, src, count * sizeof(T), hipMemcpyHostToDevice));
   return 0;
+}
+
+// Tables of a bilinear form sum C(x, y) a_x b_y over n elements (offsets of x in
+// ofs), appended to buf, with f's pointers as offsets into it; sym: a = b.
+// Rows that share columns (connected through entries of C: equal Delta m and
+// parity) are tiled together by four, a tile takes only the columns with an
+// entry in it, and tiles of similar column counts form a group, so little is
+// padded (pf shell: half of the 15,488 rho entries are non-zero).
+struct BilTerm {
+  int x, y;
+  double v;
+};
+static void bil_table(std::vector<double> &buf, BilForm &f, int n, bool sym, std::vector<BilTerm> &C,
+                      const std::vector<unsigned> &ofs) {
+  std::vector<int> root(2 * n);
+  for (int i = 0; i < 2 * n; ++i) root[i] = i;
+  auto find = [&](int i) {
+    while (root[i] != i) i = root[i] = root[root[i]];
+    return i;
+  };
+  std::vector<char> used(n, 0);
+  for (const BilTerm &e : C) {
+    root[find(e.x)] = find(sym ? e.y : n + e.y);
+    used[e.x] = 1;
+    if (sym) used[e.y] = 1;
+  }
+  std::vector<std::pair<int, int>> ord;  // (component, row)
+  for (int x = 0; x < n; ++x)
+    if (used[x]) ord.push_back({find(x), x});
+  std::sort(ord.begin(), ord.end());
+  std::vector<int> pos(n, n);
+  for (size_t i = 0; i < ord.size(); ++i) pos[ord[i].second] = (int)i;
+  std::vector<size_t> first(n + 1, 0);  // entries by their row's place in ord
+  for (BilTerm &e : C) {
+    if (sym && pos[e.y] < pos[e.x]) std::swap(e.x, e.y);
+    e.x = pos[e.x];
+    ++first[e.x + 1];
+  }
+  for (int x = 0; x < n; ++x) first[x + 1] += first[x];
+  std::vector<BilTerm> T(C.size());
+  for (const BilTerm &e : C) T[first[e.x]++] = e;
+  struct Tile {
+    int x0, nx;
+    size_t e0, e1;       // its entries
+    std::vector<int> y;  // its columns
+  };
+  std::vector<Tile> tiles;
+  std::vector<int> at(n, -1);
+  size_t e = 0;
+  for (size_t i = 0; i < ord.size();) {
+    Tile t{(int)i, 0, e, e, {}};
+    while (i < ord.size() && t.nx < 4 && ord[i].first == ord[t.x0].first) ++t.nx, ++i;
+    for (; e < T.size() && T[e].x < t.x0 + t.nx; ++e)
+      if (at[T[e].y] != t.x0) {
+        at[T[e].y] = t.x0;
+        t.y.push_back(T[e].y);
+      }
+    t.e1 = e;
+    if (!t.y.empty()) tiles.push_back(std::move(t));
+  }
+  std::stable_sort(tiles.begin(), tiles.end(), [](const Tile &a, const Tile &b) { return a.y.size() > b.y.size(); });
+  std::vector<int> pairs;
+  int np = 0;
+  for (size_t g = 0; g < tiles.size(); g += 4) {
+    pairs.push_back(((int)tiles[g].y.size() + 7) / 8);
+    np += pairs.back();
+  }
+  f.np = (np + BIL_RING - 1) / BIL_RING * BIL_RING;
+  const size_t ap = (size_t)f.np + BIL_RING, v0 = (buf.size() + 1) / 2 * 2, c0 = v0 + 128 * ap;
+  buf.resize(c0 + 32 * ap, 0.0);
+  double *const v = buf.data() + v0;
+  uint4 *const of = (uint4 *)(buf.data() + c0);
+  f.v = (const double *)v0;
+  f.ofs = (const uint4 *)c0;
+  std::vector<int> place(n, 0);
+  size_t s0 = 0;  // first step of the group
+  for (size_t g = 0; g < tiles.size(); g += 4) {
+    const size_t last = s0 / 2 + pairs[g / 4] - 1;
+    for (int k = 0; k < 16; ++k) of[last * 16 + k].w = 1u;
+    for (size_t b = 0; b < 4 && g + b < tiles.size(); ++b) {
+      const Tile &t = tiles[g + b];
+      for (int i = 0; i < t.nx; ++i) of[last * 16 + 4 * i + b].z = ofs[ord[t.x0 + i].second];
+      for (size_t k = 0; k < t.y.size(); ++k) {
+        const size_t st = s0 + k / 4;
+        place[t.y[k]] = (int)k;
+        uint4 &q = of[(st / 2) * 16 + 4 * (k % 4) + b];
+        (st % 2 ? q.y : q.x) = ofs[t.y[k]];
+      }
+      for (size_t q = t.e0; q < t.e1; ++q) {
+        const int k = place[T[q].y];
+        v[(s0 + k / 4) * 64 + 16 * (k % 4) + 4 * b + T[q].x - t.x0] += T[q].v;
+      }
+    }
+    s0 += 2 * (size_t)pairs[g / 4];
+  }
 }
 
 extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *inter,
@@ -2893,25 +3186,6 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
       mt[2 * h + a] = j * (j + 1);
     }
     if ((r = dupload(c, &c->d_mtab, mt.data(), mt.size()))) return bail(r, c->err);
-    // per species and element (a, b) of rho, e = a + b h: t1(b, a), m_a m_b,
-    // c_a c_b (0 unless a, b > 0), d_ab, m_a d_ab, j_a(j_a+1) d_ab,
-    // c_a d_{a,b+1}, c_b d_{b,a+1} (the kinetic energy and <J^2> loop of k_fac_phi)
-    std::vector<double> jt(2 * (size_t)h * h * 8, 0.0);
-    for (int sp = 0; sp < 2; ++sp)
-      for (int b = 0; b < h; ++b)
-        for (int a = 0; a < h; ++a) {
-          double *q = jt.data() + ((size_t)sp * h * h + a + (size_t)b * h) * 8;
-          const double ma = mt[a], mb = mt[b], ca = mt[h + a], cb = mt[h + b];
-          q[0] = inter->t1b[(size_t)(sp * h + b) + (size_t)(sp * h + a) * n];
-          q[1] = ma * mb;
-          q[2] = (a > 0 && b > 0) ? ca * cb : 0.0;
-          q[3] = (a == b) ? 1.0 : 0.0;
-          q[4] = (a == b) ? ma : 0.0;
-          q[5] = (a == b) ? mt[2 * h + a] : 0.0;
-          q[6] = (a == b + 1) ? ca : 0.0;
-          q[7] = (b == a + 1) ? cb : 0.0;
-        }
-    if ((r = dupload(c, &c->d_jtab, jt.data(), jt.size()))) return bail(r, c->err);
   }
   if ((r = dupload(c, &c->d_pk_a, pa.data(), pa.size())) || (r = dupload(c, &c->d_pk_b, pb.data(), pb.size())) ||
       (r = dupload(c, &c->d_blk_off, off.data(), h)) || (r = dupload(c, &c->d_blk_sz, sz.data(), h)) ||
@@ -2999,37 +3273,42 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
       }
     }
     for (int k = 0; k < 3; ++k) c->nme_s[k] = (int)ls[k].size();
-    // pp and nn lists for k_fac_phi: one term per entry, the (kl)(ij) partner
-    // of an entry with a + b != c + d as an entry of its own, LDS byte
-    // offsets precomputed (rho at ld h + 1, then the A-block at ld h)
-    for (int k = 0; k < 2; ++k) {
-      std::vector<uint4> lo, lw;
-      const unsigned hp = h + 1, msz = h * (h + 1);
-      auto rb = [&](int row, int col) { return (unsigned)(row + col * hp) * 16u; };
-      auto ab = [&](int row, int col) { return (msz + (unsigned)(row + col * h)) * 16u; };
-      auto term = [&](int i, int j, int kk, int l, double me) {
-        uint64_t mb;
-        std::memcpy(&mb, &me, 8);
-        lo.push_back(make_uint4(rb(kk, i), rb(l, j), rb(l, i), rb(kk, j)));
-        lw.push_back(make_uint4(ab(i, j), ab(l, kk), (unsigned)mb, (unsigned)(mb >> 32)));
-      };
-      for (const VEntry &e : ls[k]) {
-        const int i = e.idx & 255, j = (e.idx >> 8) & 255, kk = (e.idx >> 16) & 255, l = e.idx >> 24;
-        if (!(i < j && kk < l)) {  // a = b or c = d: the A-block holds index pairs in increasing order only
-          c->fac_list_ok = false;
-          c->fac_reason = "factored and mixed forms need list entries with a != b and c != d";
-          break;
+    // pp and nn lists for k_fac_dens as bilinear forms, x = row + column h of a
+    // species block: V [rho_ki rho_lj - rho_li rho_kj] + V A01_ij A10_kl / 4 (the
+    // A-blocks hold A01 in the upper and A10 / 4 in the lower triangle), the
+    // (kl)(ij) partner of an entry with a + b != c + d as an entry of its own
+    {
+      std::vector<double> buf;
+      std::vector<unsigned> rb(h * h), ab(h * h);
+      for (int x = 0; x < h * h; ++x) {
+        rb[x] = (unsigned)(x % h + x / h * (h + 1)) * 16u;
+        ab[x] = (unsigned)x * 16u;
+      }
+      for (int k = 0; k < 2; ++k) {
+        std::vector<BilTerm> cr, ck;
+        auto term = [&](int i, int j, int kk, int l, double me) {
+          cr.push_back({kk + i * h, l + j * h, me});
+          cr.push_back({l + i * h, kk + j * h, -me});
+          ck.push_back({i + j * h, l + kk * h, me});
+        };
+        for (const VEntry &e : ls[k]) {
+          const int i = e.idx & 255, j = (e.idx >> 8) & 255, kk = (e.idx >> 16) & 255, l = e.idx >> 24;
+          if (!(i < j && kk < l)) {  // a = b or c = d: the A-block holds index pairs in increasing order only
+            c->fac_list_ok = false;
+            c->fac_reason = "factored and mixed forms need list entries with a != b and c != d";
+            break;
+          }
+          term(i, j, kk, l, e.me);
+          if (kk + l != i + j) term(kk, l, i, j, e.me);
         }
-        term(i, j, kk, l, e.me);
-        if (kk + l != i + j) term(kk, l, i, j, e.me);
+        bil_table(buf, c->frho[k], h * h, true, cr, rb);
+        bil_table(buf, c->fkap[k], h * h, false, ck, ab);
       }
-      while (lo.size() % 256) {  // zero terms (offset 0, matrix element 0)
-        lo.push_back(make_uint4(0u, 0u, 0u, 0u));
-        lw.push_back(make_uint4(0u, 0u, 0u, 0u));
+      if ((r = dupload(c, &c->d_bil, buf.data(), buf.size()))) return bail(r, c->err);
+      for (BilForm *f : {&c->frho[0], &c->frho[1], &c->fkap[0], &c->fkap[1]}) {
+        f->v = c->d_bil + (size_t)f->v;
+        f->ofs = (const uint4 *)(c->d_bil + (size_t)f->ofs);
       }
-      c->nl[k] = (int)lo.size();
-      lo.insert(lo.end(), lw.begin(), lw.end());
-      if ((r = dupload(c, &c->d_lofs[k], lo.data(), lo.size()))) return bail(r, c->err);
     }
     // W_pn by rows x = c + a h, columns y = d + b h (species-local indices)
     const int hh = h * h;
@@ -3578,9 +3857,8 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     fp.binv = c->d_binv; fp.pfb = c->d_pfb;
     const bool pfs = c->schur_allowed && c->pfs_any, both = pfs && !c->pfs_all && c->tune.pf_waves == 0;
     fp.pfs_ok = both ? c->d_pfs_ok : nullptr;
-    fp.jtab = (const double2 *)c->d_jtab;
     for (int q = 0; q < 2; ++q) {
-      fp.lofs[q] = c->d_lofs[q]; fp.nl[q] = c->nl[q];
+      fp.frho[q] = c->frho[q]; fp.fkap[q] = c->fkap[q];
     }
     fp.out = c->d_fout; fp.rho = c->d_frho; fp.status = c->d_fstatus;
     for (int q = 0; q < 2; ++q) {
@@ -3637,10 +3915,8 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
         cp.zres = c->d_zres + (size_t)p0 * c->NE * NOBS;
         cp.status = c->d_status + (size_t)p0 * c->NE;
         if (direct) cp.samples = samples + (size_t)p0 * c->NE * c->nphi * c->nphi * 2;
-        const size_t nwg = (size_t)np * nec * 2 * nd;
-        fp.nwg = (int)nwg;
         hipLaunchKernelGGL(k_fac_setup, dim3(nec, np, 2), dim3(NTS), setup_lds, c->stream, sp);
-        launch_phi_h(h, mix, c->tune, pfs ? (both ? 2 : 1) : 0, (unsigned)((nwg + 7) / 8 * 8), c->stream, fp);
+        launch_phi_h(h, mix, c->tune, pfs ? (both ? 2 : 1) : 0, (size_t)np * nec * 2, c->stream, fp);
         if (mix != MIX_FP64) {
           const int ncols = (int)(cols_pp * np);
           for (int q = 0; q < NVPROB; ++q) vp.prob[q].ncols = ncols;
@@ -4190,7 +4466,7 @@ extern "C" int pnamp_autotune(pnamp_ctx *c, int npairs, const int32_t *q0, const
   if (!c || npairs <= 0 || !q0 || !q1) return PNAMP_E_ARG;
   if (c->form != PNAMP_FORM_FACTORED) return fail(c, PNAMP_E_ARG, "autotune: the FP64 factored form only");
   struct Cand {
-    int pf, rest, div;
+    int pf, div;
   };
   std::vector<Cand> cands;
   const int h = c->h;
@@ -4200,16 +4476,14 @@ extern "C" int pnamp_autotune(pnamp_ctx *c, int npairs, const int32_t *q0, const
   std::vector<int> pfs;
   if (schur) pfs.push_back(0);
   if (h >= 8) pfs.insert(pfs.end(), {3, 4, 5});
-  for (int pf : pfs)
-    for (int rest : {0, 4}) {
-      if (rest == 4 && (h > 16 || h < 8)) continue;
-      FacTune t;
-      t.pf_waves = pf;
-      t.rest_waves = rest;
-      if (phi_scratch_h(h, t, schur) != 0) continue;  // a variant that spills registers is no candidate
-      for (int div : {1, 2, 4}) cands.push_back({pf, rest, div});
-    }
-  if (cands.empty()) cands.push_back({0, 0, 1});
+  for (int pf : pfs) {
+    FacTune t;
+    t.pf_waves = pf;
+    if (phi_scratch_h(h, t, schur) != 0) continue;  // a variant that spills registers is no candidate
+    for (int div : {1, 2, 4}) cands.push_back({pf, div});
+  }
+  if (cands.empty()) cands.push_back({0, 1});
+  const int rest = 3 * h <= 64 ? 3 : 2;  // the densities' waves as reported
   const int pf_dflt = schur ? 0 : pf_default_waves(h);
   if ((int)cands.size() > PNAMP_TUNE_MAX) return fail(c, PNAMP_E_SIZE, "autotune: too many candidates");
   const FacTune keep = c->tune;
@@ -4217,7 +4491,6 @@ extern "C" int pnamp_autotune(pnamp_ctx *c, int npairs, const int32_t *q0, const
   int ib = -1;
   for (size_t i = 0; i < cands.size(); ++i) {
     c->tune.pf_waves = cands[i].pf;
-    c->tune.rest_waves = cands[i].rest;
     c->tune.chunk_div = cands[i].div;
     drop_graph(c);
     int r = kernels_impl(c, npairs, q0, q1, zval, nval, nullptr, nullptr, nullptr);  // captures
@@ -4230,7 +4503,7 @@ extern "C" int pnamp_autotune(pnamp_ctx *c, int npairs, const int32_t *q0, const
     if (ms) ms[i] = c->ms_points;
     if (cand) {
       cand[3 * i] = cands[i].pf ? cands[i].pf : pf_dflt;
-      cand[3 * i + 1] = cands[i].rest ? cands[i].rest : (3 * h <= 64 ? 3 : 2);
+      cand[3 * i + 1] = rest;
       cand[3 * i + 2] = cands[i].div;
     }
     if (ib < 0 || c->ms_points < best) {
@@ -4239,12 +4512,11 @@ extern "C" int pnamp_autotune(pnamp_ctx *c, int npairs, const int32_t *q0, const
     }
   }
   c->tune.pf_waves = cands[ib].pf;
-  c->tune.rest_waves = cands[ib].rest;
   c->tune.chunk_div = cands[ib].div;
   drop_graph(c);
   if (choice) {
     choice[0] = cands[ib].pf ? cands[ib].pf : pf_dflt;
-    choice[1] = cands[ib].rest ? cands[ib].rest : (3 * h <= 64 ? 3 : 2);  // the default
+    choice[1] = rest;
     choice[2] = cands[ib].div;
   }
   if (ncand) *ncand = (int)cands.size();
@@ -4269,7 +4541,6 @@ extern "C" int pnamp_set_tune(pnamp_ctx *c, int pf_waves, int rest_waves, int ch
       (chunk_div != 1 && chunk_div != 2 && chunk_div != 4))
     return fail(c, PNAMP_E_ARG, "pnamp_set_tune: waves 3, 4, 5 (Pfaffian), 2, 3, 4 (densities), chunk divisor 1, 2, 4");
   c->tune.pf_waves = pf_waves;                                      // 0: the default for h
-  c->tune.rest_waves = (rest_waves == 4 && c->h <= 16) ? 4 : 0;     // 2 and 3 name the default
   c->tune.chunk_div = chunk_div;
   drop_graph(c);
   return PNAMP_OK;
@@ -4292,9 +4563,9 @@ extern "C" void pnamp_destroy(pnamp_ctx *c) {
   drop_graph(c);
   void *bufs[] = {c->d_alp, c->d_walp, c->d_bet, c->d_wbet, c->d_gam, c->d_wgam, c->d_rtab, c->d_ptab,
                   c->d_pk_a, c->d_pk_b, c->d_blk_off, c->d_blk_sz, c->d_blk_base, c->d_twoj, c->d_twom,
-                  c->d_plofs, c->d_plme, c->d_pwork, c->d_t1b, c->d_jtab, c->d_U, c->d_V, c->d_Z, c->d_det, c->d_state_status, c->d_q0,
+                  c->d_plofs, c->d_plme, c->d_pwork, c->d_t1b, c->d_U, c->d_V, c->d_Z, c->d_det, c->d_state_status, c->d_q0,
                   c->d_q1, c->d_pz, c->d_pn, c->d_zres, c->d_kern, c->d_status, c->d_pair_status,
-                  c->d_lofs[0], c->d_lofs[1], c->d_Uf, c->d_Vf, c->d_binv, c->d_pfb, c->d_pfs_ok,
+                  c->d_bil, c->d_Uf, c->d_Vf, c->d_binv, c->d_pfb, c->d_pfs_ok,
                   c->d_UfT, c->d_VfT, c->d_mtab, c->d_fout, c->d_frho,
                   c->d_sbuf, c->d_fstatus, c->d_pn_rows,
                   c->d_pn_blk, c->d_pn_ycol, c->d_pn_w, c->d_ecan, c->d_gcls, c->d_gmap};
