@@ -2094,76 +2094,90 @@ __global__ __launch_bounds__(256) void k_project(ProjParams p) {
 // (per K2), then the alpha sum (per K1, K2), then the d^J_{K1K2}(beta) term,
 // (2J+1) / (8 pi^2) sum_abg w_a w_b w_g e^{iK1 a} d^J_{K1K2}(b) e^{iK2 g} ZRES
 // in nbet (ngam + nalp (2jmax+1)) (2jmax+1) + nbet npj complex products
-// instead of nalp nbet ngam npj.  Up to PROJ_MAXO outputs per thread.
-constexpr int PROJ_MAXO = 16;
-__global__ __launch_bounds__(256) void k_project_sep(ProjParams p) {
+// instead of nalp nbet ngam npj.  Bound by latency (one workgroup per pair and
+// observable): nb beta nodes, as many as 48 KB of LDS hold, go through the
+// three sums together, so their loads and barriers are waited for once, and a
+// thread keeps its own (J, K1, K2) of the npj outputs.  One node at a time by 256
+// threads, their weights and d read in the inner loops, took 35 us for one sd
+// pair on 10 nodes (now 8) and 155 us for 15 pairs on 20 nodes of 10 x 10 at jmax
+// 8 (now 34).
+constexpr int NTP = 1024, PROJ_MAXO = 2;  // threads, outputs per thread
+__global__ __launch_bounds__(NTP) void k_project_sep(ProjParams p, int nb) {
   extern __shared__ double2 ktab[];
   const int ip = blockIdx.x, io = blockIdx.y, tid = threadIdx.x;
   const int J2m = 2 * p.jmax + 1, na = p.nalp, ng = p.ngam;
-  double2 *ea = ktab, *eg = ea + (size_t)J2m * na, *zb = eg + (size_t)J2m * ng, *zg = zb + (size_t)na * ng,
-          *zag = zg + (size_t)na * J2m;
-  for (int i = tid; i < J2m * na; i += blockDim.x) ea[i] = cexpi((i / na - p.jmax) * p.alp[i % na]);
-  for (int i = tid; i < J2m * ng; i += blockDim.x) eg[i] = cexpi((i / ng - p.jmax) * p.gam[i % ng]);
+  double2 *ea = ktab, *eg = ea + (size_t)J2m * na, *zb = eg + (size_t)J2m * ng, *zg = zb + (size_t)nb * na * ng,
+          *zag = zg + (size_t)nb * na * J2m;
+  // the phases times the nodes' weights
+  for (int i = tid; i < J2m * (na + ng); i += NTP) {
+    const bool ia = i < J2m * na;
+    const int r = ia ? i : i - J2m * na, k = r / (ia ? na : ng) - p.jmax, x = r % (ia ? na : ng);
+    ktab[i] = cscale((ia ? p.walp : p.wgam)[x], cexpi(k * (ia ? p.alp : p.gam)[x]));
+  }
   const double2 *z = p.zres + (size_t)ip * p.NE * p.nobs;
   double2 *kout = p.kern + ((size_t)ip * p.nobs + io) * (p.jmax + 1) * J2m * J2m;
-  const int ntot = (p.jmax + 1) * J2m * J2m;
+  int zo[PROJ_MAXO], J[PROJ_MAXO];
   double2 acc[PROJ_MAXO];
 #pragma unroll
-  for (int m = 0; m < PROJ_MAXO; ++m) acc[m] = cz();
-  for (int ib = 0; ib < p.nbet; ++ib) {
+  for (int m = 0; m < PROJ_MAXO; ++m) {
+    const int e = min(tid + m * NTP, p.npj - 1);
+    int j = 0;
+    while ((j + 1) * (4 * (j + 1) * (j + 1) - 1) / 3 <= e) ++j;
+    const int r = e - j * (4 * j * j - 1) / 3;
+    J[m] = j;
+    zo[m] = (r / (2 * j + 1) - j + p.jmax) * J2m + r % (2 * j + 1) - j + p.jmax;
+    acc[m] = cz();
+  }
+  for (int b0 = 0; b0 < p.nbet; b0 += nb) {
+    const int n = min(nb, p.nbet - b0);
+    for (int i = tid; i < n * na * ng; i += NTP) zb[i] = z[((size_t)b0 * na * ng + i) * p.nobs + io];
     __syncthreads();
-    for (int i = tid; i < na * ng; i += blockDim.x) zb[i] = z[((size_t)ib * na * ng + i) * p.nobs + io];
-    __syncthreads();
-    for (int i = tid; i < na * J2m; i += blockDim.x) {
-      const int a = i / J2m, k2 = i % J2m;
+    for (int i = tid; i < n * na * J2m; i += NTP) {
+      const int ab = i / J2m, k2 = i % J2m;
       double2 sacc = cz();
-      for (int g = 0; g < ng; ++g) cfma(sacc, cscale(p.wgam[g], eg[k2 * ng + g]), zb[a * ng + g]);
+      for (int g = 0; g < ng; ++g) cfma(sacc, eg[k2 * ng + g], zb[ab * ng + g]);
       zg[i] = sacc;
     }
     __syncthreads();
-    for (int i = tid; i < J2m * J2m; i += blockDim.x) {
-      const int k1 = i / J2m, k2 = i % J2m;
+    for (int i = tid; i < n * J2m * J2m; i += NTP) {
+      const int b = i / (J2m * J2m), k1 = i / J2m % J2m, k2 = i % J2m;
       double2 sacc = cz();
-      for (int a = 0; a < na; ++a) cfma(sacc, cscale(p.walp[a], ea[k1 * na + a]), zg[a * J2m + k2]);
+      for (int a = 0; a < na; ++a) cfma(sacc, ea[k1 * na + a], zg[(b * na + a) * J2m + k2]);
       zag[i] = sacc;
     }
     __syncthreads();
-    const double wb = p.wbet[ib];
 #pragma unroll
     for (int m = 0; m < PROJ_MAXO; ++m) {
-      const int o = tid + m * (int)blockDim.x;
-      if (o >= ntot) break;
-      const int J = o / (J2m * J2m), K1 = (o / J2m) % J2m - p.jmax, K2 = o % J2m - p.jmax;
-      if (K1 < -J || K1 > J || K2 < -J || K2 > J) continue;
-      const int e = J * (4 * J * J - 1) / 3 + (K1 + J) * (2 * J + 1) + (K2 + J);
-      const double dp = p.ptab[((size_t)ib * 2 + 0) * p.npj + e];
-      acc[m] = cadd(acc[m], cscale(wb * dp, zag[(K1 + p.jmax) * J2m + (K2 + p.jmax)]));
+      const int e = tid + m * NTP;
+      if (e >= p.npj) break;
+#pragma unroll 4
+      for (int b = 0; b < n; ++b)
+        acc[m] = cadd(acc[m], cscale(p.wbet[b0 + b] * p.ptab[(size_t)(b0 + b) * 2 * p.npj + e], zag[b * J2m * J2m + zo[m]]));
     }
   }
   const bool onept = (na * ng == 1);
 #pragma unroll
   for (int m = 0; m < PROJ_MAXO; ++m) {
-    const int o = tid + m * (int)blockDim.x;
-    if (o >= ntot) break;
-    const int J = o / (J2m * J2m);
-    const double wJ = onept ? (2.0 * J + 1.0) / 2.0 : (2.0 * J + 1.0) / (8.0 * M_PI * M_PI);
-    kout[o] = cscale(wJ, acc[m]);
+    if (tid + m * NTP >= p.npj) break;
+    const double wJ = onept ? (2.0 * J[m] + 1.0) / 2.0 : (2.0 * J[m] + 1.0) / (8.0 * M_PI * M_PI);
+    kout[J[m] * J2m * J2m + zo[m]] = cscale(wJ, acc[m]);
+  }
+  for (int o = tid; o < (p.jmax + 1) * J2m * J2m; o += NTP) {  // |K| > J
+    const int j = o / (J2m * J2m), k1 = o / J2m % J2m - p.jmax, k2 = o % J2m - p.jmax;
+    if (max(abs(k1), abs(k2)) > j) kout[o] = cz();
   }
   if (io == 0) {
-    __shared__ int st[256];
+    __shared__ int st[4];
     int sv = 0;
-    for (int i = tid; i < p.NE; i += blockDim.x) {
+    for (int i = tid; i < p.NE && tid < 256; i += 256) {
       const int v = p.status[(size_t)ip * p.NE + i];
       if (v && !sv) sv = v;
     }
-    st[tid] = sv;
+    // of the first 256 threads' statuses the first that is not zero
+    const unsigned long long any = __ballot(sv != 0);
+    if (tid < 256 && (tid & 63) == (any ? __ffsll(any) - 1 : 0)) st[tid >> 6] = sv;
     __syncthreads();
-    if (tid == 0) {
-      int r = 0;
-      for (int i = 0; i < (int)blockDim.x; ++i)
-        if (st[i]) { r = st[i]; break; }
-      p.pair_status[ip] = r;
-    }
+    if (tid == 0) p.pair_status[ip] = st[0] ? st[0] : (st[1] ? st[1] : (st[2] ? st[2] : st[3]));
   }
 }
 
@@ -3681,14 +3695,17 @@ extern "C" int pnamp_state_overlaps(pnamp_ctx *c, double *det) {
 
 static hipError_t launch_project(pnamp_ctx *c, int npairs, const ProjParams &pr) {
   const size_t J2m = 2 * (size_t)c->jmax + 1;
-  if (c->fold == PNAMP_FOLD_PLAIN && (size_t)(c->jmax + 1) * J2m * J2m <= 256 * (size_t)PROJ_MAXO) {
-    const size_t lds = sizeof(double2) * (J2m * (c->nalp + c->ngam) + (size_t)c->nalp * c->ngam +
-                                          (size_t)c->nalp * J2m + J2m * J2m);
+  if (c->fold == PNAMP_FOLD_PLAIN && (c->jmax + 1) * J2m * J2m <= 4096) {  // (jmax <= 9: npj <= 1330)
+    const size_t tab = sizeof(double2) * J2m * (c->nalp + c->ngam),
+                 per = sizeof(double2) * ((size_t)c->nalp * c->ngam + (size_t)c->nalp * J2m + J2m * J2m);
+    const size_t fit = tab + per < 48 * 1024 ? (48 * 1024 - tab) / per : 1;
+    const int nb = (int)std::min<size_t>(fit, c->nbet);
+    const size_t lds = tab + nb * per;
     if (lds > 48 * 1024) {
       const hipError_t e = hipFuncSetAttribute((const void *)k_project_sep, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_project_sep, dim3(npairs, pr.nobs), dim3(256), lds, c->stream, pr);
+    hipLaunchKernelGGL(k_project_sep, dim3(npairs, pr.nobs), dim3(NTP), lds, c->stream, pr, nb);
     return hipGetLastError();
   }
   const size_t lds = sizeof(double2) * (2 * (size_t)c->jmax + 1) * (c->nalp + c->ngam);
