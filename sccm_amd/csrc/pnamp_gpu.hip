@@ -233,8 +233,7 @@ struct VEntry {
 //   k_fac_combine  one workgroup per (pair, Euler point): the p-n bilinear form
 //                  and the nphi^2 gauge sum.
 constexpr int NTS = 256;     // threads of the setup workgroup
-constexpr int NTC = 512;     // threads of the combine workgroup: one G row per thread (h^2 <= 484),
-                              // so the longest row (pf: 60 entries) bounds the pass; eight waves
+constexpr int NTC = 512;     // threads of the combine workgroup: eight waves, two workgroups per CU
 constexpr int NPHI_MAX = 16;
 constexpr int FAC_OUT = 9;   // per (pair, Euler, species, phi): Pf, E2, Ekin, Tr rho, A, t_+, t_-, t_z, E2 (kappa part, mixed forms)
 constexpr int MIX_FP64 = 0, MIX_FP32 = 1, MIX_BF16 = 2;  // precision of the V contraction
@@ -362,7 +361,7 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
 struct BilForm {
   const double *v;   // [2 pairs][64]: A of lane 16 k + 4 b + i = C(row i of tile b, column k of the step)
   const uint4 *ofs;  // [pairs][16], LDS byte offsets, entry 4 k + b: column k of tile b in both steps of the
-                     // pair, row k of tile b, and 1 in the last pair of a group
+                     // pair, row k of tile b (in every pair of a group), and 1 in a group's last pair
   int np;            // pairs of steps, a multiple of BIL_RING (BIL_RING more, all zero, follow)
 };
 constexpr int BIL_RING = 8;
@@ -1171,13 +1170,11 @@ struct CombParams {
   const double *det;
   const int *q0, *q1;
   const int *pz, *pn;               // valence numbers per pair, or NULL
-  // W_pn (rows x = c + a h, columns y = d + b h) in dense blocks of equal
-  // Delta m = m_c - m_a = -(m_d - m_b): the interaction conserves M
-  const int2 *pn_rows;              // [h^2] by block order: (x, block)
-  const int *pn_blk;                // [nblk][5]: first row position, rows, first column (in pn_ycol), columns, offset in pn_w
-  const int *pn_ycol;               // [h^2] column lists of the blocks
-  const double *pn_w;               // blocks, column-major
-  int pn_ncol;                      // length of pn_ycol
+  // W_pn as a bilinear form, rows x = c + a h (offsets 16 x in rho_p), columns y =
+  // d + b h (16 y in rho_n)
+  BilForm wpn;
+  const int2 *pn_grp;               // its groups: first pair, pairs (even)
+  int pn_ng;
   const double2 *out, *rho;
   const int *fstatus;               // [npairs][NE][2][nphi]
   const float2 *gpn;                // mixed forms: G = W_pn rho_n from k_vgemm, [npairs][NE][nphi][h*h]
@@ -1191,29 +1188,42 @@ struct CombParams {
 // W[(c,a),(d,b)] = V_abcd and W[(a,c),(b,d)] += V_abcd for list entries with
 // a + b != c + d (for a, c protons and b, d neutrons the eight-term sum of
 // HFB_Energy_COMPLEX reduces to V [rho_p(c,a) rho_n(d,b) + rho_p(a,c) rho_n(b,d)]).
-// G = W rho_n(phi_n) is formed once per phi_n from the dense Delta-m blocks of W, then
-// the nphi^2 dot products with rho_p(phi_p); the gauge points are summed into
-// ZRES.  NP = nd (the gauge angles evaluated) is a template argument so the
-// per-gauge register arrays stay in registers; the dot products also take
-// rho_p* G (four real sums, the same multiply-adds), for the gauge pairs of
-// which one angle is a conjugate.  With GMIX (mixed forms) G comes from k_vgemm instead.
+// Its groups of four row tiles are dealt to the eight waves: G = W rho_n of all
+// phi_n by v_mfma_f64_4x4x4_4b with rho_n in LDS (columns: phi_n, re / im), and the
+// 16 rows of G in D layout are at once the B operand of the products with
+// rho_p(phi_p), whose four real parts (re / im by re / im) per gauge pair stay in
+// registers over the groups: rho_p^T G, and rho_p^+ G for the gauge pairs of which
+// one angle is a conjugate.  NP = nd (the gauge angles evaluated) is a template
+// argument so these stay in registers.  Then the gauge points are summed into
+// ZRES.  With GMIX (mixed forms) G comes from k_vgemm and the dot products are
+// taken from LDS.
+//
+// One row of G per thread with broadcast reads of rho_n from LDS was bound by
+// those reads, and the gauge sum by loads one after the other (outputs, 2 NP
+// statuses); now by the latency of the phases at the two workgroups per CU
+// that the LDS allows (rho_n in, products, gauge sum).  15 pf pairs at 1000 Euler
+// points, NP = 9: 1270 -> 973 us (the products alone 160 us at the FP64 rate);
+// f5pg9, NP = 4: 820 -> 675 us; sd, NP = 7: 368 -> 265 us.
 template <int NP, bool GMIX>
 // (up to nine gauge angles four waves per SIMD: two eight-wave workgroups per
 // CU, as many as their LDS allows; more angles need more than 128 VGPRs)
 __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4 : 2))) void k_fac_combine(CombParams p) {
-  extern __shared__ double2 dsm[];  // rho_n -> G [NP][h^2], then the block column lists; rho_p from global memory
+  extern __shared__ double2 dsm[];  // rho_n or G [NP][ldf], then the partial sums of the products; rho_p from global memory
   __shared__ double2 epn[NP * NP], epc[NP * NP];  // rho_p^T G, rho_p^+ G
   __shared__ double red[(NTC + 63) / 64 * 2 * NOBS];
+  __shared__ double2 so[2 * NP * FAC_OUT];  // the species outputs
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int iang = blockIdx.x, ip = blockIdx.y;
   const int h = p.h, hh = h * h;
   const size_t base = ((size_t)ip * p.NE + iang) * 2;
   double2 *rn = dsm;
-  int *ycol = (int *)(dsm + (size_t)NP * hh);
+  // the outputs and statuses of the gauge sum are loaded first, with rho_n
+  const int fst = (tid < 2 * NP) ? p.fstatus[base * NP + tid] : 0;
+  for (int e = tid; e < 2 * NP * FAC_OUT; e += NTC) so[e] = p.out[base * NP * FAC_OUT + e];
+  const int ldf = GMIX ? hh : hh + 1;  // (h^2 + 1: two angles' elements in different banks)
   // rho_n (or G) into LDS: every load of a thread issued before the first
   // store (indices clamped, no load in a branch), so the HBM latency is
   // paid once per thread rather than once per element
-  for (int e = tid; e < p.pn_ncol; e += NTC) ycol[e] = p.pn_ycol[e];
   {
     constexpr int NB = 8;  // loads in flight per thread (the register cap is 128)
     const int nt = NP * hh;
@@ -1233,64 +1243,95 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
       // again with its own value (a store in a branch would pull its load
       // into the branch and wait on it there)
 #pragma unroll
-      for (int u = 0; u < NB; ++u) rn[min(e0 + tid + NTC * u, nt - 1)] = tmp[u];
-    }
-  }
-  __syncthreads();
-  if (!GMIX) {
-  // G rows in block order (row position tid + r NTC), all phi_n, in
-  // registers.  The lanes of one block walk the same column list, so each
-  // rho_n read is an LDS broadcast.
-  constexpr int RPT = (FAC_HMAX * FAC_HMAX + NTC - 1) / NTC;
-  double2 g[RPT][NP];
-  int xrow[RPT];
-#pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-#pragma unroll
-    for (int f = 0; f < NP; ++f) g[r][f] = cz();
-    const int px = tid + r * NTC;
-    xrow[r] = -1;
-    if (px < hh) {
-      const int2 rw = p.pn_rows[px];
-      const int *bk = p.pn_blk + 5 * rw.y;
-      const int nrows = bk[1], ncol = bk[3];
-      const int *yc = ycol + bk[2];
-      const double *wb = p.pn_w + bk[4] + (px - bk[0]);
-      xrow[r] = rw.x;
-      // four block entries per group, the next group's loads issued before
-      // this group's products (indices clamped to the last entry, weight 0
-      // past it)
-      double v0 = wb[0], v1 = wb[(size_t)min(1, ncol - 1) * nrows], v2 = wb[(size_t)min(2, ncol - 1) * nrows],
-             v3 = wb[(size_t)min(3, ncol - 1) * nrows];
-      for (int k = 0; k < ncol; k += 4) {
-        const double c0 = v0, c1 = v1, c2 = v2, c3 = v3;
-        v0 = wb[(size_t)min(k + 4, ncol - 1) * nrows];
-        v1 = wb[(size_t)min(k + 5, ncol - 1) * nrows];
-        v2 = wb[(size_t)min(k + 6, ncol - 1) * nrows];
-        v3 = wb[(size_t)min(k + 7, ncol - 1) * nrows];
-        const double cv[4] = {c0, c1, c2, c3};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const bool ok = k + u < ncol;
-          const int y = yc[ok ? k + u : 0];
-          const double vv = ok ? cv[u] : 0.0;
-#pragma unroll
-          for (int f = 0; f < NP; ++f) rfma(g[r][f], vv, rn[(size_t)f * hh + y]);
-        }
+      for (int u = 0; u < NB; ++u) {
+        const int e = min(e0 + tid + NTC * u, nt - 1);
+        rn[GMIX ? e : e + e / hh] = tmp[u];
       }
     }
   }
   __syncthreads();
+  if constexpr (!GMIX) {
+    constexpr int NC = (NP + 1) / 2, NW = NTC / 64;
+    auto mac = [](double a, double b, double d) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, d, 0, 0, 0); };
+    // lane (li, b, k): column li of B, row li of A: angle 2 c + li / 2 (the last
+    // repeated past NP), re / im
+    int bv[NC], av[NC];
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int x = xrow[r];
-    if (x >= 0) {
-#pragma unroll
-      for (int f = 0; f < NP; ++f) rn[(size_t)f * hh + x] = g[r][f];
+    for (int c = 0; c < NC; ++c) {
+      const int f = min(2 * c + ((lane >> 1) & 1), NP - 1);
+      bv[c] = f * ldf * 16 + (lane & 1) * 8;
+      av[c] = f * hh * 16 + (lane & 1) * 8;
     }
-  }
-  __syncthreads();
-  }
+    const char *const lds = (const char *)dsm, *const rp = (const char *)(p.rho + base * NP * hh);
+    double e[NC][NC];
+#pragma unroll
+    for (int i = 0; i < NC * NC; ++i) e[i / NC][i % NC] = 0.0;
+    const auto groups = ro_const((const int *)p.pn_grp);
+    for (int g = __builtin_amdgcn_readfirstlane(wave); g < p.pn_ng; g += NW) {
+      const size_t q0 = groups[2 * g];
+      const int nq = groups[2 * g + 1];
+      const double *vp = p.wpn.v + q0 * 128 + lane;
+      const uint4 *cp = p.wpn.ofs + q0 * 16 + (lane >> 2);
+      uint4 o[2] = {cp[0], cp[16]};
+      double v[2][2] = {{vp[0], vp[64]}, {vp[128], vp[192]}};
+      double a[NC], d[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        a[c] = *(const double *)(rp + av[c] + o[0].z);
+        d[c] = 0.0;
+      }
+#pragma unroll 1
+      for (int q = 0; q < nq; q += 2) {
+        vp += 256;
+        cp += 32;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          double b[NC];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) b[c] = *(const double *)(lds + bv[c] + o[u].x);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) d[c] = mac(v[u][0], b[c], d[c]);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) b[c] = *(const double *)(lds + bv[c] + o[u].y);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) d[c] = mac(v[u][1], b[c], d[c]);
+          o[u] = cp[16 * u];  // (two pairs past the last group's are zeros)
+          v[u][0] = vp[128 * u];
+          v[u][1] = vp[128 * u + 64];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) e[i][c] = mac(a[i], d[c], e[i][c]);
+    }
+    // sums over the four blocks (lanes 4 b in a row of 16), then over the waves
+    __syncthreads();
+    double *const part = (double *)dsm;  // [wave][NC][NC][4 i + j]
+#pragma unroll
+    for (int i = 0; i < NC * NC; ++i) {
+      double x = e[i / NC][i % NC];
+      x += __shfl_xor(x, 4);
+      x += __shfl_xor(x, 8);
+      if ((lane & 12) == 0) part[(wave * NC * NC + i) * 16 + (lane >> 4) * 4 + (lane & 3)] = x;
+    }
+    __syncthreads();
+    for (int t = tid; t < NP * NP; t += NTC) {
+      const int fp = t / NP, fn = t % NP;
+      const double *q = part + ((fp / 2) * NC + fn / 2) * 16 + (fp % 2) * 8 + (fn % 2) * 2;
+      double rr = 0.0, ri = 0.0, ir = 0.0, ii = 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const double *x = q + w * NC * NC * 16;
+        rr += x[0];
+        ri += x[1];
+        ir += x[4];
+        ii += x[5];
+      }
+      epn[t] = make_double2(rr - ii, ri + ir);
+      epc[t] = make_double2(rr + ii, ri - ir);
+    }
+  } else {
   const int grp = tid >> 5, gl = tid & 31;
   for (int fp = grp; fp < NP; fp += NTC / 32) {
     double2 acc[NP], acq[NP];  // (re re, im im), (re im, im re)
@@ -1335,8 +1376,9 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
       }
     }
   }
+  }
   __syncthreads();
-  const double2 *op = p.out + base * NP * FAC_OUT, *on = p.out + (base + 1) * NP * FAC_OUT;
+  const double2 *op = so, *on = so + NP * FAC_OUT;
   const double vac = p.snpfaf * p.sgn_h * (p.det[p.q0[ip]] * p.vac_scale) * (p.det[p.q1[ip]] * p.vac_scale);
   double v[2 * NOBS] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   const int nphi = p.nphi;
@@ -1386,22 +1428,20 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
   if (lane == 0)
     for (int k = 0; k < 2 * NOBS; ++k) red[wave * 2 * NOBS + k] = v[k];
   __syncthreads();
-  if (tid == 0) {
-    const double inv = 1.0 / (double)(nphi * nphi);
-    double2 *z = p.zres + ((size_t)ip * p.nefull + en.x) * NOBS;
-    for (int k = 0; k < NOBS; ++k) {
-      double re = 0, im = 0;
-      for (int w = 0; w < (NTC + 63) / 64; ++w) {
-        re += red[w * 2 * NOBS + 2 * k];
-        im += red[w * 2 * NOBS + 2 * k + 1];
-      }
-      z[k] = make_double2(inv * re, inv * im);
-      if (en.y >= 0) p.zres[((size_t)ip * p.nefull + en.y) * NOBS + k] = make_double2(inv * re, -inv * im);
+  if (tid < 2 * NOBS) {  // value tid of the 2 NOBS, over the waves
+    double x = 0.0;
+#pragma unroll
+    for (int w = 0; w < NTC / 64; ++w) x += red[w * 2 * NOBS + tid];
+    x *= 1.0 / (double)(nphi * nphi);
+    ((double *)(p.zres + ((size_t)ip * p.nefull + en.x) * NOBS))[tid] = x;
+    if (en.y >= 0) ((double *)(p.zres + ((size_t)ip * p.nefull + en.y) * NOBS))[tid] = (tid & 1) ? -x : x;
+  }
+  if (wave == 0) {  // the first status of the 2 NP that is not zero
+    const unsigned long long any = __ballot(fst != 0);
+    if (lane == (any ? __ffsll(any) - 1 : 0)) {
+      p.status[(size_t)ip * p.nefull + en.x] = fst;
+      if (en.y >= 0) p.status[(size_t)ip * p.nefull + en.y] = fst;
     }
-    int st = 0;
-    for (int q = 0; q < 2 * NP && !st; ++q) st = p.fstatus[base * NP + q];
-    p.status[(size_t)ip * p.nefull + en.x] = st;
-    if (en.y >= 0) p.status[(size_t)ip * p.nefull + en.y] = st;
   }
 }
 
@@ -2841,10 +2881,9 @@ struct pnamp_ctx {
   double *d_mtab = nullptr;         // [3][h]: m, <m+1|J_+|m>, j(j+1) per species-local state
   double2 *d_fout = nullptr, *d_frho = nullptr, *d_sbuf = nullptr;
   int *d_fstatus = nullptr;
-  int2 *d_pn_rows = nullptr;
-  int *d_pn_blk = nullptr, *d_pn_ycol = nullptr;
-  double *d_pn_w = nullptr;
-  int pn_ncol = 0;
+  BilForm wpn = {};                                 // W_pn, in d_bil
+  int2 *d_pn_grp = nullptr;
+  int pn_ng = 0;
   size_t fac_cap = 0;  // pairs the factored scratch holds
   // captured launch sequence of the factored form, valid for (npairs, zval,
   // nval) and the current buffers; dropped whenever a buffer is reallocated
@@ -2954,7 +2993,8 @@ static int dupload(pnamp_ctx *c, T **p, const T *src, size_t count) {
 }
 
 // Tables of a bilinear form sum C(x, y) a_x b_y over n elements (offsets of x in
-// ofs), appended to buf, with f's pointers as offsets into it; sym: a = b.
+// ofs), appended to buf, with f's pointers as offsets into it; sym: a = b; a
+// group's pairs are a multiple of round.
 // Rows that share columns (connected through entries of C: equal Delta m and
 // parity) are tiled together by four, a tile takes only the columns with an
 // entry in it, and tiles of similar column counts form a group, so little is
@@ -2964,7 +3004,7 @@ struct BilTerm {
   double v;
 };
 static void bil_table(std::vector<double> &buf, BilForm &f, int n, bool sym, std::vector<BilTerm> &C,
-                      const std::vector<unsigned> &ofs) {
+                      const std::vector<unsigned> &ofs, int round = 1, std::vector<int2> *groups = nullptr) {
   std::vector<int> root(2 * n);
   for (int i = 0; i < 2 * n; ++i) root[i] = i;
   auto find = [&](int i) {
@@ -3015,7 +3055,8 @@ static void bil_table(std::vector<double> &buf, BilForm &f, int n, bool sym, std
   std::vector<int> pairs;
   int np = 0;
   for (size_t g = 0; g < tiles.size(); g += 4) {
-    pairs.push_back(((int)tiles[g].y.size() + 7) / 8);
+    pairs.push_back((((int)tiles[g].y.size() + 7) / 8 + round - 1) / round * round);
+    if (groups) groups->push_back(make_int2(np, pairs.back()));
     np += pairs.back();
   }
   f.np = (np + BIL_RING - 1) / BIL_RING * BIL_RING;
@@ -3032,7 +3073,8 @@ static void bil_table(std::vector<double> &buf, BilForm &f, int n, bool sym, std
     for (int k = 0; k < 16; ++k) of[last * 16 + k].w = 1u;
     for (size_t b = 0; b < 4 && g + b < tiles.size(); ++b) {
       const Tile &t = tiles[g + b];
-      for (int i = 0; i < t.nx; ++i) of[last * 16 + 4 * i + b].z = ofs[ord[t.x0 + i].second];
+      for (size_t q = s0 / 2; q <= last; ++q)
+        for (int i = 0; i < t.nx; ++i) of[q * 16 + 4 * i + b].z = ofs[ord[t.x0 + i].second];
       for (size_t k = 0; k < t.y.size(); ++k) {
         const size_t st = s0 + k / 4;
         place[t.y[k]] = (int)k;
@@ -3287,12 +3329,12 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
       }
     }
     for (int k = 0; k < 3; ++k) c->nme_s[k] = (int)ls[k].size();
+    std::vector<double> bil;  // the tables of all forms
     // pp and nn lists for k_fac_dens as bilinear forms, x = row + column h of a
     // species block: V [rho_ki rho_lj - rho_li rho_kj] + V A01_ij A10_kl / 4 (the
     // A-blocks hold A01 in the upper and A10 / 4 in the lower triangle), the
     // (kl)(ij) partner of an entry with a + b != c + d as an entry of its own
     {
-      std::vector<double> buf;
       std::vector<unsigned> rb(h * h), ab(h * h);
       for (int x = 0; x < h * h; ++x) {
         rb[x] = (unsigned)(x % h + x / h * (h + 1)) * 16u;
@@ -3315,13 +3357,8 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
           term(i, j, kk, l, e.me);
           if (kk + l != i + j) term(kk, l, i, j, e.me);
         }
-        bil_table(buf, c->frho[k], h * h, true, cr, rb);
-        bil_table(buf, c->fkap[k], h * h, false, ck, ab);
-      }
-      if ((r = dupload(c, &c->d_bil, buf.data(), buf.size()))) return bail(r, c->err);
-      for (BilForm *f : {&c->frho[0], &c->frho[1], &c->fkap[0], &c->fkap[1]}) {
-        f->v = c->d_bil + (size_t)f->v;
-        f->ofs = (const uint4 *)(c->d_bil + (size_t)f->ofs);
+        bil_table(bil, c->frho[k], h * h, true, cr, rb);
+        bil_table(bil, c->fkap[k], h * h, false, ck, ab);
       }
     }
     // W_pn by rows x = c + a h, columns y = d + b h (species-local indices)
@@ -3344,44 +3381,34 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
       for (auto &e : rows[x]) { wcol.push_back(e.first); wval.push_back(e.second); }
       wptr[x + 1] = (int)wcol.size();
     }
-    // dense Delta-m blocks of W_pn for k_fac_combine: row x = c + a h has
-    // Delta m = m_c - m_a, column y = d + b h has m_d - m_b, and a non-zero
-    // needs Delta m(x) = -Delta m(y)
+    // W_pn as a bilinear form for k_fac_combine: row x = c + a h has Delta m = m_c
+    // - m_a, column y = d + b h has m_d - m_b, and a non-zero needs Delta m(x) =
+    // -Delta m(y)
     {
       auto dm = [&](int idx) { return basis->twom[idx % h] - basis->twom[idx / h]; };
-      std::vector<int> dvals;
-      for (int x = 0; x < hh; ++x) dvals.push_back(dm(x));
-      std::sort(dvals.begin(), dvals.end());
-      dvals.erase(std::unique(dvals.begin(), dvals.end()), dvals.end());
-      std::vector<int2> prow;
-      std::vector<int> blk, ycol;
-      std::vector<double> wblk;
-      for (size_t bi = 0; bi < dvals.size(); ++bi) {
-        const int D = dvals[bi];
-        std::vector<int> xs, ys;
-        for (int x = 0; x < hh; ++x) if (dm(x) == D) xs.push_back(x);
-        for (int y = 0; y < hh; ++y) if (dm(y) == -D) ys.push_back(y);
-        blk.insert(blk.end(), {(int)prow.size(), (int)xs.size(), (int)ycol.size(), (int)ys.size(), (int)wblk.size()});
-        const size_t w0 = wblk.size();
-        wblk.resize(w0 + xs.size() * ys.size(), 0.0);
-        for (size_t i = 0; i < xs.size(); ++i) {
-          for (const auto &e : rows[xs[i]]) {
-            const auto it = std::lower_bound(ys.begin(), ys.end(), e.first);
-            if (it == ys.end() || *it != e.first) {  // the plain form takes the list as it is
-              c->fac_list_ok = false;
-              c->fac_reason = "factored and mixed forms need proton-neutron list entries that conserve M";
-              continue;
-            }
-            wblk[w0 + (size_t)(it - ys.begin()) * xs.size() + i] = e.second;
+      std::vector<BilTerm> cw;
+      std::vector<unsigned> xb(hh);
+      for (int x = 0; x < hh; ++x) {
+        xb[x] = (unsigned)x * 16u;
+        for (const auto &e : rows[x]) {
+          if (dm(x) != -dm(e.first)) {  // the plain form takes the list as it is
+            c->fac_list_ok = false;
+            c->fac_reason = "factored and mixed forms need proton-neutron list entries that conserve M";
+            continue;
           }
-          prow.push_back(make_int2(xs[i], (int)bi));
+          cw.push_back({x, e.first, e.second});
         }
-        ycol.insert(ycol.end(), ys.begin(), ys.end());
       }
-      c->pn_ncol = (int)ycol.size();
-      if ((r = dupload(c, &c->d_pn_rows, prow.data(), prow.size())) || (r = dupload(c, &c->d_pn_blk, blk.data(), blk.size())) ||
-          (r = dupload(c, &c->d_pn_ycol, ycol.data(), ycol.size())) || (r = dupload(c, &c->d_pn_w, wblk.data(), wblk.size())))
+      std::vector<int2> grp;
+      bil_table(bil, c->wpn, hh, false, cw, xb, 2, &grp);
+      c->pn_ng = (int)grp.size();
+      if ((r = dupload(c, &c->d_pn_grp, grp.data(), std::max<size_t>(grp.size(), 0))) ||
+          (r = dupload(c, &c->d_bil, bil.data(), bil.size())))
         return bail(r, c->err);
+      for (BilForm *f : {&c->frho[0], &c->frho[1], &c->fkap[0], &c->fkap[1], &c->wpn}) {
+        f->v = c->d_bil + (size_t)f->v;
+        f->ofs = (const uint4 *)(c->d_bil + (size_t)f->ofs);
+      }
     }
     // dense forms of the mixed-precision contraction (rows x, columns y, x and
     // y = species-local pair index c + a h of rho(c, a)): for each species entry
@@ -3812,7 +3839,7 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     const int mix = (c->form == PNAMP_FORM_FACTORED) ? MIX_FP64 : (c->form == PNAMP_FORM_MIXED_FP32 ? MIX_FP32 : MIX_BF16);
     const int h = c->h, hh = h * h, kp = c->kp;
     if (c->nphi > NPHI_MAX) return fail(c, PNAMP_E_SIZE, "factored form supports nphi <= 16");
-    const size_t comb_lds = sizeof(double2) * (size_t)c->nphi * hh + sizeof(int) * (size_t)c->pn_ncol;
+    const size_t comb_lds = sizeof(double2) * (size_t)c->nphi * hh + sizeof(int) * (size_t)hh;
     if (comb_lds > 150 * 1024) return fail(c, PNAMP_E_SIZE, "nphi h^2 complex exceeds the combine LDS");
     if (hh > ((FAC_HMAX * FAC_HMAX + NTC - 1) / NTC) * NTC)
       return fail(c, PNAMP_E_SIZE, "h^2 exceeds the combine rows per workgroup");
@@ -3860,7 +3887,8 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
         if ((r = upload_vmat(c, q, mix))) return r;
       c->va_mix = mix;
     }
-    const size_t comb_nd = sizeof(double2) * (size_t)nd * hh + sizeof(int) * (size_t)c->pn_ncol;
+    const size_t ncol = (nd + 1) / 2;  // column tiles of k_fac_combine
+    const size_t comb_nd = std::max(sizeof(double2) * (size_t)nd * (hh + 1), sizeof(double) * (NTC / 64) * ncol * ncol * 16);
     if (!combine_attr(nd, comb_nd)) return fail(c, PNAMP_E_SIZE, "factored form supports nphi <= 16");
     const size_t setup_lds = sizeof(double2) * 3 * (size_t)hh;
     SetupParams sp;
@@ -3902,8 +3930,7 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     cp.h = h; cp.NE = nec; cp.nefull = c->NE; cp.nphi = c->nphi; cp.self = c->eself; cp.ecan = c->d_ecan;
     cp.zval = zval; cp.nval = nval;
     cp.vac_scale = c->vac_scale; cp.snpfaf = c->snpfaf; cp.sgn_h = (h & 1) ? -1.0 : 1.0; cp.e0 = c->e0;
-    cp.det = c->d_det; cp.pn_rows = c->d_pn_rows; cp.pn_blk = c->d_pn_blk; cp.pn_ycol = c->d_pn_ycol;
-    cp.pn_w = c->d_pn_w; cp.pn_ncol = c->pn_ncol;
+    cp.det = c->d_det; cp.wpn = c->wpn; cp.pn_grp = c->d_pn_grp; cp.pn_ng = c->pn_ng;
     cp.out = c->d_fout; cp.rho = c->d_frho; cp.fstatus = c->d_fstatus; cp.gpn = (const float2 *)c->d_gpn;
     cp.samples = nullptr;
     if (c->fac_graph && (c->g_np != npairs || c->g_form != c->form || c->g_zn != (int)per_pair ||
@@ -4584,8 +4611,8 @@ extern "C" void pnamp_destroy(pnamp_ctx *c) {
                   c->d_q1, c->d_pz, c->d_pn, c->d_zres, c->d_kern, c->d_status, c->d_pair_status,
                   c->d_bil, c->d_Uf, c->d_Vf, c->d_binv, c->d_pfb, c->d_pfs_ok,
                   c->d_UfT, c->d_VfT, c->d_mtab, c->d_fout, c->d_frho,
-                  c->d_sbuf, c->d_fstatus, c->d_pn_rows,
-                  c->d_pn_blk, c->d_pn_ycol, c->d_pn_w, c->d_ecan, c->d_gcls, c->d_gmap};
+                  c->d_sbuf, c->d_fstatus, c->d_pn_grp,
+                  c->d_ecan, c->d_gcls, c->d_gmap};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   for (int q = 0; q < NVPROB; ++q) {
