@@ -1202,8 +1202,8 @@ struct CombParams {
 // those reads, and the gauge sum by loads one after the other (outputs, 2 NP
 // statuses); now by the latency of the phases at the two workgroups per CU
 // that the LDS allows (rho_n in, products, gauge sum).  15 pf pairs at 1000 Euler
-// points, NP = 9: 1270 -> 973 us (the products alone 160 us at the FP64 rate);
-// f5pg9, NP = 4: 820 -> 675 us; sd, NP = 7: 368 -> 265 us.
+// points, NP = 9: 1270 -> 904 us (the products alone 160 us at the FP64 rate);
+// f5pg9, NP = 4: 820 -> 651 us; sd, NP = 7: 368 -> 232 us.
 template <int NP, bool GMIX>
 // (up to nine gauge angles four waves per SIMD: two eight-wave workgroups per
 // CU, as many as their LDS allows; more angles need more than 128 VGPRs)
@@ -1388,23 +1388,23 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
     const double phip = (2.0 * M_PI / nphi) * fp;
     const double phin = (2.0 * M_PI / nphi) * fn;
     const GaugeClass gp = gauge_class(fp, nphi, p.self), gn = gauge_class(fn, nphi, p.self);
-    double2 a[8], b[8];  // the outputs of the two angles
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      a[k] = cconj_if(gp.conj, op[gp.c * FAC_OUT + k]);
-      b[k] = cconj_if(gn.conj, on[gn.c * FAC_OUT + k]);
-    }
+    // the outputs of the two angles, read where they are used (all of them in
+    // registers at once would spill)
+    auto A = [&](int k) { return cconj_if(gp.conj, op[gp.c * FAC_OUT + k]); };
+    auto B = [&](int k) { return cconj_if(gn.conj, on[gn.c * FAC_OUT + k]); };
     const double2 epv = cconj_if(gn.conj, (gp.conj == gn.conj ? epn : epc)[gp.c * NP + gn.c]);
-    const double2 zn = cmul(cscale(vac, cmul(a[0], b[0])),
+    const double2 zn = cmul(cscale(vac, cmul(A(0), B(0))),
                             cexpi(-phip * (p.pz ? p.pz[ip] : p.zval) - phin * (p.pn ? p.pn[ip] : p.nval)));
-    const double2 ekin = cadd(a[2], b[2]);
-    const double2 a8 = cconj_if(gp.conj, op[gp.c * FAC_OUT + 8]), b8 = cconj_if(gn.conj, on[gn.c * FAC_OUT + 8]);
-    const double2 e2s = cadd(cadd(a[1], b[1]), cadd(a8, b8));
+    __builtin_amdgcn_sched_barrier(0);
+    const double2 ekin = cadd(A(2), B(2));
+    const double2 e2s = cadd(cadd(A(1), B(1)), cadd(A(8), B(8)));
     const double2 E = cadd(cadd(e2s, epv), cadd(ekin, make_double2(p.e0, 0.0)));
+    __builtin_amdgcn_sched_barrier(0);
     // <J^2> = A_p + A_n + (t_zp + t_zn)^2 + (t_+p + t_+n)(t_-p + t_-n)
-    const double2 tzs = cadd(a[7], b[7]);
-    const double2 J2 = cadd(cadd(cadd(a[4], b[4]), cmul(tzs, tzs)), cmul(cadd(a[5], b[5]), cadd(a[6], b[6])));
-    const double2 o[NOBS] = {zn, cmul(zn, a[3]), cmul(zn, b[3]), cmul(zn, ekin), cmul(zn, E), cmul(zn, J2)};
+    const double2 tzs = cadd(A(7), B(7));
+    const double2 J2 = cadd(cadd(cadd(A(4), B(4)), cmul(tzs, tzs)), cmul(cadd(A(5), B(5)), cadd(A(6), B(6))));
+    __builtin_amdgcn_sched_barrier(0);
+    const double2 o[NOBS] = {zn, cmul(zn, A(3)), cmul(zn, B(3)), cmul(zn, ekin), cmul(zn, E), cmul(zn, J2)};
     if (p.samples) {
       double2 *sm = p.samples + (((size_t)ip * p.nefull + en.x) * nphi * nphi + t) * 2;
       sm[0] = zn;
@@ -3341,7 +3341,16 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
         ab[x] = (unsigned)x * 16u;
       }
       for (int k = 0; k < 2; ++k) {
+        // (the same list for protons and neutrons, as a charge-symmetric interaction has: the same tables)
+        if (k == 1 && ls[1].size() == ls[0].size() &&
+            !std::memcmp(ls[1].data(), ls[0].data(), ls[0].size() * sizeof(VEntry))) {
+          c->frho[1] = c->frho[0];
+          c->fkap[1] = c->fkap[0];
+          break;
+        }
         std::vector<BilTerm> cr, ck;
+        cr.reserve(4 * ls[k].size());
+        ck.reserve(2 * ls[k].size());
         auto term = [&](int i, int j, int kk, int l, double me) {
           cr.push_back({kk + i * h, l + j * h, me});
           cr.push_back({l + i * h, kk + j * h, -me});
