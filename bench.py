@@ -52,38 +52,49 @@ def plain_terms(inter, n: int) -> int:
 
 
 def plain_own_flops(n: int, nterms: int, nphi: int) -> float:
-    """Real flops of one mesh point along the plain kernels' own algorithm
-    (complex multiply = 6, complex multiply-add = 8): the full-pivot Pfaffian
-    (22 per trailing entry per step, 3 per pivot-scanned entry), Gauss-Jordan
-    column operations on the stacked 3n x n matrix (24 n^3), the three density
-    products (12 n^3), T assembly and phases (42 n^2), the regrouped list
+    """Real flops of one mesh point evaluated along the plain kernels' own algorithm
+    (complex multiply = 6, complex multiply-add = 8): the row-pivot Pfaffian
+    (16 per trailing entry per step), T^-1 and the two products with it (24 n^3),
+    the three density products (12 n^3), T assembly and phases (42 n^2), the regrouped list
     (26 per term), <J^2> / E_kin / traces (40 n^2), and the setup's
     gauge-independent products shared by the nphi^2 gauge points (8 n^3 / nphi^2)."""
     pf = 0.0
     for k in range(n - 1):
         m = 2 * n - 2 * k
-        pf += 22.0 * (m - 2) * (m - 3) / 2 + 3.0 * m * (m - 1) / 2
+        pf += 16.0 * (m - 2) * (m - 3) / 2
     return pf + 36.0 * n ** 3 + 82.0 * n ** 2 + 26.0 * nterms + 8.0 * n ** 3 / (nphi * nphi)
 
 
 def factored_flops(h: int, sum_b2: int, nphi: int, l_species: int, l_cross: int, nnz_pn: int,
                    schur: bool = False) -> float:
-    """Algorithmic real flops of the factored form per (pair, Euler point),
-    complex multiply-add = 8 flops.  Per species: R V1, R* U1, R Z1 (block-sparse,
+    """Algorithmic real flops of the factored form per (pair, Euler point) evaluated,
+    ``nphi`` gauge angles of them, complex multiply-add = 8 flops.  Per species: R V1, R* U1, R Z1 (block-sparse,
     12 sum_b2 h), X, Y (8 h^3), M0 (8 sum_b2 h); then per gauge angle the
-    Pfaffian of the 2h x 2h skew matrix (32 h^3 / 3), Gauss-Jordan on
-    [T^T | W-right-hand sides] (20 h^3), rho, kappa10, kappa01 (12 h^3), the
-    <J^2> ladder sums and traces (40 h^2) and the regrouped species list
-    (28 flops per entry, 56 when its (cd, ab) partner term is present:
+    Pfaffian of the 2h x 2h skew matrix (32 h^3 / 3), T^-1 (8 h^3), the two
+    products with it (16 h^3), rho, kappa10, kappa01 (12 h^3), the <J^2> ladder
+    sums and traces (40 h^2) and the species list as bilinear forms (three real
+    by complex multiply-adds per entry, doubled with its (cd, ab) partner term:
     ``l_species`` entries, ``l_cross`` of them with the partner).  Per Euler
     point once: G = W_pn rho_n (4 flops per CSR entry and phi_n), the nphi^2
     dot products (8 h^2 each) and the gauge sums (100 per gauge pair).  With
     ``schur`` the Pfaffian is the h x h one of the Schur complement (4 h^3 / 3)."""
     setup = 12.0 * sum_b2 * h + 8.0 * h ** 3 + 8.0 * sum_b2 * h
     pfaffian = (4.0 / 3.0 if schur else 32.0 / 3.0) * h ** 3
-    per_phi = pfaffian + (20.0 + 12.0) * h ** 3 + 40.0 * h * h + 28.0 * (l_species + l_cross)
+    per_phi = pfaffian + (8.0 + 16.0 + 12.0) * h ** 3 + 40.0 * h * h + 12.0 * (l_species + l_cross)
     combine = 4.0 * nnz_pn * nphi + 8.0 * nphi * nphi * h * h + 100.0 * nphi * nphi
     return 2.0 * (setup + nphi * per_phi) + combine
+
+
+def evaluated(mesh) -> tuple[int, int]:
+    """(Euler points, gauge angles) the kernels evaluate: one of two points
+    (alpha, gamma), (2 pi - alpha, 2 pi - gamma), and half of an even number of
+    gauge angles; the others are conjugates or repetitions.  (On meshes where every point
+    is its own mirror fewer angles; the bench's is not one.)"""
+    import numpy as np
+    idx = [[int(np.argmin(np.abs(x + y - 2 * np.pi))) if np.abs(x + y - 2 * np.pi).min() < 1e-12 else -1 for y in x]
+           for x in (mesh.alp, mesh.gam)]
+    n = sum(1 for a, i in enumerate(idx[0]) for g, j in enumerate(idx[1]) if i < 0 or j < 0 or (a, g) <= (i, j))
+    return n * mesh.bet.size, mesh.nphi if mesh.nphi % 2 else mesh.nphi // 2
 
 
 def traffic_per_launch(form: str, pairs: int):
@@ -340,28 +351,32 @@ def main():
             nz.add((c + a * h, dl + bl * h))
             if a + b != c + d:
                 nz.add((a + c * h, bl + dl * h))
-        fl = factored_flops(h, sum_b2, w.mesh.nphi, l_sp, l_cr, len(nz), schur) * w.mesh.n_euler * P
-        kname = "k_fac_setup + k_fac_phi + k_fac_combine"
+        nec, nd = evaluated(w.mesh)
+        fl = factored_flops(h, sum_b2, nd, l_sp, l_cr, len(nz), schur) * nec * P
+        kname = "k_fac_setup + k_fac_phi + k_fac_dens + k_fac_combine"
         tform = {FORM_FACTORED: "factored_fp64", FORM_MIXED_FP32: "mixed_fp32", FORM_MIXED_BF16: "mixed_bf16"}[form]
         if form != FORM_FACTORED:
             kname += " + k_vgemm"
     else:
-        fl = plain_flops_per_point(w.n, w.inter.nme) * pts_step
-        kname, tform = "k_plain_setup + k_plain_gauge + k_plain_sum", "plain_fp64"
+        nec, nd = evaluated(w.mesh)
+        own = plain_own_flops(w.n, plain_terms(w.inter, w.n), nd)
+        fl = own * nec * nd * nd * P
+        kname, tform = "k_plain_setup + k_plain_pf + k_plain_gauge + k_plain_sum", "plain_fp64"
     achieved = fl / (k_avg * 1e-3) / 1e12
     # the reference call sequence's count (147 n^3 + 190 L per mesh point) at
     # the same time: what the step's work costs done the reference's way
     plain_equiv = plain_flops_per_point(w.n, w.inter.nme) * pts_step / (k_avg * 1e-3) / 1e12
     form_text = {
         FORM_FACTORED: "factored FP64: per-species Pfaffians and densities, exact algebraic refactoring of the "
-                       "reference sequence, FP64 throughout, batched launches replayed from a captured hipGraph; "
-                       "no MFMA contraction, no surrogate",
+                       "reference sequence, FP64 throughout (products on the FP64 matrix units), mirrored Euler "
+                       "points by conjugation, batched launches replayed from a captured hipGraph; "
+                       "no reduced-precision contraction, no surrogate",
         FORM_MIXED_FP32: "factored, V contraction as FP32 GEMMs on MFMA, everything else FP64, hipGraph",
         FORM_MIXED_BF16: "factored, V contraction as split-BF16 GEMMs on MFMA (FP32 accumulation), everything "
                          "else FP64, hipGraph",
         FORM_PLAIN: "plain FP64 drop-in, any states: per (pair, Euler point) the gauge-independent rotation "
-                    "products, then per gauge point the full-pivot Pfaffian, T^-1 by Gauss-Jordan, densities, "
-                    "regrouped energy list, <J^2>; FP64 throughout",
+                    "products, then per gauge point the row-pivot Pfaffian, T^-1 by Gauss-Jordan, densities, "
+                    "regrouped energy list, <J^2>; mirrored Euler points by conjugation; FP64 throughout",
     }[form]
     out = {
         "metric": "mesh-pts/s: mixed+batched+surrogate vs plain FP64 GPU at |dE_GCM|<1 keV",
@@ -394,8 +409,7 @@ def main():
             "traffic": traffic_per_launch(tform, P),
             "kernel": kname,
             "algorithmic_flops_per_launch": fl,
-            "flops_count": ("the measured form's own algorithm" if form != FORM_PLAIN
-                            else "the reference call sequence, 147 n^3 + 190 L per mesh point"),
+            "flops_count": "the measured form's own algorithm at the mesh points it evaluates",
             "kernel_ms_per_launch": k_avg,
             "reference_sequence_equivalent_tflops": plain_equiv,
         },
@@ -410,11 +424,6 @@ def main():
         }
     if tune is not None:
         out["autotune"] = tune
-    if form == FORM_PLAIN:
-        own = plain_own_flops(w.n, plain_terms(w.inter, w.n), w.mesh.nphi) * pts_step
-        out["roofline"]["own_algorithm_flops_per_launch"] = own
-        out["roofline"]["own_algorithm_tflops"] = own / (k_avg * 1e-3) / 1e12
-        out["roofline"]["own_algorithm_frac"] = own / (k_avg * 1e-3) / 1e12 / PEAK_FP64_TFLOPS
     if form != FORM_PLAIN and not args.no_plain:
         log("bench: plain FP64 reference pass over all pairs")
         ctx.set_form(FORM_PLAIN)

@@ -329,7 +329,7 @@ __global__ __launch_bounds__(NTS) void k_fac_setup(SetupParams p) {
     RZ1[e] = c;
   }
   __syncthreads();
-  for (int e = tid; e < hh; e += NTS) {  // row-major (k_fac_dens reads rows as wave-uniform operands)
+  for (int e = tid; e < hh; e += NTS) {  // row-major (k_fac_dens reads tiles of its rows)
     const int j = e % h, i = e / h;
     out[2 * hh + e] = RV1[i + j * h];
     out[3 * hh + e] = RcU1[i + j * h];
@@ -1447,7 +1447,7 @@ __global__ __launch_bounds__(NTC) __attribute__((amdgpu_waves_per_eu(NP <= 9 ? 4
 
 // E2 observables of the factored form, one workgroup per (pair, Euler point),
 // launched after k_fac_combine: the species densities rho_s(phi) that
-// k_fac_phi wrote give, per species and gauge angle, tr_s(Q_mu rho_s(phi))
+// k_fac_dens wrote give, per species and gauge angle, tr_s(Q_mu rho_s(phi))
 // (ZQ2, Codes/PNAMP/PNAMP_ME1B.f90:52-75) and the orbit-pair traces
 // sum_m rho(k_a(m), k_b(m)) (ZRho1B_Angles, Codes/PNAMP/PNAMP_Rho1B.f90:13-33).
 // (the densities exist at the nd gauge angles evaluated, gauge_class names the rest)
@@ -1461,7 +1461,7 @@ struct FacE2Params {
   const double *det;
   const int *q0, *q1;
   const int *pz, *pn;                // valence numbers per pair, or NULL
-  const double2 *out, *rho;          // k_fac_phi outputs
+  const double2 *out, *rho;          // k_fac_phi and k_fac_dens outputs
   const double *q2;                  // [5][n*n] column-major
   const int4 *orbp;                  // [nob2]: species, first m-state of a, of b (global), size
   double2 *ze2, *zrho;               // [npairs][NE][10], [npairs][NE][nob2]
@@ -3411,7 +3411,7 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
       std::vector<int2> grp;
       bil_table(bil, c->wpn, hh, false, cw, xb, 2, &grp);
       c->pn_ng = (int)grp.size();
-      if ((r = dupload(c, &c->d_pn_grp, grp.data(), std::max<size_t>(grp.size(), 0))) ||
+      if ((r = dupload(c, &c->d_pn_grp, grp.data(), grp.size())) ||
           (r = dupload(c, &c->d_bil, bil.data(), bil.size())))
         return bail(r, c->err);
       for (BilForm *f : {&c->frho[0], &c->frho[1], &c->fkap[0], &c->fkap[1], &c->wpn}) {
@@ -3683,7 +3683,7 @@ extern "C" int pnamp_set_states(pnamp_ctx *c, int nstates, const double *U, cons
   c->pfs_all = all;
   if (sep) {
     int r2 = 0;
-    // row-major copies (U_s(j, k) at j h + k) for the wave-uniform reads of k_fac_phi
+    // row-major copies (U_s(j, k) at j h + k) for the tile reads of k_fac_dens
     std::vector<double> UfT(Uf.size()), VfT(Vf.size());
     for (size_t b = 0; b < (size_t)nstates * 2; ++b)
       for (int j = 0; j < h; ++j)

@@ -35,3 +35,26 @@ def test_grouped_angles_equal_single_ones(h):
         assert np.abs(zb[i] - z1[0]).max() <= 1e-14 * np.abs(z1[0]).max()
         assert np.abs(kb[i] - k1[0]).max() <= 1e-14 * np.abs(k1[0]).max()
     g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["none", "pp", "nn", "pn", "one"])
+def test_lists_with_empty_species_parts(kind):
+    """Tables without groups, of one species only, of a single tile: against the plain form."""
+    from sccm_amd.interaction import Interaction
+    from sccm_amd.pnamp import FORM_FACTORED, FORM_PLAIN, PNAMP
+    b = make_basis("sd")
+    it = synthetic_interaction(b, 1.2, 301, 302)
+    h = b.n // 2
+    pa, pb = it.ka <= h, it.kb <= h
+    keep = {"none": pa & ~pa, "pp": pa & pb, "nn": ~pa & ~pb, "pn": pa & ~pb, "one": np.arange(it.nme) == 3}[kind]
+    it = Interaction(it.ka[keep], it.kb[keep], it.kc[keep], it.kd[keep], it.me[keep], it.t1b, it.e0)
+    g = PNAMP(b, it, make_mesh(2, 2, 3, 3, 2))
+    U, V = zip(*[synthetic_state(b, 2, 2, seed=s) for s in (71, 72)])
+    g.set_states(np.array(U), np.array(V))
+    out = []
+    for form in (FORM_PLAIN, FORM_FACTORED):
+        g.set_form(form)
+        out.append(g.kernels_batched([(0, 1)], 2, 2, want_zres=True)[0])
+    assert np.abs(out[0] - out[1]).max() <= 1e-10 * np.abs(out[0]).max()  # the repository's bar for the FP64 forms
+    g.close()
