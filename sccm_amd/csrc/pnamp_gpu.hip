@@ -3941,7 +3941,6 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     cp.vac_scale = c->vac_scale; cp.snpfaf = c->snpfaf; cp.sgn_h = (h & 1) ? -1.0 : 1.0; cp.e0 = c->e0;
     cp.det = c->d_det; cp.wpn = c->wpn; cp.pn_grp = c->d_pn_grp; cp.pn_ng = c->pn_ng;
     cp.out = c->d_fout; cp.rho = c->d_frho; cp.fstatus = c->d_fstatus; cp.gpn = (const float2 *)c->d_gpn;
-    cp.samples = nullptr;
     if (c->fac_graph && (c->g_np != npairs || c->g_form != c->form || c->g_zn != (int)per_pair ||
                          (!per_pair && (c->g_z != zval || c->g_n != nval))))
       drop_graph(c);
@@ -3956,7 +3955,7 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
       // the launches of all chunks: captured once into a graph that later
       // calls of the same shape and form replay (the pair lists are copied
       // into the same device buffers before each replay), or issued directly
-      // when gauge-point samples are requested
+      // when gauge-point samples or E2 observables are requested
       if (!direct) HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       for (int p0 = 0; p0 < npairs; p0 += chunk) {
         const int np = std::min(chunk, npairs - p0);
@@ -3967,7 +3966,8 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
         cp.pn = per_pair ? c->d_pn + p0 : nullptr;
         cp.zres = c->d_zres + (size_t)p0 * c->NE * NOBS;
         cp.status = c->d_status + (size_t)p0 * c->NE;
-        if (direct) cp.samples = samples + (size_t)p0 * c->NE * c->nphi * c->nphi * 2;
+        // (an E2 call is direct without samples: no offset to a null pointer)
+        cp.samples = samples ? samples + (size_t)p0 * c->NE * c->nphi * c->nphi * 2 : nullptr;
         hipLaunchKernelGGL(k_fac_setup, dim3(nec, np, 2), dim3(NTS), setup_lds, c->stream, sp);
         launch_phi_h(h, mix, c->tune, pfs ? (both ? 2 : 1) : 0, (size_t)np * nec * 2, c->stream, fp);
         if (mix != MIX_FP64) {
