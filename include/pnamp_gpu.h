@@ -230,7 +230,8 @@ int pnamp_hw_solve(pnamp_ctx *ctx, int dim, const double *N, const double *H, do
  * eigenvalues (descending), *m = M, E and var [M][kmax] (row NOS - 1; zero
  * for k >= NOS), and per level the NOS of least variance nos_best[kmax]
  * (strictly below the reference's starting value 100, else 0) with its
- * energy e_best[kmax].  Returns 1 (IFL) if M = 0. */
+ * energy e_best[kmax].  Returns 1 (IFL) if M = 0.  Up to 640 MiB of device
+ * workspace stay with the context for its later Hill-Wheeler calls. */
 int pnamp_hw_presolve(pnamp_ctx *ctx, int dim, const double *N, const double *H, double eps, int kmax, double *EN,
                       int *m, double *E, double *var, int *nos_best, double *e_best);
 

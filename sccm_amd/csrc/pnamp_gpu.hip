@@ -2803,13 +2803,15 @@ void *noalloc_scratch_ptr(int device, std::string &err) {
 }  // namespace
 
 // ====================================================================== host
-// Buffers of the Hill-Wheeler entry points, kept by the context up to HW_KEEP bytes each.
+// Buffers of the Hill-Wheeler entry points, kept by the context between calls
+// up to HW_KEEP bytes in all: the rotation log of the largest scan in LDS (0.5
+// GB) and the matrices beside it.  Kept because a call of 23.0 ms (dim 180, log
+// of 0.4 GB) took 0.4 ms more when it was given back each time.
 struct HwSlot {
   void *p = nullptr;
   size_t cap = 0;
 };
-// (the rotation log of a scan over M = 200 natural states holds 0.5 GB)
-constexpr size_t HW_KEEP = (size_t)1 << 30;
+constexpr size_t HW_KEEP = (size_t)640 << 20;
 
 struct pnamp_ctx {
   std::vector<HwSlot> hw_slot;
@@ -4265,18 +4267,22 @@ extern "C" int pnamp_kernels_batched_noalloc(pnamp_ctx *c, int npairs, const int
 }
 
 // Device buffers of one Hill-Wheeler solve: the context's slots, taken in
-// order and grown where too small; on scope exit the ones above HW_KEEP bytes
-// are given back (the others with the context).
+// order and grown where too small; on scope exit the largest are given back
+// until at most HW_KEEP bytes are left (these go with the context).
 struct HwBufs {
   pnamp_ctx *c;
   size_t next = 0;
   explicit HwBufs(pnamp_ctx *ctx) : c(ctx) {}
   ~HwBufs() {
-    for (auto &s : c->hw_slot)
-      if (s.cap > HW_KEEP) {
-        (void)hipFree(s.p);
-        s = HwSlot{};
-      }
+    size_t kept = 0;
+    for (const HwSlot &s : c->hw_slot) kept += s.cap;
+    while (kept > HW_KEEP) {
+      HwSlot &s = *std::max_element(c->hw_slot.begin(), c->hw_slot.end(),
+                                    [](const HwSlot &a, const HwSlot &b) { return a.cap < b.cap; });
+      kept -= s.cap;
+      (void)hipFree(s.p);
+      s = HwSlot{};
+    }
   }
   template <class T>
   bool alloc(T **q, size_t cnt) {
