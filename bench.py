@@ -51,18 +51,18 @@ def plain_terms(inter, n: int) -> int:
     return int(keep.sum() + (keep & cross).sum())
 
 
-def plain_own_flops(n: int, nterms: int, nphi: int) -> float:
+def plain_own_flops(n: int, nterms: int, ngauge: int) -> float:
     """Real flops of one mesh point evaluated along the plain kernels' own algorithm
     (complex multiply = 6, complex multiply-add = 8): the row-pivot Pfaffian
     (16 per trailing entry per step), T^-1 and the two products with it (24 n^3),
     the three density products (12 n^3), T assembly and phases (42 n^2), the regrouped list
     (26 per term), <J^2> / E_kin / traces (40 n^2), and the setup's
-    gauge-independent products shared by the nphi^2 gauge points (8 n^3 / nphi^2)."""
+    gauge-independent products shared by the ``ngauge`` gauge pairs (8 n^3 / ngauge)."""
     pf = 0.0
     for k in range(n - 1):
         m = 2 * n - 2 * k
         pf += 16.0 * (m - 2) * (m - 3) / 2
-    return pf + 36.0 * n ** 3 + 82.0 * n ** 2 + 26.0 * nterms + 8.0 * n ** 3 / (nphi * nphi)
+    return pf + 36.0 * n ** 3 + 82.0 * n ** 2 + 26.0 * nterms + 8.0 * n ** 3 / ngauge
 
 
 def factored_flops(h: int, sum_b2: int, nphi: int, l_species: int, l_cross: int, nnz_pn: int,
@@ -86,7 +86,7 @@ def factored_flops(h: int, sum_b2: int, nphi: int, l_species: int, l_cross: int,
 
 
 def evaluated(mesh) -> tuple[int, int]:
-    """(Euler points, gauge angles) the kernels evaluate: one of two points
+    """(Euler points, gauge angles) the factored kernels evaluate: one of two points
     (alpha, gamma), (2 pi - alpha, 2 pi - gamma), and half of an even number of
     gauge angles; the others are conjugates or repetitions.  (On meshes where every point
     is its own mirror fewer angles; the bench's is not one.)"""
@@ -97,11 +97,19 @@ def evaluated(mesh) -> tuple[int, int]:
     return n * mesh.bet.size, mesh.nphi if mesh.nphi % 2 else mesh.nphi // 2
 
 
-def traffic_per_launch(form: str, pairs: int):
-    """HBM bytes per launch from the committed PMC measurement
-    (profiles/traffic.json), scaled to ``pairs`` pairs per launch."""
+def plain_gauge_pairs(nphi: int) -> int:
+    """Gauge pairs the plain kernels evaluate per Euler point (same meshes): the
+    two angles together have the period pi, so of an even count half of the
+    pairs, where the factored form needs half of each species' angles."""
+    return nphi * nphi if nphi % 2 else nphi * nphi // 2
+
+
+def traffic_per_launch(form: str, pairs: int, schur: bool = False):
+    """HBM bytes per launch from the committed PMC measurement of this form and
+    Pfaffian route (profiles/traffic.json; None without one), scaled to
+    ``pairs`` pairs per launch."""
     try:
-        t = json.load(open(os.path.join(ROOT, "profiles", "traffic.json")))[form]
+        t = json.load(open(os.path.join(ROOT, "profiles", "traffic.json")))[form + ("_schur" if schur else "")]
     except (OSError, KeyError, ValueError):
         return None
     b = 1024.0 * (t["fetch_kib_per_launch"] * t["fetch_factor"] + t["write_kib_per_launch"] * t["write_factor"])
@@ -358,9 +366,8 @@ def main():
         if form != FORM_FACTORED:
             kname += " + k_vgemm"
     else:
-        nec, nd = evaluated(w.mesh)
-        own = plain_own_flops(w.n, plain_terms(w.inter, w.n), nd)
-        fl = own * nec * nd * nd * P
+        nec, ngauge = evaluated(w.mesh)[0], plain_gauge_pairs(w.mesh.nphi)
+        fl = plain_own_flops(w.n, plain_terms(w.inter, w.n), ngauge) * nec * ngauge * P
         kname, tform = "k_plain_setup + k_plain_pf + k_plain_gauge + k_plain_sum", "plain_fp64"
     achieved = fl / (k_avg * 1e-3) / 1e12
     # the reference call sequence's count (147 n^3 + 190 L per mesh point) at
@@ -406,7 +413,7 @@ def main():
             "peak": PEAK_FP64_TFLOPS,
             "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP64_TFLOPS,
-            "traffic": traffic_per_launch(tform, P),
+            "traffic": traffic_per_launch(tform, P, schur),
             "kernel": kname,
             "algorithmic_flops_per_launch": fl,
             "flops_count": "the measured form's own algorithm at the mesh points it evaluates",
