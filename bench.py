@@ -255,7 +255,7 @@ def main():
                     help="factored forms: keep the 2h x 2h Pfaffian (by default the h x h Schur-complement "
                          "Pfaffian is allowed for states with cond_1(Z_s) <= 1e6)")
     ap.add_argument("--tune", default="", help="factored form: 'pf,rest,div' launch configuration instead of "
-                                               "autotuning (e.g. 6,3,2)")
+                                               "autotuning (e.g. 4,0,2; the second number is ignored)")
     ap.add_argument("--mesh-check", type=int, default=0,
                     help="also solve the GCM on alpha = gamma = N points (same beta, gauge) and report its levels")
     ap.add_argument("--calibrate-copy", action="store_true",
@@ -304,13 +304,15 @@ def main():
     if form == FORM_FACTORED and args.tune:
         pf_w, rest_w, div = (int(x) for x in args.tune.split(","))
         ctx.set_tune(pf_w, rest_w, div)
-        tune = {"pf_waves": pf_w, "rest_waves": rest_w, "chunk_div": div, "set": "given, not timed"}
+        tune = {"pf_waves": pf_w, "chunk_div": div, "set": "given, not timed"}
     elif form == FORM_FACTORED and not args.no_tune:
         t = time.perf_counter()
         tune = ctx.autotune(batch(0), w.zval, w.nval)
         tune["seconds"] = time.perf_counter() - t
-        log(f"bench: autotuned in {tune['seconds']:.1f} s: Pfaffian {tune['pf_waves']} waves/SIMD, "
-            f"densities {tune['rest_waves']}, chunk / {tune['chunk_div']}")
+        for x in (tune, *tune["candidates"]):
+            del x["rest_waves"]  # a label, not a choice: the density kernel has one variant
+        log(f"bench: autotuned in {tune['seconds']:.1f} s: Pfaffian waves/SIMD {tune['pf_waves']} (0: Schur route), "
+            f"chunk / {tune['chunk_div']}")
     for s in range(args.warmup):
         ctx.kernels_batched(batch(s), w.zval, w.nval)
         log(f"bench: warmup step {s} done")

@@ -245,18 +245,20 @@ int pnamp_last_timing(pnamp_ctx *ctx, float *ms_points, float *ms_total);
  * once) and keeps the fastest for later calls of this context.  Candidates
  * (species size h >= 8; smaller spaces have one): waves per SIMD of the
  * Pfaffian kernel {3, 4, 5} and the pair chunk divided by {1, 2, 4}; a kernel
- * variant that spills registers to scratch memory is no candidate.  The
- * density kernel has one variant, reported as 3 (3 h <= 64) or 2.  choice[3] receives (Pfaffian waves, density waves, chunk
- * divisor), cand[3 i .. 3 i + 2] the same for candidate i, ms[i] its kernel
- * time (at most PNAMP_TUNE_MAX candidates), *ncand their number; any may be
- * NULL.  The form must be PNAMP_FORM_FACTORED. */
+ * variant that spills registers to scratch memory is no candidate.  choice[3]
+ * receives (Pfaffian waves, density class, chunk divisor), cand[3 i .. 3 i + 2]
+ * the same for candidate i, ms[i] its kernel time (at most PNAMP_TUNE_MAX
+ * candidates), *ncand their number; any may be NULL.  The density class is a
+ * label that pnamp_set_tune accepts, 3 where 3 h <= 64, else 2: that kernel has
+ * one variant, its registers fitted to three waves per SIMD at h = 6, 8 and 12
+ * and to two elsewhere.  The form must be PNAMP_FORM_FACTORED. */
 #define PNAMP_TUNE_MAX 32
 int pnamp_autotune(pnamp_ctx *ctx, int npairs, const int32_t *q0, const int32_t *q1, int zval, int nval,
                    int *choice, int *cand, float *ms, int *ncand);
 
 /* Sets the factored form's launch configuration directly (a choice of
  * pnamp_autotune kept from an earlier run): Pfaffian waves 0 (default) / 3 /
- * 4 / 5, density waves 0 / 2 / 3 / 4 (all give the one variant), chunk divisor
+ * 4 / 5, density class 0 / 2 / 3 / 4 (all give the one variant), chunk divisor
  * 1 / 2 / 4. */
 int pnamp_set_tune(pnamp_ctx *ctx, int pf_waves, int rest_waves, int chunk_div);
 

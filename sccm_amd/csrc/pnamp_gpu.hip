@@ -4542,7 +4542,8 @@ extern "C" int pnamp_autotune(pnamp_ctx *c, int npairs, const int32_t *q0, const
     for (int div : {1, 2, 4}) cands.push_back({pf, div});
   }
   if (cands.empty()) cands.push_back({0, 1});
-  const int rest = 3 * h <= 64 ? 3 : 2;  // the densities' waves as reported
+  // the density class: a label kept for stored choices (one variant, dens_default_waves(h) waves per SIMD)
+  const int rest = 3 * h <= 64 ? 3 : 2;
   const int pf_dflt = schur ? 0 : pf_default_waves(h);
   if ((int)cands.size() > PNAMP_TUNE_MAX) return fail(c, PNAMP_E_SIZE, "autotune: too many candidates");
   const FacTune keep = c->tune;

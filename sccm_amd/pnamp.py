@@ -299,7 +299,9 @@ class PNAMP:
     def autotune(self, pairs, zval: int, nval: int) -> dict:
         """Times the FP64 factored form's launch candidates on ``pairs`` and
         keeps the fastest: {"pf_waves", "rest_waves", "chunk_div",
-        "candidates": [{"pf_waves", "rest_waves", "chunk_div", "ms"}]}."""
+        "candidates": [{"pf_waves", "rest_waves", "chunk_div", "ms"}]}.
+        ``rest_waves`` is the density class, a label for ``set_tune`` and no
+        number of waves (that kernel has one variant)."""
         pairs = np.asarray(pairs, dtype=np.int32).reshape(-1, 2)
         q0 = np.ascontiguousarray(pairs[:, 0])
         q1 = np.ascontiguousarray(pairs[:, 1])
