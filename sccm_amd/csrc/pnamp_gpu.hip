@@ -440,14 +440,14 @@ __device__ __forceinline__ double dpp_f64(double v) {  // DPP move of a double (
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-// Sum of v over the wavefront by the DPP steps of wave_umax, wave-uniform.
+// Sum of v over the wavefront (lane 63 ends with it), wave-uniform.
 __device__ __forceinline__ double wave_sum_dpp(double v) {
-  v += dpp_f64<0xB1, 0xF>(v);
-  v += dpp_f64<0x4E, 0xF>(v);
-  v += dpp_f64<0x141, 0xF>(v);
-  v += dpp_f64<0x140, 0xF>(v);
-  v += dpp_f64<0x142, 0xA>(v);
-  v += dpp_f64<0x143, 0xC>(v);
+  v += dpp_f64<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+  v += dpp_f64<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f64<0x141, 0xF>(v);  // row_half_mirror
+  v += dpp_f64<0x140, 0xF>(v);  // row_mirror
+  v += dpp_f64<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_f64<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
@@ -1882,7 +1882,7 @@ static hipError_t vgemm_attr() {
 // KP = h^2 rounded up to 32, for the instantiated species sizes
 static bool launch_vgemm(int h, int mix, dim3 grid, hipStream_t s, const VGemmParams &vp) {
   switch (h) {
-    case 2: case 4: launch_vgemm_kp<32>(mix, grid, s, vp); return true;
+    case 4: launch_vgemm_kp<32>(mix, grid, s, vp); return true;
     case 6: launch_vgemm_kp<64>(mix, grid, s, vp); return true;
     case 8: launch_vgemm_kp<64>(mix, grid, s, vp); return true;
     case 10: launch_vgemm_kp<128>(mix, grid, s, vp); return true;
@@ -1950,7 +1950,6 @@ static size_t phi_scratch(const FacTune &t, bool schur) {
 
 static size_t phi_scratch_h(int h, const FacTune &t, bool schur) {
   switch (h) {
-    case 2: return phi_scratch<2>(t, schur);
     case 4: return phi_scratch<4>(t, schur);
     case 6: return phi_scratch<6>(t, schur);
     case 8: return phi_scratch<8>(t, schur);
@@ -1965,12 +1964,11 @@ static size_t phi_scratch_h(int h, const FacTune &t, bool schur) {
   }
 }
 
-// Species sizes h = n / 2 with an instantiated k_fac_phi (every h is even:
-// an orbit holds 2j + 1 states).
+// Species sizes h = n / 2 with an instantiated k_fac_phi (every h is even, an
+// orbit holds 2j + 1 states, and n is at least 8).
 static bool launch_phi_h(int h, int mix, const FacTune &t, int route, size_t blocks, hipStream_t s,
                          const PhiParams &pp) {
   switch (h) {
-    case 2: launch_phi<2>(mix, t, route, blocks, s, pp); return true;
     case 4: launch_phi<4>(mix, t, route, blocks, s, pp); return true;
     case 6: launch_phi<6>(mix, t, route, blocks, s, pp); return true;
     case 8: launch_phi<8>(mix, t, route, blocks, s, pp); return true;
@@ -1991,7 +1989,8 @@ static void launch_combine(bool gmix, dim3 grid, size_t lds, hipStream_t s, cons
   else hipLaunchKernelGGL((k_fac_combine<NP, false>), grid, dim3(NTC), lds, s, cp);
 }
 
-// Dynamic LDS limit of k_fac_combine<np, *>, set before any capture.
+// Dynamic LDS limit of k_fac_combine<np, *>, set before any capture; np is the
+// number of angles evaluated (gauge_classes of up to 16: odd above 8).
 template <int NP>
 static bool combine_attr_np(size_t lds) {
   return hipFuncSetAttribute((const void *)k_fac_combine<NP, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2010,13 +2009,9 @@ static bool combine_attr(int np, size_t lds) {
     case 7: return combine_attr_np<7>(lds);
     case 8: return combine_attr_np<8>(lds);
     case 9: return combine_attr_np<9>(lds);
-    case 10: return combine_attr_np<10>(lds);
     case 11: return combine_attr_np<11>(lds);
-    case 12: return combine_attr_np<12>(lds);
     case 13: return combine_attr_np<13>(lds);
-    case 14: return combine_attr_np<14>(lds);
     case 15: return combine_attr_np<15>(lds);
-    case 16: return combine_attr_np<16>(lds);
     default: return false;
   }
 }
@@ -2032,13 +2027,9 @@ static bool launch_combine_np(int np, bool gmix, dim3 grid, size_t lds, hipStrea
     case 7: launch_combine<7>(gmix, grid, lds, s, cp); return true;
     case 8: launch_combine<8>(gmix, grid, lds, s, cp); return true;
     case 9: launch_combine<9>(gmix, grid, lds, s, cp); return true;
-    case 10: launch_combine<10>(gmix, grid, lds, s, cp); return true;
     case 11: launch_combine<11>(gmix, grid, lds, s, cp); return true;
-    case 12: launch_combine<12>(gmix, grid, lds, s, cp); return true;
     case 13: launch_combine<13>(gmix, grid, lds, s, cp); return true;
-    case 14: launch_combine<14>(gmix, grid, lds, s, cp); return true;
     case 15: launch_combine<15>(gmix, grid, lds, s, cp); return true;
-    case 16: launch_combine<16>(gmix, grid, lds, s, cp); return true;
     default: return false;
   }
 }
@@ -2377,11 +2368,9 @@ __host__ __device__ inline size_t jacobi_lds_bytes(int dim) {  // packed matrix,
   const size_t m = (size_t)dim + (dim & 1);
   return 8 * ((m * (m + 1) / 2 + 1) & ~(size_t)1) + 16 * (m / 2) + 16 * (JNT / 64);
 }
-// jpk(i, j) = max(t_i + j, t_j + i), t_i = i (i + 1) / 2: the larger index's
-// triangle number wins
-// (24-bit products: full rate)
+// Triangle number t_i = i (i + 1) / 2 (a 24-bit product: full rate); entry (i, j)
+// in any order is at max(t_i + j, t_j + i): the larger index's triangle number wins
 __device__ __forceinline__ int jtri(int i) { return (int)(__umul24((unsigned)i, (unsigned)i + 1u) >> 1); }
-__device__ __forceinline__ int jpk(int i, int j) { return max(jtri(i) + j, jtri(j) + i); }
 
 __device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2867,7 +2856,6 @@ struct pnamp_ctx {
   int e2_cap = 0;
   int form = PNAMP_FORM_PLAIN;
   bool separable = false;
-  int nme_s[3] = {0, 0, 0};
   BilForm frho[2] = {}, fkap[2] = {};               // species lists of k_fac_dens (p, n), in d_bil
   double *d_bil = nullptr;
   bool fac_list_ok = false;
@@ -3330,7 +3318,6 @@ extern "C" int pnamp_create(const pnamp_basis *basis, const pnamp_interaction *i
         ls[2].push_back(e);
       }
     }
-    for (int k = 0; k < 3; ++k) c->nme_s[k] = (int)ls[k].size();
     std::vector<double> bil;  // the tables of all forms
     // pp and nn lists for k_fac_dens as bilinear forms, x = row + column h of a
     // species block: V [rho_ki rho_lj - rho_li rho_kj] + V A01_ij A10_kl / 4 (the
@@ -3852,8 +3839,6 @@ static int kernels_impl(pnamp_ctx *c, int npairs, const int32_t *q0, const int32
     if (c->nphi > NPHI_MAX) return fail(c, PNAMP_E_SIZE, "factored form supports nphi <= 16");
     const size_t comb_lds = sizeof(double2) * (size_t)c->nphi * hh + sizeof(int) * (size_t)hh;
     if (comb_lds > 150 * 1024) return fail(c, PNAMP_E_SIZE, "nphi h^2 complex exceeds the combine LDS");
-    if (hh > ((FAC_HMAX * FAC_HMAX + NTC - 1) / NTC) * NTC)
-      return fail(c, PNAMP_E_SIZE, "h^2 exceeds the combine rows per workgroup");
     if (h > FAC_HMAX || (h & 1)) return fail(c, PNAMP_E_SIZE, "factored form: species size h must be even and <= 22");
     // per pair, with nec Euler points and nd gauge angles evaluated: rho
     // [nec][2][nd][h^2], setup blocks [nec][2][5][h^2], per-phi scalars and status;
