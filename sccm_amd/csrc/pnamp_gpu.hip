@@ -2364,19 +2364,21 @@ __device__ __forceinline__ int2 jacobi_pair(int k, int step, int m) {
 // sweeps go to log[(sweep (m - 1) + step) (m / 2) + pair]; the eigenvectors are
 // made from it (k_jacobi_vec, k_nos_vec).
 constexpr int JNT = 1024, LDS_JACOBI_MAX = 200, JBLK = 5;
-__host__ __device__ inline size_t jacobi_lds_bytes(int dim) {  // packed matrix, angles, sums
-  const size_t m = (size_t)dim + (dim & 1);
-  return 8 * ((m * (m + 1) / 2 + 1) & ~(size_t)1) + 16 * (m / 2) + 16 * (JNT / 64);
+__host__ __device__ constexpr int jacobi_cs_offset(int m) { return (m * (m + 1) / 2 + 1) & ~1; }  // doubles; 16-byte aligned
+__host__ __device__ constexpr size_t jacobi_lds_bytes(int dim) {  // packed matrix, angles, sums
+  const int m = dim + (dim & 1);
+  return 8 * (size_t)jacobi_cs_offset(m) + 16 * (size_t)(m / 2) + 16 * (JNT / 64);
 }
+static_assert(jacobi_lds_bytes(LDS_JACOBI_MAX) <= 160 * 1024, "the largest matrix in LDS fits a CU");
 // Triangle number t_i = i (i + 1) / 2 (a 24-bit product: full rate); entry (i, j)
 // in any order is at max(t_i + j, t_j + i): the larger index's triangle number wins
 __device__ __forceinline__ int jtri(int i) { return (int)(__umul24((unsigned)i, (unsigned)i + 1u) >> 1); }
 
 __device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m = dim + (dim & 1), hp = m / 2, ntri = m * (m + 1) / 2;
+  const int m = dim + (dim & 1), hp = m / 2;
   double *const A = sm;  // 16-byte aligned, as cs and red then are
-  double2 *const cs = (double2 *)(A + ((ntri + 1) & ~1));
+  double2 *const cs = (double2 *)(A + jacobi_cs_offset(m));
   double2 *const red = cs + hp;
   // blocks of this thread: the triangle a < b of hp pairs, a <= b' = b - 1 of
   // hb = hp - 1, folded into a rectangle of he / 2 columns (he = hb rounded up
@@ -2605,11 +2607,13 @@ __host__ __device__ inline size_t nos_work_offset(int b, int lim) {  // doubles,
 }
 
 __global__ __launch_bounds__(JNT) void k_nos_scan(NosParams p) {
-  extern __shared__ double jsm[];  // Jacobi part, then the eigenvalues [nos]
+  extern __shared__ double jsm[];
   const int b = p.M - 1 - blockIdx.x;  // the largest blocks first
   const int nos = b + 1, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool lds = nos <= p.lim;
-  double *const dg = jsm + (lds ? (jacobi_lds_bytes(nos) + 7) / 8 : (sizeof(JacobiLds) + 7) / 8);
+  // the eigenvalues [nos]: in place of the angles, which lds_jacobi leaves
+  // unread (m doubles), else after block_jacobi's part
+  double *const dg = jsm + (lds ? jacobi_cs_offset(nos + (nos & 1)) : (int)(sizeof(JacobiLds) + 7) / 8);
   double *A = nullptr, *Vv = nullptr;
   int sw = 0;
   if (lds) {
@@ -4453,12 +4457,10 @@ extern "C" int pnamp_hw_presolve(pnamp_ctx *c, int dim, const double *N, const d
       !B.alloc(&dsw, M) || !B.alloc(&dx, (size_t)M * kmax * M))
     return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in pnamp_hw_presolve");
   NosParams np{dim, M, kmax, 0, dN, dH, dR, dG, nullptr, nullptr, dx, dord, dsw, dE, dvar};
-  constexpr size_t LDS_CAP = 160 * 1024;
-  auto scan_lds = [](int nos) { return (jacobi_lds_bytes(nos) + 7) / 8 * 8 + sizeof(double) * nos; };
-  while (np.lim < std::min(M, LDS_JACOBI_MAX) && scan_lds(np.lim + 1) <= LDS_CAP) ++np.lim;
+  np.lim = std::min(M, LDS_JACOBI_MAX);
   std::vector<int> sw(M);
   for (int pass = 0; pass < 2; ++pass) {
-    size_t lds = scan_lds(np.lim);
+    size_t lds = jacobi_lds_bytes(np.lim);
     if (M > np.lim) {
       lds = std::max(lds, (sizeof(JacobiLds) + 7) / 8 * 8 + sizeof(double) * (size_t)M);
       if (!B.alloc(&dwork, nos_work_offset(M, np.lim)))
