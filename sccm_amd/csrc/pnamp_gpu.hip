@@ -2359,15 +2359,26 @@ __device__ __forceinline__ int2 jacobi_pair(int k, int step, int m) {
 // the LDS reads and writes of the blocks.  A thread keeps its blocks (a, b),
 // a < b, of pair indices for the whole run, consecutive threads take
 // consecutive a of one b (consecutive LDS words); the thread that computes a
-// pair's angle also updates its own 2 x 2 block (a_PP - t a_PQ, a_QQ + t a_PQ,
-// 0: no block of another pair reads it).  The rotations of the first logcap
-// sweeps go to log[(sweep (m - 1) + step) (m / 2) + pair]; the eigenvectors are
-// made from it (k_jacobi_vec, k_nos_vec).
+// pair's angle also updates its own 2 x 2 block, which no block of another pair
+// reads (beside the others' blocks, out of the chain of the angles).  The block
+// is a_PP - t a_PQ, a_QQ + t a_PQ, 0, times c^2 + s^2, which is 1 to an ulp: the
+// error that this leaves in a vector's length over some 1,800 rotations is then
+// in its diagonal entry as well, and V / sqrt(diagonal) solves R^T N R = 1 without
+// it.  The eigenvalue is better without the factor; its (small) difference to the
+// diagonal is kept beside it in 32 bits.  Largest level error of 60 matrices of
+// dimension 40 to 220 against 80-bit solves, geometric mean: both from the diagonal
+// rotated by c, s 1.9e-13, both from the one without the factor 2.7e-13, as
+// here 1.7e-13; norm eigenvalues 3.4e-14, 1.5e-15, 1.6e-15 of the largest.  The
+// rotations of the first logcap sweeps go to log[(sweep (m - 1) + step) (m / 2) +
+// pair]; the eigenvectors are made from it (k_jacobi_vec, k_nos_vec).
 constexpr int JNT = 1024, LDS_JACOBI_MAX = 200, JBLK = 5;
 __host__ __device__ constexpr int jacobi_cs_offset(int m) { return (m * (m + 1) / 2 + 1) & ~1; }  // doubles; 16-byte aligned
-__host__ __device__ constexpr size_t jacobi_lds_bytes(int dim) {  // packed matrix, angles, sums
+__host__ __device__ constexpr int jacobi_ev_offset(int m) {  // floats
+  return 2 * jacobi_cs_offset(m) + 2 * m + 4 * (JNT / 64);
+}
+__host__ __device__ constexpr size_t jacobi_lds_bytes(int dim) {  // packed matrix, angles, sums, eigenvalues' differences
   const int m = dim + (dim & 1);
-  return 8 * (size_t)jacobi_cs_offset(m) + 16 * (size_t)(m / 2) + 16 * (JNT / 64);
+  return (4 * (size_t)(jacobi_ev_offset(m) + m) + 7) / 8 * 8;
 }
 static_assert(jacobi_lds_bytes(LDS_JACOBI_MAX) <= 160 * 1024, "the largest matrix in LDS fits a CU");
 // Triangle number t_i = i (i + 1) / 2 (a 24-bit product: full rate); entry (i, j)
@@ -2380,6 +2391,8 @@ __device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
   double *const A = sm;  // 16-byte aligned, as cs and red then are
   double2 *const cs = (double2 *)(A + jacobi_cs_offset(m));
   double2 *const red = cs + hp;
+  float *const ev = (float *)sm + jacobi_ev_offset(m);
+  for (int i = tid; i < m; i += JNT) ev[i] = 0.0f;
   // blocks of this thread: the triangle a < b of hp pairs, a <= b' = b - 1 of
   // hb = hp - 1, folded into a rectangle of he / 2 columns (he = hb rounded up
   // to even)
@@ -2417,21 +2430,29 @@ __device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
     off *= 2.0;
     if (off <= 1e-30 * (off + dg) || off == 0.0) break;  // uniform: every thread summed the same words
     for (int step = 0; step < m - 1; ++step) {
+      int2 p = make_int2(0, 0);
+      double app = 0.0, aqq = 0.0, apq = 0.0, t = 0.0;
+      double2 r = make_double2(1.0, 0.0);
       if (tid < hp) {
-        const int2 p = jacobi_pair(tid, step, m);
-        const int ipp = jtri(p.x) + p.x, iqq = jtri(p.y) + p.y, ipq = jtri(p.y) + p.x;
-        const double app = A[ipp], aqq = A[iqq], apq = A[ipq];
-        double t;
-        const double2 r = jacobi_angle(app, aqq, apq, p.y < dim, t);
-        if (t != 0.0) {
-          A[ipp] = fma(-t, apq, app);
-          A[iqq] = fma(t, apq, aqq);
-          A[ipq] = 0.0;
-        }
+        p = jacobi_pair(tid, step, m);
+        app = A[jtri(p.x) + p.x];
+        aqq = A[jtri(p.y) + p.y];
+        apq = A[jtri(p.y) + p.x];
+        r = jacobi_angle(app, aqq, apq, p.y < dim, t);
         cs[tid] = r;
         if (sweep < logcap) log[((size_t)sweep * (m - 1) + step) * hp + tid] = r;
       }
       __syncthreads();
+      if (t != 0.0) {  // the pair's own block (not in the chain of the angles)
+        const double g = fma(r.x - 1.0, r.x + 1.0, r.y * r.y);  // c^2 + s^2 - 1
+        const double epp = fma(-t, apq, app), eqq = fma(t, apq, aqq);
+        const double bpp = fma(epp, g, epp), bqq = fma(eqq, g, eqq);
+        A[jtri(p.x) + p.x] = bpp;
+        A[jtri(p.y) + p.y] = bqq;
+        A[jtri(p.y) + p.x] = 0.0;
+        ev[p.x] += (float)(epp - bpp);
+        ev[p.y] += (float)(eqq - bqq);
+      }
 #pragma unroll
       for (int u = 0; u < JBLK; ++u) {
         if (ab[u] < 0) continue;
@@ -2457,14 +2478,19 @@ __device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
 }
 
 // One workgroup, the matrix in LDS; A (dim x dim) receives the eigenvalues on
-// its diagonal.
-__global__ __launch_bounds__(JNT) void k_jacobi_lds(double *A, int dim, double2 *log, int *nsweeps) {
+// its diagonal, cong (where not NULL) the diagonal of the rotated matrix.
+__global__ __launch_bounds__(JNT) void k_jacobi_lds(double *A, double *cong, int dim, double2 *log, int *nsweeps) {
   extern __shared__ double jsm[];
   const int m = dim + (dim & 1);
   for (int j = threadIdx.x >> 6; j < m; j += JNT / 64)
     for (int i = threadIdx.x & 63; i <= j; i += 64) jsm[j * (j + 1) / 2 + i] = j < dim ? A[i + (size_t)j * dim] : 0.0;
   const int sw = lds_jacobi(jsm, dim, log, log ? 60 : 0);
-  for (int i = threadIdx.x; i < dim; i += JNT) A[i + (size_t)i * dim] = jsm[jtri(i) + i];
+  const float *const ev = (const float *)jsm + jacobi_ev_offset(m);
+  for (int i = threadIdx.x; i < dim; i += JNT) {
+    const double b = jsm[jtri(i) + i];
+    A[i + (size_t)i * dim] = b + ev[i];
+    if (cong) cong[i] = b;
+  }
   if (threadIdx.x == 0) *nsweeps = sw;
 }
 
@@ -2621,7 +2647,8 @@ __global__ __launch_bounds__(JNT) void k_nos_scan(NosParams p) {
     for (int j = wave; j < m; j += JNT / 64)
       for (int i = lane; i <= j; i += 64) jsm[jtri(j) + i] = j < nos ? p.G[i + (size_t)j * p.M] : 0.0;
     sw = lds_jacobi(jsm, nos, p.log + nos_log_offset(b), NOS_LOGCAP);
-    for (int i = tid; i < nos; i += JNT) dg[i] = jsm[jtri(i) + i];
+    const float *const ev = (const float *)jsm + jacobi_ev_offset(m);
+    for (int i = tid; i < nos; i += JNT) dg[i] = jsm[jtri(i) + i] + ev[i];
   } else {
     A = p.work + nos_work_offset(b, p.lim);
     Vv = A + (size_t)nos * nos;
@@ -4293,10 +4320,11 @@ struct HwBufs {
 };
 
 // Eigenvalues of the symmetric dA (dim x dim; on its diagonal afterwards) and,
-// where dV is not NULL, its eigenvectors.  Up to LDS_JACOBI_MAX the matrix
+// where dV is not NULL, its eigenvectors; cong (device, may be NULL) receives
+// diag(V^T A V) for V as it was computed, where that is not the same.  Up to LDS_JACOBI_MAX the matrix
 // stays in one workgroup's LDS; beyond, one launch per step and a test of the
 // off-diagonal norm per sweep.
-static int hw_eig(pnamp_ctx *c, HwBufs &B, double *dA, double *dV, int dim) {
+static int hw_eig(pnamp_ctx *c, HwBufs &B, double *dA, double *dV, int dim, double *cong = nullptr) {
   const int m = dim + (dim & 1), hp = m / 2;
   const size_t sweep = (size_t)(m - 1) * hp;
   const dim3 gv((dim + JVR - 1) / JVR), bv((hp + 63) / 64 * 64);
@@ -4308,7 +4336,7 @@ static int hw_eig(pnamp_ctx *c, HwBufs &B, double *dA, double *dV, int dim) {
     if (dV && !B.alloc(&dlog, 60 * sweep)) return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
     HIPCHK(c, hipFuncSetAttribute((const void *)k_jacobi_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)jacobi_lds_bytes(dim)));
-    hipLaunchKernelGGL(k_jacobi_lds, dim3(1), dim3(JNT), jacobi_lds_bytes(dim), c->stream, dA, dim, dlog, dns);
+    hipLaunchKernelGGL(k_jacobi_lds, dim3(1), dim3(JNT), jacobi_lds_bytes(dim), c->stream, dA, cong, dim, dlog, dns);
     if (dV) hipLaunchKernelGGL(k_jacobi_vec, gv, bv, lv, c->stream, dV, dim, dlog, dns, 1);
     HIPCHK(c, hipGetLastError());
     return PNAMP_OK;
@@ -4354,17 +4382,18 @@ static int hw_prepare(pnamp_ctx *c, HwBufs &B, int dim, const double *N, const d
                       double *EN, int *Mout, double **dN, double **dH, double **dR, double **dG) {
   const size_t dd = (size_t)dim * dim;
   double *dA = nullptr, *dV = nullptr, *dD = nullptr, *dw = nullptr, *dX = nullptr;
-  if (!B.alloc(&dA, dd) || !B.alloc(&dV, dd) || !B.alloc(dN, dd) || !B.alloc(dH, dd))
+  const size_t nc = dim <= LDS_JACOBI_MAX ? dim : 0;  // diag(D^T N D) after A (beyond, it is the eigenvalue)
+  if (!B.alloc(&dA, dd + dim) || !B.alloc(&dV, dd) || !B.alloc(dN, dd) || !B.alloc(dH, dd))
     return fail(c, PNAMP_E_DEVICE, "hipMalloc failed in the Hill-Wheeler solve");
   std::vector<double> negN(dd);
   for (size_t i = 0; i < dd; ++i) negN[i] = -N[i];
   HIPCHK(c, hipMemcpyAsync(dA, negN.data(), sizeof(double) * dd, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(*dN, N, sizeof(double) * dd, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(*dH, H, sizeof(double) * dd, hipMemcpyHostToDevice, c->stream));
-  const int re = hw_eig(c, B, dA, dV, dim);
+  const int re = hw_eig(c, B, dA, dV, dim, dA + dd);
   if (re) return re;
-  std::vector<double> A(dd), Vv(dd);
-  HIPCHK(c, hipMemcpyAsync(A.data(), dA, sizeof(double) * dd, hipMemcpyDeviceToHost, c->stream));
+  std::vector<double> A(dd + nc), Vv(dd);
+  HIPCHK(c, hipMemcpyAsync(A.data(), dA, sizeof(double) * A.size(), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(Vv.data(), dV, sizeof(double) * dd, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   // ascending eigenvalues of -N == descending EN
@@ -4379,7 +4408,9 @@ static int hw_prepare(pnamp_ctx *c, HwBufs &B, int dim, const double *N, const d
   if (M <= 0) return PNAMP_OK;
   std::vector<double> D((size_t)dim * M), w(M);
   for (int k = 0; k < M; ++k) {
+    // R = D / sqrt(D^T N D): the rotated matrix's diagonal, unless EN is of the size of its rounding
     w[k] = EN[k];
+    if (nc && std::fabs(A[dd + ord[k]] + EN[k]) < 1e-6 * EN[k]) w[k] = -A[dd + ord[k]];
     for (int i = 0; i < dim; ++i) D[i + (size_t)k * dim] = Vv[i + (size_t)ord[k] * dim];
   }
   if (!B.alloc(&dD, (size_t)dim * M) || !B.alloc(&dw, M) || !B.alloc(dR, (size_t)dim * M) ||
