@@ -7,8 +7,9 @@
 // gauge_class in pnamp_gpu.hip).  For a range of units it runs
 //   k_plain_setup  per unit: the gauge-independent products of the rotation
 //                  with the states (7 n x n complex matrices) -> work buffer;
-//   k_plain_gauge  per (unit, gauge point): Pfaffian, T^-1, densities, energy,
-//                  <J^2>, traces (and the E2 traces) -> work buffer;
+//   k_plain_pf     per (unit, gauge point): the Pfaffian -> work buffer;
+//   k_plain_gauge  per (unit, gauge point): T^-1, densities, energy, <J^2>,
+//                  traces (and the E2 traces) -> work buffer;
 //   k_plain_sum    per unit: the Fomenko sum over the gauge points -> ZRES.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -46,9 +47,9 @@ struct PlainArgs {
 };
 
 // n supported by the plain kernels: even, 8 <= n <= 64 (size classes
-// 16, 24, 32, 40, 48, 64; the Pfaffian's 64-bit pivot keys carry the
-// row-major rank of an entry of the 2n x 2n matrix in 14 bits, and the
-// Gauss-Jordan keeps its used columns in a 64-bit mask)
+// 16, 24, 32, 40, 48, 64; the Pfaffian's 32-bit pivot keys carry the column in
+// six bits, seven for n > 32, and the Gauss-Jordan keeps its used columns in a
+// 64-bit mask)
 bool plain_supported(int n);
 // work-buffer bytes per unit
 size_t plain_unit_bytes(const PlainArgs &a);

@@ -244,7 +244,11 @@ struct PfCfg {
   static constexpr int G = (2 * N <= 48) ? 8 : 16;
   static constexpr int NT = G * G;
   static constexpr int T = (2 * N + G - 1) / G, NS = T * (T + 1) / 2;
-  // slots, held R and C, addresses: the waves per SIMD that fit
+  // slots, held R and C, addresses: the waves per SIMD that fit (512 / waves
+  // registers).  Of the size classes only N = 40 lies between four waves' 128 and
+  // the line's 136: 128 registers and 20 bytes spilled, faster than three waves
+  // (above); the others take 103 (16, 32: 4 waves), 166 (24, 48: 3), 248 (64: 2)
+  // and spill nothing
   static constexpr int REGS = 4 * NS + 8 * T + 36;
   static constexpr int WV = REGS <= 102 ? 5 : (REGS <= 136 ? 4 : (REGS <= 168 ? 3 : 2));
 };

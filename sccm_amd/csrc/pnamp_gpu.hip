@@ -1921,8 +1921,12 @@ static void launch_phi(int mix, const FacTune &t, int route, size_t blocks, hipS
   else if (H >= 8 && mix == MIX_FP64 && t.pf_waves == 5) hipLaunchKernelGGL((k_fac_phi<H, PART_PF, 5>), g, b, 0, s, pp);
   else hipLaunchKernelGGL((k_fac_phi<H, PART_PF>), g, b, 0, s, pp);
   // the fewest groups of angles, of equal size; more groups while all waves
-  // still run at once, one per SIMD (one sd pair, 10 Euler points, 4 angles:
-  // 31 us in groups of five, 23 us one by one)
+  // still run at once, one per SIMD.  Mesh-point kernels of a call, always in
+  // the fewest groups / single angles / this rule: h = 12, 4 angles, 40 blocks
+  // 61 / 54 / 54 us, 512 blocks 70 / 77 / 69 us; h = 20, 9 angles, 40 blocks 118 /
+  // 107 / 107 us, 960 blocks 305 / 479 / 306 us.  Over h = 6 .. 22, 4 and 9 angles
+  // and 10 to 2,048 blocks the rule is within 1 % of the better one, but h = 20 and
+  // 22 at exactly 1,024 waves (6 and 4 %).
   pp.ngrp = (pp.nd + dens_angles(H) - 1) / dens_angles(H);
   pp.geff = (pp.nd + pp.ngrp - 1) / pp.ngrp;
   while (pp.geff > 1 && blocks * (size_t)((pp.nd + pp.geff - 2) / (pp.geff - 1)) <= 1024) --pp.geff;
