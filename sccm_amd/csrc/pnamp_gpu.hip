@@ -10,17 +10,18 @@
 //                 vacuum overlap det(1 + Z^T Z)^{-1/4} (Cholesky).
 //   k_plain_*     plain form (plain_gpu.hip): per (pair, Euler point) the
 //                 gauge-independent rotation products, then one workgroup
-//                 per gauge point: Pfaffian of the 2n x 2n skew matrix (full
-//                 pivoting, the ZPfaffianF algorithm), T^{-1} applied by
-//                 Gauss-Jordan, rho / kappa, Tr rho per species, E_kin, <J^2>
-//                 and the two-body energy from the regrouped m-scheme list;
-//                 then the gauge sum into ZRES(pair, Euler, obs).
+//                 per gauge point: Pfaffian of the 2n x 2n skew matrix (row
+//                 pivoting), T^{-1} applied by Gauss-Jordan, rho / kappa, Tr rho
+//                 per species, E_kin, <J^2> and the two-body energy from the
+//                 regrouped m-scheme list; then the gauge sum into
+//                 ZRES(pair, Euler, obs).
 //   k_fac_*       factored form for states without proton-neutron mixing.
-//   k_project     one workgroup per (pair, observable): J-projection sums
+//   k_project*    one workgroup per (pair, observable): J-projection sums
 //                 over the Euler mesh (plain or literal fold).
-//   k_hw_*        Hill-Wheeler: Jacobi eigen-solves of N and N^-1/2 H N^-1/2.
+//   k_jacobi_*, k_nos_*  Hill-Wheeler: Jacobi eigen-solves of N and N^-1/2 H
+//                 N^-1/2, the scan over natural states.
 //
-// Everything is FP64.  No CPU fallback: every numerical step of a kernel
+// Everything is FP64 but the mixed forms' contraction.  No CPU fallback: every numerical step of a kernel
 // call runs on the device.
 #include <hip/hip_runtime.h>
 
@@ -2400,17 +2401,20 @@ __device__ int lds_jacobi(double *sm, int dim, double2 *log, int logcap) {
   // blocks of this thread: the triangle a < b of hp pairs, a <= b' = b - 1 of
   // hb = hp - 1, folded into a rectangle of he / 2 columns (he = hb rounded up
   // to even)
-  const int hb = hp - 1, he = hb + (hb & 1);
+  const int hb = hp - 1, he = hb + (hb & 1), w = max(he / 2, 1);
+  // few blocks go to other waves than the pairs, which have their own to update
+  // (a solve of dim 20 0.47 -> 0.44 ms)
+  const int off = w * (he + 1) <= JNT - 128 ? 128 : 0;
   int ab[JBLK];
 #pragma unroll
   for (int u = 0; u < JBLK; ++u) {
-    const int w = max(he / 2, 1), e = tid + u * JNT, i = e % w, j = e / w;
+    const int e = max(tid - off, 0) + u * JNT, i = e % w, j = e / w;
     int a = i, b = j - 1;
     if (j <= i) {
       a = he - 1 - i;
       b = he - 1 - j;
     }
-    ab[u] = (hb > 0 && j <= he && a < hb && b < hb) ? (a | ((b + 1) << 16)) : -1;
+    ab[u] = (tid >= off && hb > 0 && j <= he && a < hb && b < hb) ? (a | ((b + 1) << 16)) : -1;
   }
   int sweep = 0;
   for (; sweep < 60; ++sweep) {
@@ -2613,7 +2617,7 @@ __global__ __launch_bounds__(JNT) void k_jacobi_done(const double *A, int dim, i
 // Three launches: k_nos_scan the eigenvalues (LDS, rotations logged, nos <=
 // lim; else block_jacobi in work), k_nos_vec the kmax lowest eigenvectors from
 // the log, k_nos_var the amplitudes and the variance.
-constexpr int NOS_LOGCAP = 24;      // sweeps logged (about ten are needed; a block with more takes block_jacobi)
+constexpr int NOS_LOGCAP = 24;      // sweeps logged (about ten are needed, graded matrices up to twenty; with more in a block all take block_jacobi)
 struct NosParams {
   int dim, M, kmax, lim;
   const double *N, *H, *R, *G;
