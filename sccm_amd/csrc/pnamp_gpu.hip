@@ -2360,7 +2360,7 @@ __device__ __forceinline__ int2 jacobi_pair(int k, int step, int m) {
 // each 2 x 2 block of a pair of pairs once instead of twice and nothing leaves
 // the CU.  Up to m = 200 (LDS_JACOBI_MAX; 202 would exceed the CU's 160 KB).
 // With the matrix streaming through L2 a solve of one workgroup took 87 ms at
-// dim 180, here 5.1 ms (the mean of a call's three solves), bound by
+// dim 180, here 5.1 to 5.4 ms (the mean of a call's three solves), bound by
 // the LDS reads and writes of the blocks.  A thread keeps its blocks (a, b),
 // a < b, of pair indices for the whole run, consecutive threads take
 // consecutive a of one b (consecutive LDS words); the thread that computes a
